@@ -81,6 +81,15 @@ uint64_t extent(const uint64_t *shape, const uint64_t *strides, uint64_t ndim) {
   return hi + 1;
 }
 
+// Gradient term of one operand, for the reduction path: g and the operands the term reads.
+template <Bin OP, bool B>
+struct BinTerm {
+  static constexpr int NIN = 1 + int(kGradUsesA<OP, B>) + int(kGradUsesB<OP, B>);
+  __device__ __forceinline__ float eval(const float *v) const {
+    return bin_grad_term<OP, B>(v, false);
+  }
+};
+
 // Accumulate one operand's gradient. The reference's broadcast backward addresses the gradient
 // buffer with the operand's *data* strides (kernel_macros.h:314-317 passes a->strides as
 // da_strides; its contiguous path indexes da flat, the same offsets for a contiguous operand). A
@@ -90,9 +99,10 @@ uint64_t extent(const uint64_t *shape, const uint64_t *strides, uint64_t ndim) {
 // deterministic reduction over the axes that repeat an offset (broadcast or expanded axes; the
 // reference uses `omp atomic` here: kernel_macros.h:283-299). Offsets past the gradient's own
 // extent (the reference would write out of bounds) are refused.
-template <class Elem, class Term>
+template <Bin OP, bool B>
 void grad_into(const Tensor *x, const Tensor *out, const Tensor *a, const Tensor *b,
-               const Elem &elem, const Term &term, const char *where) {
+               uint64_t simd, const char *where) {
+  using Elem = BinGradBody<OP, B>;
   const Tensor *g = out->grad;
   const int rank = int(g->ndim);
   int64_t tst[kMaxRank];
@@ -108,32 +118,31 @@ void grad_into(const Tensor *x, const Tensor *out, const Tensor *a, const Tensor
   for (int d = 0; d < rank; ++d) repeats = repeats || (tst[d] == 0 && g->shape[d] > 1);
   Space s;
   init_space(s, g->shape, rank);
+  // the terms' operands: g and what the term reads of a and b, behind the gradient itself when the
+  // target is elementwise
+  const void *ins[Elem::NIN];
+  int n = 0;
+  if (!repeats) ins[n++] = x->grad->data;
+  set_own(s, n, g);
+  ins[n++] = g->data;
+  if (kGradUsesA<OP, B>) {
+    set_operand(s, n, a);
+    ins[n++] = a->data;
+  }
+  if (kGradUsesB<OP, B>) {
+    set_operand(s, n, b);
+    ins[n++] = b->data;
+  }
+  for (int d = 0; d < rank; ++d) s.st[n][d] = tst[d];
   if (!repeats) {
-    for (int d = 0; d < rank; ++d) s.st[0][d] = s.st[4][d] = tst[d];
-    set_own(s, 1, g);
-    set_operand(s, 2, a);
-    set_operand(s, 3, b);
-    const void *ins[4] = {x->grad->data, g->data, a->data, b->data};
+    for (int d = 0; d < rank; ++d) s.st[0][d] = tst[d];
+    Elem elem;
+    elem.simd_end = simd;
     launch_elementwise(elem, ins, x->grad->data, s, where);
   } else {
-    set_own(s, 0, g);
-    set_operand(s, 1, a);
-    set_operand(s, 2, b);
-    for (int d = 0; d < rank; ++d) s.st[3][d] = tst[d];
-    const void *ins[3] = {g->data, a->data, b->data};
-    reduce_accumulate(term, ins, static_cast<float *>(x->grad->data), s, where);
+    reduce_accumulate(BinTerm<OP, B>{}, ins, static_cast<float *>(x->grad->data), s, where);
   }
 }
-
-// Gradient term of one operand from (g, a, b), for the reduction path.
-template <Bin OP, bool B>
-struct BinTerm {
-  static constexpr int NIN = 3;
-  __device__ __forceinline__ float eval(const float *v) const {
-    if constexpr (B) return grad_b<OP>(v[0], v[1], v[2], false);
-    else return grad_a<OP>(v[0], v[1], v[2]);
-  }
-};
 
 template <Bin OP>
 void binary_backward(Tensor **in, const Tensor *out, const char *where) {
@@ -145,18 +154,12 @@ void binary_backward(Tensor **in, const Tensor *out, const char *where) {
     return;
   }
   const bool da = a->requires_grad && a->grad, db = b->requires_grad && b->grad;
-  const Tensor *g = out->grad;
   const uint64_t n = numel(out);
   // The reference's contiguous same-shape path (kernel_macros.h:306-311) rounds the B-gradient of
   // sub/div from 0 - g inside its SIMD blocks.
   const bool ref_contig = contiguous(a) && contiguous(b) && contiguous(out) && same_shape(a, b);
-  if (da) grad_into(a, out, a, b, BinGradABody<OP>{}, BinTerm<OP, false>{}, where);
-  if (db) {
-    BinGradBBody<OP> body;
-    body.simd_end = ref_contig ? simd_end(n) : 0;
-    grad_into(b, out, a, b, body, BinTerm<OP, true>{}, where);
-  }
-  (void)g;
+  if (da) grad_into<OP, false>(a, out, a, b, 0, where);
+  if (db) grad_into<OP, true>(b, out, a, b, ref_contig ? simd_end(n) : 0, where);
   finish(where);
 }
 

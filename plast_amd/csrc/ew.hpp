@@ -81,6 +81,9 @@ struct ScalarBody {
   static constexpr bool kTape = false;             // selects the vectorised launch shape
   static constexpr bool kTileFixed3 = false;       // fixed-role tile kernels for 3 operands
   static constexpr int kTileRows = 1;              // tile rows per evaluation
+  // host: whether no element's value depends on its linear index (the NEG rule), so that the axes
+  // may be walked in another order
+  bool index_free() const { return true; }
   template <int U, int N>
   __device__ __forceinline__ void eval_units(const f4 (&x)[U][N], const uint64_t (&idx)[U],
                                              const bool (&valid)[U], f4 (&acc)[U]) const {
@@ -124,6 +127,7 @@ struct UnBody : ScalarBody<UnBody<OP>> {
   static constexpr int NIN = 1;
   float alpha;
   uint64_t simd_end;  // 0 when the reference would take its non-contiguous path
+  bool index_free() const { return OP != Un::Neg || simd_end == 0; }
   __device__ __forceinline__ float eval(const float *v, uint64_t i) const {
     return un_op<OP>(v[0], alpha, i < simd_end);
   }
@@ -140,22 +144,30 @@ struct UnGradBody : ScalarBody<UnGradBody<OP>> {
   }
 };
 
-// operands: da, g, a, b  ->  da + grad_a
-template <Bin OP>
-struct BinGradABody : ScalarBody<BinGradABody<OP>> {
-  static constexpr int NIN = 4;
-  __device__ __forceinline__ float eval(const float *v, uint64_t) const {
-    return v[0] + grad_a<OP>(v[1], v[2], v[3]);
-  }
-};
+// Which of a binary op's operands a gradient term reads: the others are not passed, so not loaded
+// (an add's gradient is 12 B an element, not 20).
+template <Bin OP, bool B>
+constexpr bool kGradUsesA = B && (OP == Bin::Mul || OP == Bin::Div);
+template <Bin OP, bool B>
+constexpr bool kGradUsesB = OP == Bin::Div || (OP == Bin::Mul && !B);
 
-// operands: db, g, a, b  ->  db + grad_b
-template <Bin OP>
-struct BinGradBBody : ScalarBody<BinGradBBody<OP>> {
-  static constexpr int NIN = 4;
+// The gradient term of operand A or B (B) from v = g and the operands it reads, in order.
+template <Bin OP, bool B>
+__device__ __forceinline__ float bin_grad_term(const float *v, bool simd) {
+  const float x = kGradUsesA<OP, B> ? v[1] : 0.0f;
+  const float y = kGradUsesB<OP, B> ? v[kGradUsesA<OP, B> ? 2 : 1] : 0.0f;
+  if constexpr (B) return grad_b<OP>(v[0], x, y, simd);
+  else return grad_a<OP>(v[0], x, y);
+}
+
+// operands: d, g and those of a, b that the term reads  ->  d + term
+template <Bin OP, bool B>
+struct BinGradBody : ScalarBody<BinGradBody<OP, B>> {
+  static constexpr int NIN = 2 + int(kGradUsesA<OP, B>) + int(kGradUsesB<OP, B>);
   uint64_t simd_end;
+  bool index_free() const { return simd_end == 0; }
   __device__ __forceinline__ float eval(const float *v, uint64_t i) const {
-    return v[0] + grad_b<OP>(v[1], v[2], v[3], i < simd_end);
+    return v[0] + bin_grad_term<OP, B>(v + 1, i < simd_end);
   }
 };
 
@@ -235,6 +247,7 @@ struct TapeBody {
   // bit i: the NEG at instruction i follows the reference's contiguous path (0 - x below simd_end,
   // -x in the tail); a NEG whose bit is clear takes its strided path (-x everywhere)
   uint32_t neg_simd;
+  bool index_free() const { return neg_simd == 0; }
 
   template <class F>
   __device__ __forceinline__ static f4 map(f4 a, F f) {
