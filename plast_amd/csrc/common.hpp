@@ -53,6 +53,23 @@ constexpr int kBlock = 256;  // threads per workgroup for streaming kernels (4 w
 #ifndef PLAST_TAPE_XCD
 #define PLAST_TAPE_XCD 0
 #endif
+// Tape launches of at most this many elements take the generic kernel, one element per lane: a short
+// launch lasts as long as one wave's walk through the interpreter, whose code and live values are
+// a quarter with one element per lane. Device time of config 2's chain, vector kernel / generic:
+// 4096 elements 4.22 / 3.45 us, 65536 4.47 / 3.60, 262144 4.58 / 4.33, 400000 4.69 / 5.47, 2^20
+// 5.10 / 9.34; config 3's chain, tile kernel / generic: [4, 64, 64] 4.20 / 3.05, [4, 256, 256]
+// 4.34 / 4.08, [16, 256, 256] 4.73 / 9.32. Fixed bodies gain nothing (six launches of
+// [10, 100] 13.05 / 13.62 us).
+#ifndef PLAST_TAPE_SMALL
+#define PLAST_TAPE_SMALL (1u << 18)
+#endif
+// Spaces of whole 64x64 tiles always take the fixed-role tile kernel; with ragged extents, from this
+// many elements on. Config 3's chain, ragged tile / generic: [8, 301, 150] 5.82 / 4.12 us,
+// [8, 200, 301] 5.82 / 5.22, [8, 301, 301] 5.95 / 6.58, [12, 301, 301] 6.56 / 9.91,
+// [64, 513, 301] 22 / 56 us.
+#ifndef PLAST_TILE_RAGGED_MIN
+#define PLAST_TILE_RAGGED_MIN (1u << 19)
+#endif
 // Workgroup size of a tape launch that re-reads an operand (a broadcast one) from cache. Measured
 // in one process on relu(X + b) over [16384, 4096]: 256 lanes 6372 GB/s, 512 6539, 1024 6593
 // (every tape instantiation stays under 128 VGPRs, no spills); config 1's call unchanged.
@@ -272,6 +289,9 @@ constexpr int kBlock = 256;  // threads per workgroup for streaming kernels (4 w
 #endif
 
 typedef float f4 __attribute__((ext_vector_type(4)));
+// The same at any float's address: one 16-byte access of a lane, which gfx950 takes at 4-byte
+// alignment (a wave still covers one contiguous 1 KiB, at most one line more).
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // The dispatch packet's grid size is 32-bit: a launch holds fewer than 2^32 work-items per
 // dimension, i.e. at most max_blocks(threads) workgroups of `threads` lanes along x.
@@ -290,6 +310,12 @@ template <bool NT>
 __device__ __forceinline__ void store_stream(f4 v, f4 *p) {
   if constexpr (NT) __builtin_nontemporal_store(v, p);
   else *p = v;
+}
+// The same at any float's address.
+template <bool NT>
+__device__ __forceinline__ void store_unit(f4 v, float *p) {
+  if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<f4u *>(p));
+  else *reinterpret_cast<f4u *>(p) = v;
 }
 
 // ------------------------------------------------------------------------- runtime / errors

@@ -1,33 +1,10 @@
-// elementwise.hip — binary and unary ops (forward and backward), the view ops' metadata forwards
-// and GPU backwards, and the fused elementwise-chain op.
+// elementwise.hip — binary and unary ops (forward and backward), and the view ops' metadata forwards
+// and GPU backwards. The fused elementwise-chain op is in fused.hip.
 #include "ew_impl.hpp"
 #include "red_impl.hpp"
 
 namespace plast {
 namespace {
-
-bool check_f32(const Tensor *t, const char *where) {
-  if (t->dtype != FLOAT32) {
-    report_error(where, "unsupported dtype %d", int(t->dtype));
-    return false;
-  }
-  return true;
-}
-
-// Fill the first `rank` axes of operand k from tensor t aligned to `shape` (broadcast rule).
-void set_operand(Space &s, int k, const Tensor *t) {
-  bcast_strides(t, s.shape, s.rank, s.st[k]);
-}
-
-// Operand k follows tensor t's own strides over an identical shape.
-void set_own(Space &s, int k, const Tensor *t) {
-  for (int d = 0; d < s.rank; ++d) s.st[k][d] = t->shape[d] == 1 ? 0 : int64_t(t->strides[d]);
-}
-
-void init_space(Space &s, const uint64_t *shape, int rank) {
-  s.rank = rank;
-  for (int d = 0; d < rank; ++d) s.shape[d] = shape[d];
-}
 
 // ------------------------------------------------------------------------- binary
 
@@ -58,17 +35,6 @@ void binary_forward(const Tensor **in, Tensor *out, const char *where) {
   const void *ins[2] = {a->data, b->data};
   launch_elementwise(BinBody<OP>{}, ins, out->data, s, where);
   finish(where);
-}
-
-// Does tensor t cover every element of `shape` exactly once (no broadcast axis)?
-bool covers(const Tensor *t, const uint64_t *shape, int rank) {
-  if (int(t->ndim) > rank) return false;
-  int lead = rank - int(t->ndim);
-  for (int d = 0; d < rank; ++d) {
-    uint64_t e = d < lead ? 1 : t->shape[d - lead];
-    if (e != shape[d]) return false;
-  }
-  return true;
 }
 
 // One past the largest element offset that shape and strides address (0 for an empty shape).
@@ -275,18 +241,6 @@ void expand_like_forward(const Tensor **in, Tensor *out) {
   }
 }
 
-// A fused chain on the interpreter instantiated for op set OPS and its input count.
-template <uint32_t OPS>
-void launch_tape(const PlastFusedTape &t, uint64_t se, uint32_t neg_simd, int nin,
-                 const void *const *ins, void *out, const Space &s, const char *where) {
-  switch (nin) {
-  case 1: launch_elementwise(TapeBody<1, OPS>{t, se, neg_simd}, ins, out, s, where); break;
-  case 2: launch_elementwise(TapeBody<2, OPS>{t, se, neg_simd}, ins, out, s, where); break;
-  case 3: launch_elementwise(TapeBody<3, OPS>{t, se, neg_simd}, ins, out, s, where); break;
-  default: launch_elementwise(TapeBody<4, OPS>{t, se, neg_simd}, ins, out, s, where); break;
-  }
-}
-
 }  // namespace
 }  // namespace plast
 
@@ -418,78 +372,5 @@ void transpose_backward_hip(float *da, const float *dout, const u64 *a_shape, co
   launch_elementwise(AccumBody{}, ins, da, s, "transpose_backward_hip");
   finish("transpose_backward_hip");
 }
-
-// ---- fused elementwise chain
-
-void fused_elementwise_hip_forward(const Tensor **inputs, Tensor *output, KernelParams params) {
-  const char *where = "fused_elementwise_hip_forward";
-  if (!ensure_init()) return;
-  const PlastFusedTape *tape = reinterpret_cast<const PlastFusedTape *>(uintptr_t(params.dim));
-  if (!tape || tape->num_inputs == 0 || tape->num_inputs > PLAST_TAPE_MAX_INPUTS ||
-      tape->num_ins == 0 || tape->num_ins > PLAST_TAPE_MAX_INS || tape->ins[0].op != TAPE_LOAD) {
-    report_error(where, "malformed tape");
-    return;
-  }
-  for (uint32_t i = 0; i < tape->num_ins; ++i) {
-    const PlastTapeIns &t = tape->ins[i];
-    if (t.op >= TAPE_NUM_OPS || ((t.src == TAPE_SRC_INPUT || t.op == TAPE_LOAD) &&
-                                 t.idx >= tape->num_inputs)) {
-      report_error(where, "tape instruction %u is invalid", i);
-      return;
-    }
-  }
-  if (!check_f32(output, where)) return;
-  for (uint32_t k = 0; k < tape->num_inputs; ++k)
-    if (!check_f32(inputs[k], where)) return;
-  const uint64_t n = numel(output);
-  Space s;
-  init_space(s, output->shape, int(output->ndim));
-  const void *ins[PLAST_TAPE_MAX_INPUTS];
-  bool all_contig = contiguous(output);
-  for (uint32_t k = 0; k < tape->num_inputs; ++k) {
-    if (!covers(inputs[k], output->shape, int(output->ndim))) {
-      // broadcast inputs are fine; shapes that do not broadcast are not
-      uint64_t bs[kMaxRank];
-      int br;
-      if (!broadcast_shape(inputs[k], output, bs, &br) || br != int(output->ndim)) {
-        report_error(where, "input %u does not broadcast to the output", k);
-        return;
-      }
-      all_contig = false;
-    }
-    all_contig = all_contig && contiguous(inputs[k]);
-    set_operand(s, int(k), inputs[k]);
-    ins[k] = inputs[k]->data;
-  }
-  const int nin = int(tape->num_inputs);
-  set_own(s, nin, output);
-  // The reference's neg takes its 8-wide SIMD path (0 - x below simd_end) only when its input and
-  // its output are both contiguous (DEFINE_UNARY_CPU_FORWARD, kernel_macros.h:19-31), and -x
-  // otherwise. Every intermediate of the unfused chain is a fresh contiguous tensor, so only a NEG
-  // reading the loaded input directly or writing the chain's output can meet a strided tensor.
-  uint32_t neg_simd = 0;
-  for (uint32_t i = 1; i < tape->num_ins; ++i) {
-    if (tape->ins[i].op != TAPE_NEG) continue;
-    const bool in_ok = i > 1 || contiguous(inputs[tape->ins[0].idx]);
-    const bool out_ok = i + 1 < tape->num_ins || contiguous(output);
-    if (in_ok && out_ok) neg_simd |= 1u << i;
-  }
-  const uint64_t se = simd_end(n);
-  (void)all_contig;
-  switch (tape_ops_class(*tape)) {
-  case kTapeArith: launch_tape<kTapeArith>(*tape, se, neg_simd, nin, ins, output->data, s, where); break;
-  case kTapeExp: launch_tape<kTapeExp>(*tape, se, neg_simd, nin, ins, output->data, s, where); break;
-  case kTapeExp | kTapeLog:
-    launch_tape<kTapeExp | kTapeLog>(*tape, se, neg_simd, nin, ins, output->data, s, where);
-    break;
-  default:
-    launch_tape<kTapeExp | kTapeLog | kTapeTrig>(*tape, se, neg_simd, nin, ins, output->data, s, where);
-    break;
-  }
-  finish(where);
-}
-
-// fused_elementwise_hip_backward (the one chain that carries a gradient) is in epilogue.hip, beside
-// the bias-gradient kernels it shares.
 
 }  // extern "C"

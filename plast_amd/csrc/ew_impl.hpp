@@ -25,6 +25,8 @@ struct EwArgs {
   uint64_t units;         // float4 units (vec kernel)
   MagicDiv dinner4;       // innermost extent / 4 (vec kernel)
   uint64_t shape64[kMaxRank];  // extents, for the 64-bit generic kernel
+  MagicDiv dinner;             // innermost extent (flat kernel)
+  uint32_t linear;             // bit k: input k is contiguous over the whole space (flat kernel)
 };
 
 
@@ -34,8 +36,29 @@ struct EwArgs {
 // re-read along a broadcast axis use ordinary loads, so the reuse hits in the caches.
 template <bool REUSE>
 __device__ __forceinline__ f4 load_operand(const float *p) {
-  if constexpr (REUSE) return *reinterpret_cast<const f4 *>(p);
-  else return __builtin_nontemporal_load(reinterpret_cast<const f4 *>(p));
+  if constexpr (REUSE) return *reinterpret_cast<const f4u *>(p);
+  else return __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p));
+}
+
+// The first m (1..4) floats at p, the rest 0; and a store of a unit's first m.
+template <bool REUSE>
+__device__ __forceinline__ f4 load_part(const float *p, uint32_t m) {
+  if (m >= 4) return load_operand<REUSE>(p);
+  f4 v = f4(0.0f);
+#pragma unroll
+  for (uint32_t c = 0; c < 3; ++c)
+    if (c < m) v[c] = p[c];
+  return v;
+}
+template <bool NT>
+__device__ __forceinline__ void store_part(f4 v, float *p, uint32_t m) {
+  if (m >= 4) {
+    store_unit<NT>(v, p);
+    return;
+  }
+#pragma unroll
+  for (uint32_t c = 0; c < 3; ++c)
+    if (c < m) p[c] = v[c];
 }
 
 template <bool REUSE, int NIN>
@@ -115,7 +138,88 @@ __global__ __launch_bounds__((VecLaunch<Body, REUSE>::block)) void ew_vec_kernel
   body.template eval_units_with<kEwUnroll>(words, x, idx, valid, r);
 #pragma unroll
   for (int u = 0; u < kEwUnroll; ++u)
-    if (valid[u]) store_stream<kNtStore>(r[u], reinterpret_cast<f4 *>(A.out + oo[u]));
+    if (valid[u]) store_unit<kNtStore>(r[u], A.out + oo[u]);
+}
+
+// Flat kernel: the output is contiguous over the whole space, of any extents, and a lane takes four
+// consecutive elements of it wherever a row ends. Inputs contiguous the same way are read as one
+// 16-byte access; any other input (a broadcast row or column, a strided view) is gathered element
+// by element, its coordinates decoded for each with magic division. What bounds it is the
+// streaming: about 10 instructions an element and decoded axis are far under the 5 a byte the
+// issue rate allows. The generic kernel's one element per lane ran the same spaces at a quarter of
+// the copy's rate.
+//
+// ORANK: axes outside the innermost one (0: every input contiguous; < 0: run-time count). A constant
+// count keeps the decode short and its scalar loads independent: a launch of a few thousand elements
+// lasts as long as its instruction fetches and scalar loads in series (5.4 us with a run-time
+// count unrolled to the maximum rank, measured on 646 elements, against the generic kernel's 2.8).
+template <class Body, int ORANK>
+struct FlatLaunch {
+  static constexpr int block = Body::kTape ? PLAST_TAPE_BLOCK : PLAST_EW_BLOCK;
+  static constexpr int unroll = Body::kTape ? PLAST_TAPE_UNROLL : 1;
+  static constexpr bool xcd = ORANK == 0 && (Body::kTape ? PLAST_TAPE_XCD : PLAST_EW_XCD) != 0;
+};
+
+template <class Body, int ORANK>
+__global__ __launch_bounds__((FlatLaunch<Body, ORANK>::block)) void ew_flat_kernel(EwArgs<Body::NIN> A,
+                                                                                  Body body) {
+  using L = FlatLaunch<Body, ORANK>;
+  constexpr int NIN = Body::NIN, U = L::unroll;
+  const uint32_t bid = L::xcd ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint64_t base = uint64_t(bid) * (L::block * U) + threadIdx.x;
+  const uint32_t words = body.load_words();
+  f4 x[U][NIN];
+  uint64_t idx[U];
+  bool valid[U];
+  uint32_t m[U];  // elements of the unit inside the space
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    idx[u] = (base + uint64_t(u) * L::block) * 4;
+    valid[u] = idx[u] < A.n;
+    m[u] = !valid[u] ? 0 : A.n - idx[u] < 4 ? uint32_t(A.n - idx[u]) : 4u;
+    if constexpr (ORANK == 0) {
+      if (valid[u]) {
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) x[u][k] = load_part<false>(A.in[k] + idx[u], m[u]);
+      }
+    } else {
+      // offsets of the unit's elements (an element past the end decodes the last one)
+      int64_t off[4][NIN];
+#pragma unroll
+      for (uint32_t c = 0; c < 4; ++c) {
+        const uint64_t ec = idx[u] + c < A.n ? idx[u] + c : A.n - 1;
+        uint32_t row = A.dinner.div(uint32_t(ec));
+        const int64_t ci = int64_t(uint32_t(ec) - row * A.dinner.d);
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) off[c][k] = ci * A.ist[k][ORANK > 0 ? ORANK : A.rank - 1];
+        const int nouter = ORANK > 0 ? ORANK : A.rank - 1;
+#pragma unroll
+        for (int j = 0; j < (ORANK > 0 ? ORANK : kMaxRank - 1); ++j) {
+          if (ORANK < 0 && j >= nouter) break;
+          const int d = nouter - 1 - j;
+          const uint32_t nxt = A.dv[d].div(row);
+          const int64_t cd = int64_t(row - nxt * A.dv[d].d);
+          row = nxt;
+#pragma unroll
+          for (int k = 0; k < NIN; ++k) off[c][k] += cd * A.ist[k][d];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < NIN; ++k) {
+        if (A.linear >> k & 1u) {
+          if (valid[u]) x[u][k] = load_part<false>(A.in[k] + idx[u], m[u]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c) x[u][k][c] = A.in[k][off[c][k]];
+        }
+      }
+    }
+  }
+  f4 r[U];
+  body.template eval_units_with<U>(words, x, idx, valid, r);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+    if (valid[u]) store_part<false>(r[u], A.out + idx[u], m[u]);
 }
 
 // Generic kernel: any strides, one element per lane per step. IDX64 selects 64-bit division for
@@ -166,7 +270,8 @@ __global__ __launch_bounds__(kBlock) void ew_generic_kernel(EwArgs<Body::NIN> A,
 // unit-stride along the innermost axis p. Each workgroup owns a 64x64 (q, p) tile of one batch
 // index: transposed inputs are read coalesced along q (float4) into LDS, then every output row is
 // produced coalesced along p (float4) with the other inputs read directly (float4 along p, or a
-// broadcast scalar). Requires extents of q and p divisible by 4 and 16-byte aligned rows.
+// broadcast scalar). Any extents and alignment: units at a ragged edge move their valid elements
+// one by one (config 3's chain at [64, 513, 301]: 59.7 us on the generic kernel).
 constexpr int kTile = 64;
 constexpr int kTilePad = 1;
 
@@ -188,15 +293,17 @@ struct TileArgs {
 
 // DIRECT: whether some operand has role 3 (below); without one, the produce loop issues no global
 // load at all, so nothing in it waits on the memory counter that its stores advance.
-template <class Body, bool DIRECT>
+// RAGGED: an extent of q or p is no multiple of 4, so units at the edges are partial (testing for
+// them costs 3% where none are).
+template <class Body, bool DIRECT, bool RAGGED>
 __global__ __launch_bounds__(kBlock) void ew_tile_kernel(TileArgs<Body::NIN> A, Body body) {
   constexpr int NIN = Body::NIN;
   extern __shared__ float lds[];
-  uint32_t bid = PLAST_TILE_XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
-  const uint32_t tpi = bid % A.tp;
-  bid /= A.tp;
-  const uint32_t tqi = bid % A.tq;
-  uint32_t bi = bid / A.tq;
+  const uint32_t bid = PLAST_TILE_XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
+  const uint32_t bq = A.dtp.div(bid);  // blockIdx = (batch * tq + tqi) * tp + tpi
+  const uint32_t tpi = bid - bq * A.tp;
+  uint32_t bi = A.dtq.div(bq);
+  const uint32_t tqi = bq - bi * A.tq;
   int64_t base[NIN + 1] = {};
   for (int d = A.nbatch - 1; d >= 0; --d) {
     const uint32_t nxt = A.bdv[d].div(bi);
@@ -219,8 +326,9 @@ __global__ __launch_bounds__(kBlock) void ew_tile_kernel(TileArgs<Body::NIN> A, 
     for (int r = 0; r < 4; ++r) {
       const uint32_t b = (t >> 4) + 16 * r;
       if (q0 + a4 < A.eq && p0 + b < A.ep)
-        v[r] = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(
-            A.in[k] + base[k] + int64_t(q0 + a4) * A.qst[k] + int64_t(p0 + b) * A.pst[k]));
+        v[r] = load_part<false>(
+            A.in[k] + base[k] + int64_t(q0 + a4) * A.qst[k] + int64_t(p0 + b) * A.pst[k],
+            RAGGED ? A.eq - (q0 + a4) : 4u);
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -258,7 +366,8 @@ __global__ __launch_bounds__(kBlock) void ew_tile_kernel(TileArgs<Body::NIN> A, 
         if (q0 + a < A.eq) pre[k][r] = in[int64_t(q0 + a) * A.qst[k]];
       }
     } else if (role == 2u) {
-      if (p0 + b4 < A.ep) pre[k] = load_operand<true>(in + int64_t(p0 + b4) * A.pst[k]);
+      if (p0 + b4 < A.ep) pre[k] = load_part<true>(in + int64_t(p0 + b4) * A.pst[k],
+                                                    RAGGED ? A.ep - (p0 + b4) : 4u);
     }
   }
   // consume every prefetched register on every path here, so no wait for them lands after a store
@@ -266,36 +375,51 @@ __global__ __launch_bounds__(kBlock) void ew_tile_kernel(TileArgs<Body::NIN> A, 
   for (int k = 0; k < NIN; ++k) asm volatile("" : "+v"(pre[k]));
   __syncthreads();
   // produce: thread t writes float4 (along p) of output rows a = t/16 + 16r, one row per body
-  // evaluation (fewer live registers)
+  // evaluation (fewer live registers, stores out earlier: config 3's chain at [64, 513, 301] 22.0
+  // us, 23.4 with two rows, 24.2 with this loop rolled)
+  constexpr int TR = 1;
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const uint32_t a = (t >> 4) + 16 * r;
-    f4 x[1][NIN];
-    const uint64_t idx[1] = {0};  // the NEG rule never applies to a strided chain
-    const bool valid[1] = {q0 + a < A.eq && p0 + b4 < A.ep};
+  for (int h = 0; h < 4 / TR; ++h) {
+    f4 x[TR][NIN];
+    uint64_t idx[TR];
+    bool valid[TR];
 #pragma unroll
-    for (int k = 0; k < NIN; ++k) {
-      const uint32_t role = roles >> (2 * k) & 3u;
-      if (role == 0u) {
-        const float *tile = lds + (slots >> (2 * k) & 3u) * (kTile * (kTile + kTilePad));
+    for (int u = 0; u < TR; ++u) {
+      const int r = h * TR + u;
+      const uint32_t a = (t >> 4) + 16 * r;
+      idx[u] = 0;  // the NEG rule never applies to a strided chain
+      valid[u] = q0 + a < A.eq && p0 + b4 < A.ep;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) x[0][k][c] = tile[(b4 + c) * (kTile + kTilePad) + a];
-      } else if (role == 1u) {
-        x[0][k] = f4(pre[k][r]);
-      } else if (role == 2u) {
-        x[0][k] = pre[k];
-      } else if (DIRECT && valid[0]) {
-        x[0][k] = load_operand<true>(A.in[k] + base[k] + int64_t(q0 + a) * A.qst[k] +
-                                     int64_t(p0 + b4) * A.pst[k]);
-      } else {
-        x[0][k] = f4(0.0f);
+      for (int k = 0; k < NIN; ++k) {
+        const uint32_t role = roles >> (2 * k) & 3u;
+        if (role == 0u) {
+          const float *tile = lds + (slots >> (2 * k) & 3u) * (kTile * (kTile + kTilePad));
+#pragma unroll
+          for (int c = 0; c < 4; ++c) x[u][k][c] = tile[(b4 + c) * (kTile + kTilePad) + a];
+        } else if (role == 1u) {
+          const f4 s = pre[k];
+          x[u][k] = f4(r == 0 ? s[0] : r == 1 ? s[1] : r == 2 ? s[2] : s[3]);
+        } else if (role == 2u) {
+          x[u][k] = pre[k];
+        } else if (DIRECT && valid[u]) {
+          x[u][k] = load_part<true>(A.in[k] + base[k] + int64_t(q0 + a) * A.qst[k] +
+                                        int64_t(p0 + b4) * A.pst[k],
+                                    RAGGED ? A.ep - (p0 + b4) : 4u);
+        } else {
+          x[u][k] = f4(0.0f);
+        }
       }
     }
-    f4 res[1];
-    body.template eval_units_with<1>(words, x, idx, valid, res);
-    if (valid[0])
-      store_stream<PLAST_TILE_NT_STORE>(res[0], reinterpret_cast<f4 *>(A.out + base[NIN] +
-                                                   int64_t(q0 + a) * A.qst[NIN] + int64_t(p0 + b4)));
+    f4 res[TR];
+    body.template eval_units_with<TR>(words, x, idx, valid, res);
+#pragma unroll
+    for (int u = 0; u < TR; ++u) {
+      const uint32_t a = (t >> 4) + 16 * (h * TR + u);
+      if (valid[u])
+        store_part<PLAST_TILE_NT_STORE>(res[u], A.out + base[NIN] + int64_t(q0 + a) * A.qst[NIN] +
+                                                    int64_t(p0 + b4),
+                                        RAGGED ? A.ep - (p0 + b4) : 4u);
+    }
   }
 }
 
@@ -352,8 +476,7 @@ __global__ __launch_bounds__(kBlock) void ew_tile_fixed_kernel(TileArgs<Body::NI
       const float *src = in + (q0 + l4) * A.qst[k] + (p0 + r16) * A.pst[k];
       const int64_t step = 16 * A.pst[k];
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        v[k][r] = __builtin_nontemporal_load(reinterpret_cast<const f4 *>(src + r * step));
+      for (int r = 0; r < 4; ++r) v[k][r] = load_operand<false>(src + r * step);
     } else if constexpr (role == 1) {
       const float *src = in + (q0 + r16) * A.qst[k];
       const int64_t step = 16 * A.qst[k];
@@ -419,7 +542,7 @@ __global__ __launch_bounds__(kBlock) void ew_tile_fixed_kernel(TileArgs<Body::NI
     body.template eval_units_with<TR>(words, x, idx, valid, res);
 #pragma unroll
     for (int u = 0; u < TR; ++u)
-      store_stream<PLAST_TILE_NT_STORE>(res[u], reinterpret_cast<f4 *>(dst + (h * TR + u) * dstep));
+      store_unit<PLAST_TILE_NT_STORE>(res[u], dst + (h * TR + u) * dstep);
   }
 }
 
@@ -479,7 +602,7 @@ template <class Body>
 bool try_tile(const Body &body, const void *const *in, void *out, const Space &s) {
   constexpr int NIN = Body::NIN;
   const int r = s.rank;
-  if (r < 2 || !aligned16(out) || s.st[NIN][r - 1] != 1) return false;
+  if (r < 2 || s.st[NIN][r - 1] != 1) return false;
   const int p = r - 1;
   int q = -1;
   for (int k = 0; k < NIN; ++k) {
@@ -492,8 +615,7 @@ bool try_tile(const Body &body, const void *const *in, void *out, const Space &s
     q = qk;
   }
   if (q < 0) return false;
-  if (s.shape[p] % 4 || s.shape[q] % 4 || s.shape[p] >= (1u << 31) || s.shape[q] >= (1u << 31))
-    return false;
+  if (s.shape[p] >= (1u << 31) || s.shape[q] >= (1u << 31)) return false;
   TileArgs<NIN> A;
   memset(&A, 0, sizeof A);
   uint32_t slots = 0;
@@ -502,29 +624,17 @@ bool try_tile(const Body &body, const void *const *in, void *out, const Space &s
     A.pst[k] = s.st[k][p];
     if (k < NIN) {
       A.in[k] = static_cast<const float *>(in[k]);
-      const bool staged = A.pst[k] != 0 && A.pst[k] != 1;
-      const bool vec_ok = staged ? (A.pst[k] % 4 == 0 && aligned16(in[k]))
-                                 : (A.pst[k] == 0 || aligned16(in[k]));
-      if (!vec_ok) return false;
-      if (staged) {
+      if (A.pst[k] != 0 && A.pst[k] != 1) {
         A.lds_mask |= 1u << k;
         A.lds_slot[k] = slots++;
-      } else if (A.pst[k] == 1 && A.qst[k] % 4 != 0) {
-        return false;
       }
-    } else if (A.qst[k] % 4 != 0) {
-      return false;
     }
   }
   uint64_t batch = 1;
   int nb = 0;
   for (int d = 0; d < p; ++d) {
     if (d == q) continue;
-    for (int k = 0; k <= NIN; ++k) {
-      A.bst[k][nb] = s.st[k][d];
-      const bool f4_operand = k == NIN || !((A.lds_mask >> k & 1u) == 0 && A.pst[k] == 0);
-      if (f4_operand && s.st[k][d] % 4 != 0) return false;
-    }
+    for (int k = 0; k <= NIN; ++k) A.bst[k][nb] = s.st[k][d];
     A.bdv[nb] = MagicDiv::make(uint32_t(s.shape[d]));
     batch *= s.shape[d];
     ++nb;
@@ -538,6 +648,7 @@ bool try_tile(const Body &body, const void *const *in, void *out, const Space &s
   const uint64_t blocks = batch * A.tq * A.tp;
   if (blocks > max_blocks(kBlock)) return false;
   const size_t lds_bytes = size_t(slots) * kTile * (kTile + kTilePad) * sizeof(float);
+  if (lds_bytes > size_t(64) * 1024) return false;  // four staged operands and more
   bool direct = false;
   uint32_t roles = 0;
   for (int k = 0; k < NIN; ++k) {
@@ -548,13 +659,43 @@ bool try_tile(const Body &body, const void *const *in, void *out, const Space &s
   A.dtq = MagicDiv::make(A.tq);
   A.dtp = MagicDiv::make(A.tp);
   const bool full = A.eq % kTile == 0 && A.ep % kTile == 0;
+  if (!full && batch * A.eq * A.ep < PLAST_TILE_RAGGED_MIN) return false;
+  // the tile kernels apply the NEG rule's SIMD form to every element (a whole number of blocks)
+  if (!body.index_free() && batch * A.eq * A.ep % 8 != 0) return false;
   if (full && launch_tile_fixed(A, body, roles, unsigned(blocks), lds_bytes)) return true;
-  if (direct) ew_tile_kernel<Body, true><<<unsigned(blocks), kBlock, lds_bytes, stream()>>>(A, body);
-  else ew_tile_kernel<Body, false><<<unsigned(blocks), kBlock, lds_bytes, stream()>>>(A, body);
+  const bool ragged = A.eq % 4 != 0 || A.ep % 4 != 0;
+  const unsigned grid = unsigned(blocks);
+  if (direct && ragged) ew_tile_kernel<Body, true, true><<<grid, kBlock, lds_bytes, stream()>>>(A, body);
+  else if (direct) ew_tile_kernel<Body, true, false><<<grid, kBlock, lds_bytes, stream()>>>(A, body);
+  else if (ragged) ew_tile_kernel<Body, false, true><<<grid, kBlock, lds_bytes, stream()>>>(A, body);
+  else ew_tile_kernel<Body, false, false><<<grid, kBlock, lds_bytes, stream()>>>(A, body);
   return true;
 }
 
 // ------------------------------------------------------------------------- host dispatch
+
+inline bool check_f32(const Tensor *t, const char *where) {
+  if (t->dtype != FLOAT32) {
+    report_error(where, "unsupported dtype %d", int(t->dtype));
+    return false;
+  }
+  return true;
+}
+
+// Fill the first `rank` axes of operand k from tensor t aligned to `shape` (broadcast rule).
+inline void set_operand(Space &s, int k, const Tensor *t) {
+  bcast_strides(t, s.shape, s.rank, s.st[k]);
+}
+
+// Operand k follows tensor t's own strides over an identical shape.
+inline void set_own(Space &s, int k, const Tensor *t) {
+  for (int d = 0; d < s.rank; ++d) s.st[k][d] = t->shape[d] == 1 ? 0 : int64_t(t->strides[d]);
+}
+
+inline void init_space(Space &s, const uint64_t *shape, int rank) {
+  s.rank = rank;
+  for (int d = 0; d < rank; ++d) s.shape[d] = shape[d];
+}
 
 // Returns false (launching nothing) when the grid would exceed the dispatch limit.
 template <class Body, bool REUSE>
@@ -610,20 +751,18 @@ bool launch_elementwise(const Body &body, const void *const *in, void *out, Spac
   const uint64_t inner = s.shape[in_ax];
   A.reused = reused_mask<NIN>(s);
 
+  const bool small = Body::kTape && n <= PLAST_TAPE_SMALL;
+
   // --- vectorised path
-  bool vec = (n < (uint64_t(1) << 32) || in_ax == 0) && inner % 4 == 0 && s.st[NIN][in_ax] == 1 && aligned16(out);
-  for (int k = 0; k < NIN && vec; ++k) {
+  bool vec = (n < (uint64_t(1) << 32) || in_ax == 0) && inner % 4 == 0 && s.st[NIN][in_ax] == 1;
+  bool transposed = false;  // some input's unit-stride axis is not the innermost
+  for (int k = 0; k < NIN; ++k) {
     const int64_t si = s.st[k][in_ax];
-    if (si == 0) {
-      A.bcast_inner |= 1u << k;
-    } else {
-      vec = si == 1 && aligned16(in[k]);
-    }
+    if (si == 0) A.bcast_inner |= 1u << k;
+    else if (si != 1) transposed = true;
   }
-  for (int d = 0; d < in_ax && vec; ++d)
-    for (int k = 0; k <= NIN && vec; ++k)
-      if ((k == NIN || !(A.bcast_inner & (1u << k))) && s.st[k][d] % 4 != 0) vec = false;
-  if (vec) {
+  vec = vec && !transposed;
+  if (vec && !small) {
     A.units = n / 4;
     A.dinner4 = MagicDiv::make(uint32_t(inner / 4));
     for (int d = 0; d < in_ax; ++d) A.dv[d] = MagicDiv::make(uint32_t(s.shape[d]));
@@ -634,7 +773,34 @@ bool launch_elementwise(const Body &body, const void *const *in, void *out, Spac
   }
 
   // --- transposed-operand path
-  if (n < (uint64_t(1) << 32) && try_tile(body, in, out, s)) return true;
+  if (!small && n < (uint64_t(1) << 32) && transposed && try_tile(body, in, out, s)) return true;
+
+  // --- flat path: rows that are no whole float4, over a contiguous output
+  if (!small && !transposed && n < (uint64_t(1) << 32)) {
+    uint64_t want = 1;
+    uint32_t contig = (2u << NIN) - 1;  // operands (output last) contiguous over the whole space
+    for (int d = in_ax; d >= 0; --d) {
+      for (int k = 0; k <= NIN; ++k)
+        if (s.st[k][d] != int64_t(want)) contig &= ~(1u << k);
+      want *= s.shape[d];
+    }
+    if (contig >> NIN & 1u) {
+      A.linear = contig;
+      A.dinner = MagicDiv::make(uint32_t(inner));
+      for (int d = 0; d < in_ax; ++d) A.dv[d] = MagicDiv::make(uint32_t(s.shape[d]));
+      const auto launch = [&](auto orank) {
+        constexpr int R = decltype(orank)::value;
+        using L = FlatLaunch<Body, R>;
+        constexpr uint64_t per = uint64_t(L::block) * L::unroll;
+        ew_flat_kernel<Body, R><<<unsigned(((n + 3) / 4 + per - 1) / per), L::block, 0, stream()>>>(A, body);
+      };
+      if (contig == (2u << NIN) - 1) launch(std::integral_constant<int, 0>{});
+      else if (in_ax == 1) launch(std::integral_constant<int, 1>{});
+      else if (in_ax == 2) launch(std::integral_constant<int, 2>{});
+      else launch(std::integral_constant<int, -1>{});
+      return true;
+    }
+  }
 
   // --- generic path
   uint64_t blocks = (n + kBlock - 1) / kBlock;
