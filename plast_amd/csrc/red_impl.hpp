@@ -208,6 +208,7 @@ struct RedArgs {
   uint64_t len;                // reduced extent (all reduced axes together)
   uint64_t rows;               // rows (rows kernel) / outer count (cols kernel)
   uint64_t inner;              // kept innermost extent (cols kernel)
+  uint32_t lanes;              // lanes of a wave that hold columns (cols kernel)
   uint32_t segs;               // segments per row / chunks of the reduced axis
   uint64_t seglen;
   uint32_t vec_mask;           // bit k: operand k is streamed with float4 loads (else splat)
@@ -216,6 +217,8 @@ struct RedArgs {
   float divisor;               // Mean
   int nx;                      // reduced axes outside the innermost reduced one (MULTI kernels)
   MagicDiv drun;               // extent of the innermost reduced axis (nx > 0)
+  MagicDiv dunits;             // float4 units of one run of it, the last one partial
+  uint64_t vlen;               // 4 * the units of every run (what MULTI rows with VEC segment)
   MagicDiv xdv[kMaxRank];      // extents of the outer reduced axes, outermost first
   int64_t xst[NIN][kMaxRank];  // operand strides along them
 };
@@ -393,21 +396,41 @@ __device__ float serial_sum_wave(const RedArgs<NIN> &A, const Prod &prod, const 
 
 constexpr int kRowUnroll = PLAST_ROW_UNROLL;  // float4 loads in flight per lane per operand
 
-// The float4 unit at reduced position i of every operand (a broadcast operand's value splatted).
+// The float4 unit at reduced position i (a multiple of 4) of every operand, a broadcast operand's
+// value splatted. MULTI: i / 4 counts units of runs whose last unit may be partial; that one is read
+// from four elements before the run's end. Returns the reduced index of the unit's first element;
+// the first `skip` elements belong to the unit before.
 template <bool MULTI, int NIN>
-__device__ __forceinline__ void load_unit(const RedArgs<NIN> &A, const int64_t *base, uint64_t i,
-                                          f4 *x) {
+__device__ __forceinline__ uint64_t load_unit(const RedArgs<NIN> &A, const int64_t *base, uint64_t i,
+                                              f4 *x, uint32_t &skip) {
   int64_t off[NIN];
-  if constexpr (MULTI) reduced_offset<true>(A, i, off);
+  if constexpr (MULTI) {
+    const uint32_t run = A.dunits.div(uint32_t(i / 4));
+    const uint32_t at = 4 * (uint32_t(i / 4) - run * A.dunits.d);
+    const uint32_t pos = at + 4 <= A.drun.d ? at : A.drun.d - 4;
+    skip = at - pos;
+    i = uint64_t(run) * A.drun.d + pos;
+    reduced_offset<true>(A, i, off);
+  } else {
+    skip = 0;
+  }
 #pragma unroll
   for (int k = 0; k < NIN; ++k) {
     const float *src = A.in[k] + base[k];
     if (A.vec_mask >> k & 1u)
       x[k] = __builtin_nontemporal_load(
-          reinterpret_cast<const f4 *>(src + (MULTI ? off[k] : int64_t(i))));
+          reinterpret_cast<const f4u *>(src + (MULTI ? off[k] : int64_t(i))));
     else
       x[k] = f4(src[MULTI ? off[k] : 0]);
   }
+  return i;
+}
+
+// The reduced index at which MULTI position i (a multiple of 4) starts.
+template <int NIN>
+__device__ __forceinline__ uint64_t run_index(const RedArgs<NIN> &A, uint64_t i) {
+  const uint32_t run = A.dunits.div(uint32_t(i / 4));
+  return uint64_t(run) * A.drun.d + 4 * (uint32_t(i / 4) - run * A.dunits.d);
 }
 
 template <class Prod, class Comb, bool VEC, bool MULTI>
@@ -423,7 +446,10 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
   int64_t base[NIN], tbase;
   decode_outer(A, row, base, tbase);
   const uint64_t b = uint64_t(seg) * A.seglen;
-  const uint64_t e = b + A.seglen < A.len ? b + A.seglen : A.len;
+  const uint64_t total = VEC && MULTI ? A.vlen : A.len;
+  const uint64_t e = b + A.seglen < total ? b + A.seglen : total;
+  // end of the whole float4 units; the up to three elements left are lanes 0 to 2's
+  const uint64_t eu = MULTI ? e : e - (e & 3);
 
   Part p;
   if constexpr (Comb::kExact) {
@@ -436,18 +462,21 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
       nan = nan || (x != x);
     };
     if constexpr (VEC) {
-      for (uint64_t i0 = b + uint64_t(lane) * 4; i0 < e; i0 += 256 * kRowUnroll) {
+      for (uint64_t i0 = b + uint64_t(lane) * 4; i0 < eu; i0 += 256 * kRowUnroll) {
         f4 x[kRowUnroll][NIN];
+        uint64_t at[kRowUnroll];
+        uint32_t skip[kRowUnroll];
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
           const uint64_t i = i0 + uint64_t(u) * 256;
-          if (i < e) load_unit<MULTI>(A, base, i, x[u]);
+          if (i < eu) at[u] = load_unit<MULTI>(A, base, i, x[u], skip[u]);
         }
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
-          if (i0 + uint64_t(u) * 256 >= e) continue;
+          if (i0 + uint64_t(u) * 256 >= eu) continue;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
+            if (MULTI && uint32_t(c) < skip[u]) continue;
             float v[NIN];
 #pragma unroll
             for (int k = 0; k < NIN; ++k) v[k] = x[u][k][c];
@@ -455,6 +484,7 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
           }
         }
       }
+      if (!MULTI && eu + lane < e) take(value_at_as<false>(A, prod, base, eu + lane));
     } else {
       for (uint64_t i = b + lane; i < e; i += 64) take(value_at_as<MULTI>(A, prod, base, i));
     }
@@ -463,7 +493,10 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
     if (!nan && m != 0.0f) {
       p = ExtPart{m, e > b ? kNonEmpty : 0u};
     } else if (e > b) {
-      p = exact_range<IS_MAX>(A, prod, base, b, e, lane);
+      if constexpr (VEC && MULTI)
+        p = exact_range<IS_MAX>(A, prod, base, run_index(A, b), run_index(A, e), lane);
+      else
+        p = exact_range<IS_MAX>(A, prod, base, b, e, lane);
     } else {
       p = Comb::empty();
     }
@@ -471,26 +504,30 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
     p = Comb::empty();
     Part acc[4] = {Comb::empty(), Comb::empty(), Comb::empty(), Comb::empty()};
     if constexpr (VEC) {
-      for (uint64_t i0 = b + uint64_t(lane) * 4; i0 < e; i0 += 256 * kRowUnroll) {
+      for (uint64_t i0 = b + uint64_t(lane) * 4; i0 < eu; i0 += 256 * kRowUnroll) {
         f4 x[kRowUnroll][NIN];
+        uint64_t at[kRowUnroll];
+        uint32_t skip[kRowUnroll];
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
           const uint64_t i = i0 + uint64_t(u) * 256;
-          if (i < e) load_unit<MULTI>(A, base, i, x[u]);
+          if (i < eu) at[u] = load_unit<MULTI>(A, base, i, x[u], skip[u]);
         }
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
-          const uint64_t i = i0 + uint64_t(u) * 256;
-          if (i >= e) continue;
+          if (i0 + uint64_t(u) * 256 >= eu) continue;
 #pragma unroll
           for (int c = 0; c < 4; ++c) {
+            if (MULTI && uint32_t(c) < skip[u]) continue;
             float v[NIN];
 #pragma unroll
             for (int k = 0; k < NIN; ++k) v[k] = x[u][k][c];
-            Comb::next(acc[c], prod.eval(v), int64_t(i + c));
+            Comb::next(acc[c], prod.eval(v), int64_t(at[u] + c));
           }
         }
       }
+      if (!MULTI && eu + lane < e)
+        Comb::next(acc[0], value_at_as<false>(A, prod, base, eu + lane), int64_t(eu + lane));
       p = Comb::merge(Comb::merge(acc[0], acc[1]), Comb::merge(acc[2], acc[3]));
     } else {
       for (uint64_t i = b + lane; i < e; i += 64) {
@@ -510,6 +547,94 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
   } else {
     static_cast<Part *>(A.part)[task] = p;
   }
+}
+
+// Rows of at most 16 * L elements: L lanes per row, 64 / L rows per wave, so a wave reads one
+// contiguous stretch of rows (a wave per row of 77 floats kept 20 of its 64 lanes on 308 bytes, and
+// took 15 us for 15 MB). Each lane holds up to four float4 units of its row, all loaded before the
+// first is used, and the up to three elements left. A row whose fast value could differ from the
+// reference's (max/min of a NaN or a zero extreme, a non-finite sum) is redone by the whole wave.
+template <class Prod, class Comb, int L>
+__global__ __launch_bounds__(kBlock) void red_rows_short_kernel(RedArgs<Prod::NIN> A, Prod prod) {
+  constexpr int NIN = Prod::NIN, U = 4;
+  using Part = typename Comb::Part;
+  const int lane = threadIdx.x & 63, l = lane % L;
+  const uint64_t row0 = (uint64_t(blockIdx.x) * (kBlock / 64) + (threadIdx.x >> 6)) * (64 / L);
+  if (row0 >= A.rows) return;  // whole wave
+  const uint64_t row = row0 + lane / L;
+  const bool valid = row < A.rows;
+  int64_t base[NIN], tbase;
+  decode_outer(A, uint32_t(valid ? row : A.rows - 1), base, tbase);
+  const uint32_t len = uint32_t(A.len), units = len / 4;
+  f4 x[U][NIN];
+  if (units) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      // a lane past the row reads its last unit: the loads take no branch
+      const uint32_t q = uint32_t(l) + u * L;
+      uint32_t skip;
+      load_unit<false>(A, base, uint64_t(q < units ? q : units - 1) * 4, x[u], skip);
+    }
+  }
+  const auto each = [&](auto &&take) {
+    if (units) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const uint32_t q = uint32_t(l) + u * L;
+        if (q >= units) continue;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          float v[NIN];
+#pragma unroll
+          for (int k = 0; k < NIN; ++k) v[k] = x[u][k][c];
+          take(c, prod.eval(v), int64_t(q * 4 + c));
+        }
+      }
+    }
+    for (uint32_t i = units * 4 + l; i < len; i += L)
+      take(0, value_at_as<false>(A, prod, base, i), int64_t(i));
+  };
+  Part p = Comb::empty();
+  bool redo;
+  if constexpr (Comb::kExact) {
+    constexpr bool IS_MAX = std::is_same<Comb, ExtComb<true>>::value;
+    float m = IS_MAX ? -__builtin_huge_valf() : __builtin_huge_valf();
+    uint32_t nan = 0;
+    each([&](int, float y, int64_t) {
+      m = IS_MAX ? fmaxf(m, y) : fminf(m, y);
+      nan |= y != y ? 1u : 0u;
+    });
+#pragma unroll
+    for (int s = L / 2; s >= 1; s >>= 1) {
+      const float o = __shfl_xor(m, s);
+      m = IS_MAX ? fmaxf(m, o) : fminf(m, o);
+      nan |= uint32_t(__shfl_xor(int(nan), s));
+    }
+    p = ExtPart{m, kNonEmpty};
+    redo = nan != 0 || m == 0.0f;
+  } else {
+    Part acc[4] = {Comb::empty(), Comb::empty(), Comb::empty(), Comb::empty()};
+    each([&](int c, float y, int64_t i) { Comb::next(acc[c], y, i); });
+    p = Comb::merge(Comb::merge(acc[0], acc[1]), Comb::merge(acc[2], acc[3]));
+#pragma unroll
+    for (int s = L / 2; s >= 1; s >>= 1) p = Comb::merge(p, Comb::shfl(p, s));
+    redo = false;
+    if constexpr (kSerialSum<Comb>) redo = !finite_sum(p);
+  }
+  if constexpr (Comb::kExact || kSerialSum<Comb>) {
+    for (uint64_t todo = __ballot(redo && valid && l == 0); todo; todo &= todo - 1) {
+      const int first = __ffsll((unsigned long long)todo) - 1;  // the row's first lane
+      int64_t rb[NIN], rt;
+      decode_outer(A, uint32_t(row0 + first / L), rb, rt);
+      Part r;
+      if constexpr (Comb::kExact)
+        r = exact_range<std::is_same<Comb, ExtComb<true>>::value>(A, prod, rb, 0, A.len, lane);
+      else
+        r = serial_sum_wave(A, prod, rb, A.len, __shfl(p, first), lane);
+      if (lane == first) p = r;
+    }
+  }
+  if (l == 0 && valid) store_final<Comb>(A.out, tbase, p, A.post, A.divisor);
 }
 
 // Combine the segments of each row in index order.
@@ -596,10 +721,8 @@ constexpr int kColUnroll = Prod::NIN == 1   ? PLAST_COL_UNROLL
                                             : PLAST_COL_UNROLL3;
 
 template <class Prod>
-__device__ __forceinline__ void store_col(f4 *p, f4 v) {
-  constexpr bool nt = PLAST_COL_NT_STORE == 1 || (PLAST_COL_NT_STORE == -1 && StoresOther<Prod>::value);
-  if constexpr (nt) __builtin_nontemporal_store(v, p);
-  else *p = v;
+__device__ __forceinline__ void store_col(float *p, f4 v) {
+  store_unit<PLAST_COL_NT_STORE == 1 || (PLAST_COL_NT_STORE == -1 && StoresOther<Prod>::value)>(v, p);
 }
 
 template <class Prod>
@@ -625,7 +748,8 @@ struct ExtFast {
 // zero (the cases where order decides the bits).
 // ALLV (with VEC): every operand is streamed with float4 loads, so the loads take no branch on
 // the operand mask (a broadcast operand's splat makes the compiler wait for each load in turn).
-template <class Prod, class Comb, bool VEC, bool ALLV, bool MULTI>
+// RAGGED (with VEC): a row's last unit is partial, or its slices hold fewer than 64 lanes.
+template <class Prod, class Comb, bool VEC, bool ALLV, bool MULTI, bool RAGGED>
 __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, Prod prod,
                                                           uint32_t xblocks) {
   constexpr int NIN = Prod::NIN;
@@ -641,8 +765,13 @@ __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, 
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const uint32_t bx = blockIdx.x, chunk = blockIdx.y;
   const uint32_t o = bx / xblocks;
-  const uint64_t j = (uint64_t(bx - o * xblocks) * 64 + lane) * W;
-  const bool active = j < A.inner;  // no early return: the workgroup meets at a barrier
+  // the lane's columns: W from jo on; a partial unit at the end of a row is read from four columns
+  // before the end, and its first `skip` columns are the lane before's
+  const uint32_t lanes = RAGGED ? A.lanes : 64;
+  const uint64_t jo = (uint64_t(bx - o * xblocks) * lanes + lane) * W;
+  const bool active = (!RAGGED || uint32_t(lane) < lanes) && jo < A.inner;  // no early return: a
+  const uint64_t j = !RAGGED || jo + W <= A.inner ? jo : A.inner - W;       // barrier follows
+  const int skip = RAGGED && active ? int(jo - j) : 0;
   int64_t base[NIN], lbase[NIN], tbase;
   decode_outer(A, o, base, tbase);
 #pragma unroll
@@ -675,7 +804,7 @@ __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, 
         const float *src = A.in[k] + lbase[k] + roff[k];
         if constexpr (VEC) {
           const f4 v = (ALLV || (A.vec_mask >> k & 1u))
-                           ? __builtin_nontemporal_load(reinterpret_cast<const f4 *>(src))
+                           ? __builtin_nontemporal_load(reinterpret_cast<const f4u *>(src))
                            : f4(src[0]);
 #pragma unroll
           for (int c = 0; c < W; ++c) xv[u][k][c] = v[c];
@@ -705,10 +834,17 @@ __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, 
       }
       if constexpr (kStores<Prod>) {
         float *dst = prod.dst + base[0] + int64_t(r) * A.rst[0];
-        if constexpr (VEC)
-          store_col<Prod>(reinterpret_cast<f4 *>(dst), f4{yv[0], yv[1], yv[2], yv[3]});
-        else
+        if constexpr (VEC) {
+          if (skip == 0) {
+            store_col<Prod>(dst, f4{yv[0], yv[1], yv[2], yv[3]});
+          } else {
+#pragma unroll
+            for (int c = 1; c < 4; ++c)
+              if (c >= skip) dst[c] = yv[c];
+          }
+        } else {
           dst[0] = yv[0];
+        }
       }
     }
   }
@@ -719,6 +855,7 @@ __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, 
 
 #pragma unroll
   for (int c = 0; c < W; ++c) {
+    const bool mine = c >= skip;
     Part p;
     if constexpr (kExt) {
       float m = sh[0][lane * W + c].m;
@@ -755,6 +892,7 @@ __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, 
         }
       }
     }
+    if (!mine) continue;
     if (A.segs == 1) {
       store_final<Comb>(A.out, tbase + int64_t(j + c) * A.tkst, p, A.post, A.divisor);
     } else {
@@ -784,8 +922,10 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
   const uint32_t b = PLAST_COL_SMALL_XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x;
   const uint32_t o = b / xblocks;
   const uint64_t j0 = uint64_t(b - o * xblocks) * (4 * S4);  // the slice's first column
-  const uint64_t j = j0 + 4 * c4;
-  const bool active = j < A.inner;
+  // a partial unit at the end of a row is read from four columns before the end (see red_cols_kernel)
+  const bool active = j0 + 4 * c4 < A.inner;
+  const uint64_t j = j0 + 4 * c4 + 4 <= A.inner ? j0 + 4 * c4 : A.inner - 4;
+  const int skip = active ? int(j0 + 4 * c4 - j) : 0;
   int64_t base0[NIN], base[NIN], lbase[NIN], tbase;
   decode_outer(A, o, base0, tbase);
 #pragma unroll
@@ -803,7 +943,7 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
 #pragma unroll
       for (int k = 0; k < NIN; ++k) {
         const float *src = A.in[k] + lbase[k] + int64_t(r) * A.rst[k];
-        xv[u][k] = (ALLV || (A.vec_mask >> k & 1u)) ? *reinterpret_cast<const f4 *>(src)
+        xv[u][k] = (ALLV || (A.vec_mask >> k & 1u)) ? *reinterpret_cast<const f4u *>(src)
                                                     : f4(src[0]);
       }
     }
@@ -821,8 +961,16 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
         f[c] = f[c] + y;
         yv[c] = stored_value(prod, v, y);
       }
-      if constexpr (kStores<Prod>)  // a storing producer also writes each value it sums
-        store_col<Prod>(reinterpret_cast<f4 *>(prod.dst + base[0] + int64_t(r) * A.rst[0]), yv);
+      if constexpr (kStores<Prod>) {  // a storing producer also writes each value it sums
+        float *dst = prod.dst + base[0] + int64_t(r) * A.rst[0];
+        if (skip == 0) {
+          store_col<Prod>(dst, yv);
+        } else {
+#pragma unroll
+          for (int c = 1; c < 4; ++c)
+            if (c >= skip) dst[c] = yv[c];
+        }
+      }
     }
   }
   // the wave's row groups (lanes c4, c4 + S4, ...) merge pairwise with a fixed butterfly
@@ -833,9 +981,11 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
   if (lane < uint32_t(S4)) sh[wv][lane] = f;
   __syncthreads();
   if (t >= uint32_t(4 * S4)) return;
-  // lane t finishes output column j0 + t: the waves' partials in wave order
-  const uint64_t jc = j0 + t;
-  if (jc >= A.inner) return;
+  // lane t finishes one output column, element t % 4 of unit t / 4: the waves' partials in wave order
+  const uint64_t ju = j0 + (t & ~3u);  // the unit's first column, before a partial one moves back
+  if (ju >= A.inner) return;
+  const uint64_t jc = (ju + 4 <= A.inner ? ju : A.inner - 4) + (t & 3u);
+  if (jc < ju) return;
   float p = sh[0][t / 4][t % 4];
 #pragma unroll
   for (int w = 1; w < kBlock / 64; ++w) p = p + sh[w][t / 4][t % 4];
@@ -846,6 +996,155 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
     p = serial_sum_lane(A, prod, bc, A.len);
   }
   store_final<SumComb>(A.out, tbase + int64_t(jc) * A.tkst, p, A.post, A.divisor);
+}
+
+// Narrow columns: operands contiguous over [len, inner] (or constant along the reduced axis), with
+// fewer columns than a wave's slice. The rows are read as one flat array: T lanes of the workgroup
+// take consecutive float4 units, 4 T floats being a whole number R of rows, so the columns a lane's
+// four elements fall in are the same in every step, whatever inner is, and no lane idles over a short
+// row (a slice of 64 lanes keeps 3 of them on 10 columns). The workgroup's 4 T sums, R per column,
+// are merged through LDS eight rows at a time, in order.
+constexpr int kFlatBlock = 512;
+template <class Prod>
+constexpr int kFlatUnroll = Prod::NIN == 1 ? 4 : 2;
+struct FlatCols {
+  uint32_t T, R;
+  MagicDiv dinner;
+};
+
+template <class Prod, class Comb>
+__global__ __launch_bounds__(kFlatBlock) void red_cols_flat_kernel(RedArgs<Prod::NIN> A, Prod prod,
+                                                                   FlatCols F) {
+  constexpr int NIN = Prod::NIN, kU = kFlatUnroll<Prod>;
+  using Part = typename Comb::Part;
+  constexpr bool kExt = Comb::kExact;
+  constexpr bool IS_MAX = std::is_same<Comb, ExtComb<true>>::value;
+  using Fast = typename std::conditional<kExt, ExtFast, Part>::type;
+  __shared__ Fast sh[kFlatBlock * 4];
+  const uint32_t t = threadIdx.x, o = blockIdx.x, inner = uint32_t(A.inner);
+  int64_t base[NIN], tbase;
+  decode_outer(A, o, base, tbase);
+  const uint64_t k0 = uint64_t(blockIdx.y) * A.seglen;
+  const uint64_t k1 = k0 + A.seglen < A.len ? k0 + A.seglen : A.len;
+  const uint64_t nf = (k1 - k0) * inner;  // floats of the chunk
+  const auto merge = [](const Fast &a, const Fast &b) {
+    if constexpr (kExt) return Fast{IS_MAX ? fmaxf(a.m, b.m) : fminf(a.m, b.m), a.nan | b.nan};
+    else return Comb::merge(a, b);
+  };
+  Fast f[4];
+  uint32_t row[4];
+  f4 fixed[NIN];  // the lane's columns of an operand constant along the reduced axis
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    if constexpr (kExt) f[c] = Fast{IS_MAX ? -__builtin_huge_valf() : __builtin_huge_valf(), 0u};
+    else f[c] = Comb::empty();
+    row[c] = F.dinner.div(4 * t + c);
+    const uint32_t col = 4 * t + c - row[c] * inner;
+#pragma unroll
+    for (int k = 0; k < NIN; ++k)
+      fixed[k][c] = A.rst[k] == 0 ? A.in[k][base[k] + int64_t(col) * A.kst[k]] : 0.0f;
+  }
+  if (t < F.T) {
+    uint64_t step = 0;
+    for (uint64_t f0 = 4 * t; f0 < nf; f0 += uint64_t(4) * F.T * kU, step += kU) {
+      f4 x[kU][NIN];
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const uint64_t at = f0 + uint64_t(u) * 4 * F.T;
+#pragma unroll
+        for (int k = 0; k < NIN; ++k) {
+          const float *src = A.in[k] + base[k] + k0 * inner;
+          if (A.rst[k] == 0) {
+            x[u][k] = fixed[k];
+          } else if (at + 4 <= nf) {
+            x[u][k] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(src + at));
+          } else {
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) x[u][k][c] = at + c < nf ? src[at + c] : 0.0f;
+          }
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < kU; ++u) {
+        const uint64_t at = f0 + uint64_t(u) * 4 * F.T;
+        if (at >= nf) continue;
+        f4 yv;
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+          float v[NIN];
+#pragma unroll
+          for (int k = 0; k < NIN; ++k) v[k] = x[u][k][c];
+          const float y = prod.eval(v);
+          yv[c] = stored_value(prod, v, y);
+          if (at + c >= nf) continue;
+          if constexpr (kExt) {
+            f[c].m = IS_MAX ? fmaxf(f[c].m, y) : fminf(f[c].m, y);
+            f[c].nan |= y != y ? 1u : 0u;
+          } else {
+            Comb::next(f[c], y, int64_t(k0 + (step + u) * F.R + row[c]));
+          }
+        }
+        if constexpr (kStores<Prod>) {
+          float *dst = prod.dst + base[0] + k0 * inner + at;
+          if (at + 4 <= nf) {
+            store_col<Prod>(dst, yv);
+          } else {
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c)
+              if (at + c < nf) dst[c] = yv[c];
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) sh[4 * t + c] = f[c];
+  }
+  __syncthreads();
+  // sh[r][j]: the sums of rows r, r + R, ... of column j; rows 8e .. 8e + 7 merge into row e. A round
+  // has at most T / 2 + inner of them (rounding up), two per lane.
+  for (uint32_t rows = F.R; rows > 1;) {
+    const uint32_t next = (rows + 7) / 8;
+    Fast g[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t i = t + uint32_t(h) * kFlatBlock;
+      if (i >= next * inner) continue;
+      const uint32_t e = F.dinner.div(i), j = i - e * inner;
+      g[h] = sh[8 * e * inner + j];
+#pragma unroll
+      for (uint32_t q = 1; q < 8; ++q)
+        if (8 * e + q < rows) g[h] = merge(g[h], sh[(8 * e + q) * inner + j]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      if (t + uint32_t(h) * kFlatBlock < next * inner) sh[t + uint32_t(h) * kFlatBlock] = g[h];
+    __syncthreads();
+    rows = next;
+  }
+  if (t >= inner) return;
+  int64_t bc[NIN];
+#pragma unroll
+  for (int k = 0; k < NIN; ++k) bc[k] = base[k] + int64_t(t) * A.kst[k];
+  Part p;
+  if constexpr (kExt) {
+    if (!sh[t].nan && sh[t].m != 0.0f) {
+      p = ExtPart{sh[t].m, kNonEmpty};
+    } else {
+      p = Comb::empty();
+      for (uint64_t r = k0; r < k1; ++r) {
+        const float y = value_at(A, prod, bc, r);
+        if (r == k0) Comb::first(p, y, int64_t(r));
+        else Comb::next(p, y, int64_t(r));
+      }
+    }
+  } else {
+    p = sh[t];
+    if constexpr (kSerialSum<Comb>)
+      if (A.segs == 1 && !finite_sum(p)) p = serial_sum_lane(A, prod, bc, A.len);
+  }
+  if (A.segs == 1) store_final<Comb>(A.out, tbase + int64_t(t) * A.tkst, p, A.post, A.divisor);
+  else static_cast<Part *>(A.part)[uint64_t(blockIdx.y) * (A.rows * inner) + uint64_t(o) * inner + t] = p;
 }
 
 template <class Prod, class Comb>
@@ -975,6 +1274,18 @@ __global__ __launch_bounds__(kBlock) void red_generic_kernel(GenArgs<Prod::NIN> 
 
 // ------------------------------------------------------------------------- host dispatch
 
+// Merges the chunks' partials (and, for a serial refold, reads the inputs). More than one chunk is
+// planned only below PLAST_COL_BLOCKS workgroups of columns, so nout * Q lanes (at most
+// PLAST_COL_BLOCKS * 256 * Q) stay far inside one launch.
+template <class Prod, class Comb>
+void launch_cols_finalize(const RedArgs<Prod::NIN> &A, const Prod &prod, uint64_t nout, uint64_t chunks) {
+  if (PLAST_COL_FIN_Q > 1 && chunks >= 2 * PLAST_COL_FIN_Q)
+    red_cols_finalize_q<Prod, Comb, PLAST_COL_FIN_Q>
+        <<<ceil_div(nout * PLAST_COL_FIN_Q, kBlock), kBlock, 0, stream()>>>(A, prod);
+  else
+    red_cols_finalize<Prod, Comb><<<ceil_div(nout, kBlock), kBlock, 0, stream()>>>(A, prod);
+}
+
 // Reduce over every axis where operand NIN (the target) has stride 0 and extent > 1.
 // `post` and `divisor` describe the epilogue; `out` is float* or int64_t* per Comb::Out.
 template <class Prod, class Comb>
@@ -1048,19 +1359,15 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
     memset(&A, 0, sizeof A);
     for (int k = 0; k < NIN; ++k) A.in[k] = static_cast<const float *>(in[k]);
     A.out = out;
-    bool vec = s.shape[r - 1] % 4 == 0;
+    const bool vec = !multi || s.shape[r - 1] >= 4;  // a run's partial unit is read from its end
     for (int k = 0; k < NIN; ++k) {
       A.rst[k] = s.st[k][r - 1];
-      if (A.rst[k] == 1 && aligned16(in[k])) A.vec_mask |= 1u << k;
-      else if (A.rst[k] != 0) vec = false;
-      if (A.rst[k] == 1 && !aligned16(in[k])) vec = false;
+      if (A.rst[k] == 1) A.vec_mask |= 1u << k;
     }
     bool unit = true;
     for (int k = 0; k < NIN; ++k) unit = unit && (A.rst[k] == 0 || A.rst[k] == 1);
     if (unit) {
       for (int d = 0; d < r - 1; ++d) {
-        for (int k = 0; k < NIN; ++k)
-          if ((A.vec_mask >> k & 1u) && s.st[k][d] % 4 != 0) vec = false;
         if (reduced(d)) continue;
         A.dv[A.nouter] = MagicDiv::make(uint32_t(s.shape[d]));
         A.tst[A.nouter] = s.st[NIN][d];
@@ -1069,19 +1376,23 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       }
       outer_reduced(A);
       A.rows = nout;
+      const uint64_t units = (s.shape[r - 1] + 3) / 4;
+      A.dunits = MagicDiv::make(uint32_t(units));
+      A.vlen = 4 * units * (A.len / s.shape[r - 1]);
+      const uint64_t span = multi && vec ? A.vlen : A.len;  // what segments divide
       // enough waves to cover the machine: split long rows when there are few of them
       uint32_t segs = 1;
       const uint64_t want_waves = PLAST_ROW_WAVES;
-      if (A.rows < want_waves && A.len >= 8192) {
+      if (A.rows < want_waves && span >= 8192) {
         uint64_t sg = (want_waves + A.rows - 1) / A.rows;
-        const uint64_t max_sg = A.len / 4096;
+        const uint64_t max_sg = span / 4096;
         if (sg > max_sg) sg = max_sg;
         if (sg > 65535) sg = 65535;
         segs = uint32_t(sg < 1 ? 1 : sg);
       }
-      uint64_t seglen = (A.len + segs - 1) / segs;
+      uint64_t seglen = (span + segs - 1) / segs;
       seglen = (seglen + 255) / 256 * 256;
-      segs = uint32_t((A.len + seglen - 1) / seglen);
+      segs = uint32_t((span + seglen - 1) / seglen);
       A.segs = segs;
       A.seglen = seglen;
       A.post = int(post);
@@ -1090,16 +1401,23 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
         A.part = workspace(sizeof(Part) * A.rows * segs);
         if (!A.part) return false;
       }
+      // short rows: 2, 8 or 32 lanes each. [50000, 77] a wave per row / 8 lanes: see the kernel.
+      if (!multi && A.len <= 16 * 32) {
+        const int lanes = A.len <= 16 * 2 ? 2 : A.len <= 16 * 8 ? 8 : 32;
+        const unsigned sgrid = ceil_div(A.rows, (kBlock / 64) * (64 / lanes));
+        if (lanes == 2) red_rows_short_kernel<Prod, Comb, 2><<<sgrid, kBlock, 0, stream()>>>(A, prod);
+        else if (lanes == 8) red_rows_short_kernel<Prod, Comb, 8><<<sgrid, kBlock, 0, stream()>>>(A, prod);
+        else red_rows_short_kernel<Prod, Comb, 32><<<sgrid, kBlock, 0, stream()>>>(A, prod);
+        return true;
+      }
       const uint64_t waves = A.rows * segs;
       const unsigned grid = ceil_div(waves, kBlock / 64);
       if (vec && multi)
         red_rows_kernel<Prod, Comb, true, true><<<grid, kBlock, 0, stream()>>>(A, prod);
       else if (vec)
         red_rows_kernel<Prod, Comb, true, false><<<grid, kBlock, 0, stream()>>>(A, prod);
-      else if (multi)
-        red_rows_kernel<Prod, Comb, false, true><<<grid, kBlock, 0, stream()>>>(A, prod);
       else
-        red_rows_kernel<Prod, Comb, false, false><<<grid, kBlock, 0, stream()>>>(A, prod);
+        red_rows_kernel<Prod, Comb, false, true><<<grid, kBlock, 0, stream()>>>(A, prod);
       if (segs > 1)  // the finalize reads the partials, and the inputs for a serial refold
         red_rows_finalize<Prod, Comb>
             <<<ceil_div(A.rows, kBlock / 64), kBlock, 0, stream()>>>(A, prod);
@@ -1117,7 +1435,7 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
     A.inner = s.shape[r - 1];
     A.tkst = s.st[NIN][r - 1];
     outer_reduced(A);
-    bool vec = A.inner % 4 == 0 && A.tkst == 1;
+    bool vec = A.inner >= 4 && A.tkst == 1;
     int no = 0;
     for (int d = 0; d < r - 1; ++d) {
       if (reduced(d)) continue;
@@ -1127,24 +1445,22 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       ++no;
     }
     A.nouter = no;
+    bool flat = !multi && A.inner < 256;  // narrow: rows read as one flat array
     for (int k = 0; k < NIN; ++k) {
       A.rst[k] = s.st[k][red_ax];
       A.kst[k] = s.st[k][r - 1];
-      if (A.kst[k] == 1 && aligned16(in[k])) A.vec_mask |= 1u << k;
+      if (A.kst[k] == 1) A.vec_mask |= 1u << k;
       else if (A.kst[k] != 0) vec = false;
-      if (A.kst[k] == 1 && !aligned16(in[k])) vec = false;
-      if (A.kst[k] == 1) {
-        if (A.rst[k] % 4 != 0) vec = false;
-        for (int d = 0; d < A.nx; ++d)
-          if (A.xst[k][d] % 4 != 0) vec = false;
-        for (int d = 0; d < no; ++d)
-          if (A.ost[k][d] % 4 != 0) vec = false;
-      }
+      flat = flat && (A.rst[k] == 0 || (A.kst[k] == 1 && A.rst[k] == int64_t(A.inner)));
     }
+    if (kStores<Prod> && A.rst[0] == 0) flat = false;
     A.rows = nout / A.inner;  // outer count
     const bool allv = A.vec_mask == (1u << NIN) - 1;
     const uint32_t W = vec ? 4 : 1;
     const uint32_t xblocks = ceil_div(A.inner, uint64_t(64) * W);
+    // the slices of a row share its lanes evenly, in whole 128-byte lines
+    A.lanes = ceil_div(ceil_div(A.inner, W), xblocks);
+    A.lanes = vec && A.lanes < 56 ? (A.lanes + 7) / 8 * 8 : 64;
     const uint64_t base_blocks = uint64_t(xblocks) * A.rows;
     // chunk the reduced axis until the grid has ~PLAST_COL_BLOCKS workgroups, keeping at least
     // kColMinRows rows per chunk
@@ -1164,15 +1480,51 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
     A.post = int(post);
     A.divisor = divisor;
     if constexpr (std::is_same<Comb, SumComb>::value) {
-      // small: one launch over narrow column slices instead of chunks plus a finalize
-      if (chunks > 1 && vec && !multi && A.len * nout <= PLAST_COL_SMALL_MAX &&
-          (NIN < 3 || PLAST_COL_SMALL3 != 0)) {
+      // small: one launch over narrow column slices instead of chunks plus a finalize, while a lane's
+      // share of the rows stays a few batches (narrow columns leave few workgroups)
+      const uint64_t few_rows = uint64_t(2) * kColSmallU<Prod> * (kBlock / kColSmallS4<Prod>);
+      if ((A.len >= 128 || (A.len >= 64 && base_blocks < 64)) && vec && !multi && A.len * nout <= PLAST_COL_SMALL_MAX &&
+          (!flat || A.len <= few_rows) && (NIN < 3 || PLAST_COL_SMALL3 != 0)) {
         const uint32_t sblocks = ceil_div(A.inner, uint64_t(4) * kColSmallS4<Prod>);
-        const unsigned grid = unsigned(uint64_t(sblocks) * A.rows);
-        if (allv) red_cols_small_kernel<Prod, true><<<grid, kBlock, 0, stream()>>>(A, prod, sblocks);
-        else red_cols_small_kernel<Prod, false><<<grid, kBlock, 0, stream()>>>(A, prod, sblocks);
-        return true;
+        const uint64_t sgrid = uint64_t(sblocks) * A.rows;
+        if (sgrid <= max_blocks(kBlock)) {
+          A.segs = 1;
+          const unsigned grid = unsigned(sgrid);
+          if (allv) red_cols_small_kernel<Prod, true><<<grid, kBlock, 0, stream()>>>(A, prod, sblocks);
+          else red_cols_small_kernel<Prod, false><<<grid, kBlock, 0, stream()>>>(A, prod, sblocks);
+          return true;
+        }
       }
+    }
+    if (flat && A.rows <= max_blocks(kFlatBlock)) {
+      const uint32_t in = uint32_t(A.inner);
+      const uint32_t units = in % 4 == 0 ? in / 4 : in % 2 == 0 ? in / 2 : in;  // of the shortest
+      FlatCols F;                                                             // whole rows
+      F.T = kFlatBlock / units * units;
+      F.R = uint32_t(uint64_t(4) * F.T / in);
+      F.dinner = MagicDiv::make(in);
+      // chunks of whole steps: eight steps each up to about PLAST_COL_BLOCKS workgroups, down to two
+      // where that leaves the chip idle (sum and max of [60000, 10]: 16.0 us with chunks of eight,
+      // 13.4 of two; the bias gradient of [16384, 250]: 28.3 and 30.6)
+      const uint64_t steps = (A.len + F.R - 1) / F.R;
+      uint64_t fc = steps / 8;
+      const uint64_t most = (PLAST_COL_BLOCKS + A.rows - 1) / A.rows, least = (256 + A.rows - 1) / A.rows;
+      if (fc > most) fc = most;
+      if (fc < least) fc = steps / 2 < least ? steps / 2 : least;
+      if (steps <= 8) fc = 1;
+      if (fc > 65535) fc = 65535;
+      if (fc < 1) fc = 1;
+      A.seglen = (steps + fc - 1) / fc * F.R;
+      chunks = (A.len + A.seglen - 1) / A.seglen;
+      A.segs = uint32_t(chunks);
+      if (chunks > 1) {
+        A.part = workspace(sizeof(Part) * nout * chunks);
+        if (!A.part) return false;
+      }
+      const dim3 grid{unsigned(A.rows), unsigned(chunks), 1u};
+      red_cols_flat_kernel<Prod, Comb><<<grid, kFlatBlock, 0, stream()>>>(A, prod, F);
+      if (chunks > 1) launch_cols_finalize<Prod, Comb>(A, prod, nout, chunks);
+      return true;
     }
     if (base_blocks <= max_blocks(kBlock)) {
       if (chunks > 1) {
@@ -1183,27 +1535,22 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       bool launched = false;
       if constexpr (!kStores<Prod>) {
         if (multi && vec)
-          red_cols_kernel<Prod, Comb, true, false, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+          red_cols_kernel<Prod, Comb, true, false, true, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
         else if (multi)
-          red_cols_kernel<Prod, Comb, false, false, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+          red_cols_kernel<Prod, Comb, false, false, true, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
         launched = multi;
       }
+      const bool ragged = A.inner % 4 != 0 || A.lanes < 64;
       if (launched) {
-      } else if (vec && allv)
-        red_cols_kernel<Prod, Comb, true, true, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+      } else if (vec && allv && ragged)
+        red_cols_kernel<Prod, Comb, true, true, false, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+      else if (vec && allv)
+        red_cols_kernel<Prod, Comb, true, true, false, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
       else if (vec)
-        red_cols_kernel<Prod, Comb, true, false, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+        red_cols_kernel<Prod, Comb, true, false, false, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
       else
-        red_cols_kernel<Prod, Comb, false, false, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
-      if (chunks > 1) {  // the finalize reads the partials, and the inputs for a serial refold
-        // chunks > 1 only when base_blocks < PLAST_COL_BLOCKS, so nout * Q lanes (at most
-        // PLAST_COL_BLOCKS * 256 * Q) stay far inside one launch
-        if (PLAST_COL_FIN_Q > 1 && chunks >= 2 * PLAST_COL_FIN_Q)
-          red_cols_finalize_q<Prod, Comb, PLAST_COL_FIN_Q>
-              <<<ceil_div(nout * PLAST_COL_FIN_Q, kBlock), kBlock, 0, stream()>>>(A, prod);
-        else
-          red_cols_finalize<Prod, Comb><<<ceil_div(nout, kBlock), kBlock, 0, stream()>>>(A, prod);
-      }
+        red_cols_kernel<Prod, Comb, false, false, false, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+      if (chunks > 1) launch_cols_finalize<Prod, Comb>(A, prod, nout, chunks);
       return true;
     }
   }
