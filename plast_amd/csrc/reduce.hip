@@ -141,6 +141,112 @@ struct StrictExtComb {
   __device__ static Part shfl(Part p, int m) { return __shfl_xor(p, m); }
 };
 
+// Max/min backward over unit-stride rows, in one read of the input: T threads per row (8 or 64 lanes
+// of a wave, or the workgroup) count the elements equal to the row's extreme, then add dout / count
+// to the gradient of those alone. The other elements' gradients keep their bits, so they are neither
+// read nor written: 4 bytes an element where counting in one pass and accumulating in another moved
+// 16. Operands of A: a, its gradient (written), the extreme and dout (one of each per row).
+// [50000, 77]: 14 us in two passes.
+constexpr int kExtBlock = 512;
+template <int T>
+__global__ __launch_bounds__(T > 64 ? T : kBlock) void ext_bwd_rows_kernel(RedArgs<4> A) {
+  __shared__ uint32_t sh[T > 64 ? T / 64 : 1];
+  constexpr int U = 4;
+  const uint32_t t = threadIdx.x, l = t % T;
+  constexpr uint32_t rows_per_block = (T > 64 ? T : kBlock) / T;
+  const uint64_t row = uint64_t(blockIdx.x) * rows_per_block + t / T;
+  const bool valid = row < A.rows;
+  int64_t base[4], tbase;
+  decode_outer(A, uint32_t(valid ? row : A.rows - 1), base, tbase);
+  const float *a = A.in[0] + base[0];
+  float *da = const_cast<float *>(A.in[1]) + base[1];
+  const float e = A.in[2][base[2]], g = A.in[3][base[3]];
+  const uint32_t len = uint32_t(A.len), units = len / 4;
+  uint32_t cnt = 0, pos = 0;  // this thread's ties, and the first of them
+  const auto take = [&](float x, uint32_t i) {
+    if (x == e) {
+      if (cnt == 0) pos = i;
+      ++cnt;
+    }
+  };
+  for (uint32_t q0 = l; q0 < units; q0 += T * U) {
+    f4 x[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t q = q0 + uint32_t(u) * T < units ? q0 + uint32_t(u) * T : units - 1;
+      x[u] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(a + 4 * uint64_t(q)));
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t q = q0 + uint32_t(u) * T;
+      if (q >= units) continue;
+#pragma unroll
+      for (uint32_t c = 0; c < 4; ++c) take(x[u][c], 4 * q + c);
+    }
+  }
+  for (uint32_t i = units * 4 + l; i < len; i += T) take(a[i], i);
+  uint32_t n = cnt;
+#pragma unroll
+  for (int m = (T < 64 ? T : 64) / 2; m >= 1; m >>= 1) n += uint32_t(__shfl_xor(int(n), m));
+  if constexpr (T > 64) {
+    if ((t & 63) == 0) sh[t >> 6] = n;
+    __syncthreads();
+    n = 0;
+#pragma unroll
+    for (int w = 0; w < T / 64; ++w) n += sh[w];
+  }
+  if (!valid || cnt == 0) return;
+  const float add = g / float(n);
+  da[pos] = da[pos] + add;
+  if (cnt == 1) return;
+  // several ties in one thread's share (an order of its own: units, then the elements left over)
+  for (uint32_t q = pos / 4 < units ? pos / 4 : units + l; q < units; q += T)
+    for (uint32_t i = 4 * q; i < 4 * q + 4; ++i)
+      if (i > pos && a[i] == e) da[i] = da[i] + add;
+  for (uint32_t i = units * 4 + l; i < len; i += T)
+    if (i != pos && a[i] == e) da[i] = da[i] + add;
+}
+
+// Launches ext_bwd_rows_kernel when a and its gradient are unit-stride along the reduced axis `dim`,
+// the last one, and the rows fill the chip or are short; false (launching nothing) otherwise. `ost`:
+// the output's strides over a's axes.
+bool ext_backward_rows(const Tensor *a, const Tensor *out, uint64_t dim, const int64_t *ost) {
+  const uint64_t n = numel(a), len = a->shape[dim];
+  if (dim + 1 != a->ndim || n == 0 || n >= (uint64_t(1) << 32)) return false;
+  if (len > 1 && (a->strides[dim] != 1 || a->grad->strides[dim] != 1)) return false;
+  const uint64_t rows = n / len;
+  if (len > 32768 && rows < 256) return false;
+  Space s;
+  s.rank = int(a->ndim);
+  s.nops = 4;
+  for (int d = 0; d < s.rank; ++d) {
+    const bool one = a->shape[d] == 1 || d == int(dim);
+    s.shape[d] = d == int(dim) ? 1 : a->shape[d];
+    s.st[0][d] = one ? 0 : int64_t(a->strides[d]);
+    s.st[1][d] = one ? 0 : int64_t(a->grad->strides[d]);
+    s.st[2][d] = s.st[3][d] = one ? 0 : ost[d];
+  }
+  collapse(s);
+  RedArgs<4> A;
+  memset(&A, 0, sizeof A);
+  A.in[0] = static_cast<const float *>(a->data);
+  A.in[1] = static_cast<const float *>(a->grad->data);
+  A.in[2] = static_cast<const float *>(out->data);
+  A.in[3] = static_cast<const float *>(out->grad->data);
+  A.len = len;
+  A.rows = rows;
+  for (int d = 0; d < s.rank; ++d) {
+    A.dv[d] = MagicDiv::make(uint32_t(s.shape[d]));
+    for (int k = 0; k < 4; ++k) A.ost[k][d] = s.st[k][d];
+  }
+  A.nouter = s.rank;
+  // threads per row: about four float4 units each
+  if (len <= 128) ext_bwd_rows_kernel<8><<<ceil_div(rows, kBlock / 8), kBlock, 0, stream()>>>(A);
+  else if (len <= 2048) ext_bwd_rows_kernel<64><<<ceil_div(rows, kBlock / 64), kBlock, 0, stream()>>>(A);
+  else ext_bwd_rows_kernel<kExtBlock><<<unsigned(rows), kExtBlock, 0, stream()>>>(A);
+  return true;
+}
+
 template <bool IS_MAX>
 void ext_backward(Tensor **in, const Tensor *out, KernelParams p, const char *where) {
   if (!ensure_init()) return;
@@ -153,6 +259,14 @@ void ext_backward(Tensor **in, const Tensor *out, KernelParams p, const char *wh
   }
   const bool keep = p.keepdim != 0;
   const bool all = p.dim == PLAST_DIM_ALL;
+  if (!all) {
+    int64_t rst[kMaxRank];
+    output_strides_in_input_space(a, p.dim, keep, out->strides, rst);
+    if (ext_backward_rows(a, out, p.dim, rst)) {
+      finish(where);
+      return;
+    }
+  }
   const uint64_t nout = all ? 1 : numel(out);
   // slot-1 temporaries: [count per output][recomputed extreme (full contiguous case)]
   float *tmp = static_cast<float *>(workspace(sizeof(float) * (nout + 1), 1));
