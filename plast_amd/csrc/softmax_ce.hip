@@ -13,6 +13,7 @@
 // The fast paths evaluate exp with exp_le0 (about 1 ulp); the exact-refold paths use expf.
 #include <atomic>
 #include <cfloat>
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -128,7 +129,38 @@ __device__ float serial_max_fold(const float *row, uint32_t C) {
   return acc;
 }
 
-// Row max with exact reference bits: fast block fmax + NaN flag; thread 0 refolds serially when
+// The same fold by a wave: a NaN restarts it (the result is the fold of what follows the last one),
+// and the last of several zeros that tie decides a zero result's sign.
+__device__ float wave_max_fold(const float *row, uint32_t C, int lane) {
+  int last_nan = -1;
+  for (uint32_t j = lane; j < C; j += 64)
+    if (row[j] != row[j]) last_nan = int(j);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) {
+    const int o = __shfl_xor(last_nan, m);
+    last_nan = o > last_nan ? o : last_nan;
+  }
+  const uint32_t s = uint32_t(last_nan + 1);
+  if (s >= C) return last_nan < 0 ? -FLT_MAX : row[last_nan];
+  float r = -__builtin_huge_valf();
+  for (uint32_t j = s + lane; j < C; j += 64) r = fmaxf(r, row[j]);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) r = fmaxf(r, __shfl_xor(r, m));
+  if (r == 0.0f) {
+    int zero = -1;
+    for (uint32_t j = s + lane; j < C; j += 64)
+      if (row[j] == 0.0f) zero = int(j);
+#pragma unroll
+    for (int m = 32; m >= 1; m >>= 1) {
+      const int o = __shfl_xor(zero, m);
+      zero = o > zero ? o : zero;
+    }
+    r = row[zero];
+  }
+  return last_nan >= 0 || r > -FLT_MAX ? r : -FLT_MAX;
+}
+
+// Row max with exact reference bits: fast block fmax + NaN flag; wave 0 refolds when
 // the fast value could differ (a NaN in the row, or a zero maximum whose sign depends on order).
 template <int W = kCeWaves>
 __device__ __forceinline__ float row_max_exact(float m, bool nan, const float *row, uint32_t C,
@@ -137,48 +169,86 @@ __device__ __forceinline__ float row_max_exact(float m, bool nan, const float *r
   nan = block_any<W>(nan, lds);
   if (nan || m == 0.0f) {
     __syncthreads();
-    if (threadIdx.x == 0) lds[W] = serial_max_fold(row, C);
+    if (threadIdx.x < 64) {
+      const float f = wave_max_fold(row, C, int(threadIdx.x));
+      if (threadIdx.x == 0) lds[W] = f;
+    }
     __syncthreads();
     return lds[W];
   }
   return m > -FLT_MAX ? m : -FLT_MAX;
 }
 
-// Any row length or alignment: three passes over the row (max, exp-sum, terms).
-__global__ __launch_bounds__(kCeBlock) void ce_fwd_generic_kernel(const float *__restrict__ x,
-                                                                  const int32_t *__restrict__ lab,
-                                                                  float *__restrict__ stats,
-                                                                  float *__restrict__ loss,
-                                                                  uint32_t C, uint64_t simd_end) {
-  __shared__ float lds[kCeWaves + 1];
-  const uint64_t row = blockIdx.x;
-  const float *xr = x + row * C;
-  float m = -__builtin_huge_valf();
-  bool nan = false;
-  for (uint32_t j = threadIdx.x; j < C; j += kCeBlock) {
-    m = fmaxf(m, xr[j]);
-    nan = nan || xr[j] != xr[j];
+// Rows of any length and alignment in float4 units: unit q covers elements 4q .. 4q + 3, the last
+// one partial. A partial unit of a row of four and more is read from four elements before the row's
+// end (its first `lo` elements are the unit before's), a shorter row's element by element; elements
+// [lo, hi) are the unit's own.
+struct RowUnit {
+  uint32_t pos, lo, hi;
+};
+__device__ __forceinline__ RowUnit row_unit(uint32_t q, uint32_t C) {
+  const uint32_t at = 4 * q;
+  if (C < 4) return RowUnit{0, 0, q == 0 ? C : 0};
+  const uint32_t pos = at + 4 <= C ? at : C - 4;
+  return RowUnit{pos, at < C ? at - pos : 4u, 4u};
+}
+// The unit's four elements (those past a row shorter than four repeat its last one).
+__device__ __forceinline__ f4 load_row_part(const float *row, const RowUnit &r, uint32_t C) {
+  if (C >= 4) return __builtin_nontemporal_load(reinterpret_cast<const f4u *>(row + r.pos));
+  f4 v;
+#pragma unroll
+  for (uint32_t c = 0; c < 4; ++c) v[c] = row[c < C ? c : C - 1];
+  return v;
+}
+// Stores the unit's own elements.
+__device__ __forceinline__ void store_row_part(f4 v, float *row, const RowUnit &r) {
+  if (r.lo == 0 && r.hi == 4) {
+    store_unit<true>(v, row + r.pos);
+    return;
   }
-  const float mx = row_max_exact(m, nan, xr, C, lds);
-  float s = 0.0f;
-  for (uint32_t j = threadIdx.x; j < C; j += kCeBlock) s += expf(xr[j] - mx);
-  s = block_sum(s, lds);
-  const float l = logf(s);
-  const int32_t y = lab[row];
-  bool bad = false;
-  for (uint32_t j = threadIdx.x; j < C; j += kCeBlock) {
-    const float ls = (xr[j] - mx) - l;
-    if (int32_t(j) != y) bad = bad || !(fabsf(ls) <= FLT_MAX);
-  }
-  bad = block_any(bad, lds);
-  if (threadIdx.x == 0) {
-    float t;
-    if (bad) t = __builtin_nanf("");
-    else if (y >= 0 && uint32_t(y) < C) t = 0.0f + ((xr[y] - mx) - l);
-    else t = 0.0f;
-    loss[row] = row < simd_end ? 0.0f - t : -t;
-    stats[2 * row] = mx;
-    stats[2 * row + 1] = l;
+#pragma unroll
+  for (uint32_t c = 0; c < 4; ++c)
+    if (c >= r.lo && c < r.hi) row[r.pos + c] = v[c];
+}
+
+// Sum and maximum over the T lanes that share a row (T a power of two up to 64).
+template <int T>
+__device__ __forceinline__ float group_sum(float v) {
+#pragma unroll
+  for (int m = T / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m);
+  return v;
+}
+template <int T>
+__device__ __forceinline__ float group_max(float v) {
+#pragma unroll
+  for (int m = T / 2; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
+  return v;
+}
+template <int T>
+__device__ __forceinline__ float group_min(float v) {
+#pragma unroll
+  for (int m = T / 2; m >= 1; m >>= 1) v = fminf(v, __shfl_xor(v, m));
+  return v;
+}
+
+// Lanes per row and float4 units per lane for rows held in a wave's registers: about four units a
+// lane, so that a wave always has 64 lanes of loads in flight however short the rows are (a
+// 256-lane workgroup per row of 10 used 10 of its lanes). f(lanes, units) with constants.
+constexpr uint32_t kWaveRow = 2048;  // the longest: 64 lanes of 8 units
+// Softmax takes a workgroup per row beyond these (its backward holds three operands). Forward and
+// backward over three rotating inputs, wave / workgroup per row: forward [60000, 600] 145 / 181 us,
+// [16384, 1000] 66.5 / 69.8, and with both in 8 units [30000, 1500] 185 / 163; backward [60000, 600]
+// 145 / 157, [60000, 700] 169 / 171, [16384, 1000] 70.2 / 66.5.
+constexpr uint32_t kSoftmaxWaveRow = 1024, kSoftmaxBwdWaveRow = 768;
+template <uint32_t MAX_ROW, class F>
+void with_row_lanes(uint32_t C, F &&f) {
+  using std::integral_constant;
+  if (C <= 32) f(integral_constant<int, 2>{}, integral_constant<int, 4>{});
+  else if (C <= 128) f(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+  else if (C <= 512) f(integral_constant<int, 32>{}, integral_constant<int, 4>{});
+  else if constexpr (MAX_ROW > 512) {
+    if (C <= 1024) f(integral_constant<int, 64>{}, integral_constant<int, 4>{});
+    else if constexpr (MAX_ROW > 1024) f(integral_constant<int, 64>{}, integral_constant<int, 8>{});
   }
 }
 
@@ -200,11 +270,99 @@ __device__ __forceinline__ float wave_min(float v) {
 
 constexpr int kCeUnroll = PLAST_CE_UNROLL;  // float4 loads in flight per lane
 
+// A row whose fast values could differ from the reference chain's bits, by one wave from memory: the
+// chain element by element. Every lane returns the row max, the log of the exp-sum, and whether a
+// term of the one-hot product other than the label's is not finite.
+__device__ void ce_wave_exact(const float *xr, uint32_t C, int32_t y, int lane, float &mx, float &l,
+                              bool &bad) {
+  mx = wave_max_fold(xr, C, lane);
+  float t = 0.0f;
+  for (uint32_t j = lane; j < C; j += 64) t += expf(xr[j] - mx);
+  l = logf(wave_sum(t));
+  bool b = false;
+  for (uint32_t j = lane; j < C; j += 64) {
+    const float ls = (xr[j] - mx) - l;
+    if (int32_t(j) != y) b = b || !(fabsf(ls) <= FLT_MAX);
+  }
+  bad = __any(b);
+}
+
+// A row's loss and statistics, by one lane.
+__device__ __forceinline__ void ce_row_out(const float *xr, uint32_t C, int32_t y, float mx, float l,
+                                           bool bad, uint64_t row, uint64_t simd_end,
+                                           float *__restrict__ loss, float *__restrict__ stats) {
+  float t;
+  if (bad) t = __builtin_nanf("");
+  else if (y >= 0 && uint32_t(y) < C) t = 0.0f + ((xr[y] - mx) - l);
+  else t = 0.0f;
+  loss[row] = row < simd_end ? 0.0f - t : -t;
+  stats[2 * row] = mx;
+  stats[2 * row + 1] = l;
+}
+
+// Whether a row's fast maximum M, exp-sum S or smallest logit mn could stand for values the
+// reference chain would give other bits: a non-finite or zero maximum, a NaN or overflowed sum, or a
+// shifted and normalised logit that overflows (0 * -inf = NaN in the one-hot product).
+__device__ __forceinline__ bool ce_needs_exact(float M, float S, float mn, float l) {
+  return !(fabsf(M) <= FLT_MAX) || M == 0.0f || !(S <= FLT_MAX) || !(fabsf((mn - M) - l) <= FLT_MAX);
+}
+
+// Forward over rows of at most 4 * L * U floats held in registers, L lanes each. Twenty-odd
+// instructions a logit at most; what bounds it is the one read. [60000, 10]: 89.9 us with a workgroup
+// per row.
+constexpr uint32_t kCeWaveRow = 512;  // longer rows stream through ce_fwd_wave_kernel
+template <int L, int U>
+__global__ __launch_bounds__(kCeBlock) void ce_fwd_rows_kernel(const float *__restrict__ x,
+                                                               const int32_t *__restrict__ lab,
+                                                               float *__restrict__ stats,
+                                                               float *__restrict__ loss, uint64_t N,
+                                                               uint32_t C, uint64_t simd_end) {
+  const int lane = threadIdx.x & 63, l = lane % L;
+  const uint64_t row0 = (uint64_t(blockIdx.x) * kCeWaves + (threadIdx.x >> 6)) * (64 / L);
+  if (row0 >= N) return;  // whole wave
+  const uint64_t row = row0 + lane / L;
+  const bool valid = row < N;
+  const float *xr = x + (valid ? row : N - 1) * C;
+  const int32_t y = lab[valid ? row : N - 1];
+  f4 v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = load_row_part(xr, row_unit(uint32_t(l) + u * L, C), C);
+  float M = -__builtin_huge_valf(), mn = __builtin_huge_valf();
+#pragma unroll
+  for (int u = 0; u < U; ++u)  // elements read twice change neither
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      M = fmaxf(M, v[u][c]);
+      mn = fminf(mn, v[u][c]);
+    }
+  M = group_max<L>(M);
+  mn = group_min<L>(mn);
+  float S = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const RowUnit r = row_unit(uint32_t(l) + u * L, C);
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) {
+      const float e = exp_le0(v[u][c] - M);
+      S += c >= r.lo && c < r.hi ? e : 0.0f;
+    }
+  }
+  S = group_sum<L>(S);
+  float mx = M, lg = logf(S);
+  bool bad = false;
+  for (uint64_t todo = __ballot(valid && l == 0 && ce_needs_exact(M, S, mn, lg)); todo; todo &= todo - 1) {
+    const int first = __ffsll((unsigned long long)todo) - 1;  // the row's first lane
+    float m1, l1;
+    bool b1;
+    ce_wave_exact(x + (row0 + first / L) * C, C, __shfl(y, first), lane, m1, l1, b1);
+    if (lane == first) mx = m1, lg = l1, bad = b1;
+  }
+  if (valid && l == 0) ce_row_out(xr, C, y, mx, lg, bad, row, simd_end, loss, stats);
+}
+
 // One wave64 per row, a single read of the row. Each lane keeps an online (max, exp-sum) pair,
-// rescaling its sum when its max grows; the wave merges the pairs. Rows for which the fast
-// values could differ from the reference chain's bits (a non-finite logit, a zero or non-finite
-// max, or a shifted-and-normalised logit that overflows to -inf) are recomputed exactly by the
-// same wave from memory.
+// rescaling its sum when its max grows; the wave merges the pairs. Rows for which ce_needs_exact
+// holds are recomputed by the same wave from memory.
 constexpr int kCeFwdWaves = PLAST_CE_FWD_WAVES;  // rows (waves) per workgroup
 
 __global__ __launch_bounds__(64 * kCeFwdWaves) void ce_fwd_wave_kernel(const float *__restrict__ x,
@@ -220,22 +378,22 @@ __global__ __launch_bounds__(64 * kCeFwdWaves) void ce_fwd_wave_kernel(const flo
   const float ninf = -__builtin_huge_valf();
   float m = ninf, s = 0.0f, mn = __builtin_huge_valf();
   const uint32_t C4 = C / 4;
-  const f4 *x4 = reinterpret_cast<const f4 *>(xr);
+  const auto grow = [&](float g) {  // raise the lane's maximum to g
+    s = m == ninf ? s * 0.0f : s * exp_le0(m - g);
+    m = g;
+  };
   for (uint32_t q0 = lane; q0 < C4; q0 += 64 * kCeUnroll) {
     f4 v[kCeUnroll];
 #pragma unroll
     for (int u = 0; u < kCeUnroll; ++u) {
       const uint32_t q = q0 + uint32_t(u) * 64;
-      if (q < C4) v[u] = __builtin_nontemporal_load(x4 + q);
+      if (q < C4) v[u] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(xr + 4 * q));
     }
 #pragma unroll
     for (int u = 0; u < kCeUnroll; ++u) {
       if (q0 + uint32_t(u) * 64 >= C4) continue;
       const float g = fmaxf(fmaxf(v[u][0], v[u][1]), fmaxf(v[u][2], v[u][3]));
-      if (g > m) {
-        s = m == ninf ? s * 0.0f : s * exp_le0(m - g);
-        m = g;
-      }
+      if (g > m) grow(g);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const float e = v[u][c];
@@ -244,55 +402,23 @@ __global__ __launch_bounds__(64 * kCeFwdWaves) void ce_fwd_wave_kernel(const flo
       }
     }
   }
+  if (C4 * 4 + lane < C) {  // the up to three logits after the last float4
+    const float e = xr[C4 * 4 + lane];
+    if (e > m) grow(e);
+    mn = fminf(mn, e);
+    s += exp_le0(e - m);
+  }
   const float M = wave_max(m);
   const float sc = m == ninf ? s * 0.0f : s * exp_le0(m - M);
-  float S = wave_sum(sc);
-  // a NaN logit reaches the sum (fmaxf skips NaN, exp(NaN - m) does not); an infinite one makes
-  // M or the minimum below non-finite
-  const bool nonfin = !(S <= FLT_MAX);
+  const float S = wave_sum(sc);
   mn = wave_min(mn);
-  float mx = M;
-  bool exact = false;
-  if (!(fabsf(M) <= FLT_MAX) || M == 0.0f || nonfin) {
-    exact = true;
-  }
-  float l = logf(S);
-  if (!exact && C > 0) {
-    // the most negative shifted-normalised logit must stay finite (else 0 * -inf = NaN)
-    if (!(fabsf((mn - mx) - l) <= FLT_MAX)) exact = true;
-  }
+  float mx = M, l = logf(S);
   bool bad = false;
-  if (exact) {
-    // the reference chain, element by element (rare rows)
-    float acc = -FLT_MAX;
-    if (lane == 0)
-      for (uint32_t j = 0; j < C; ++j) acc = acc > xr[j] ? acc : xr[j];
-    mx = __shfl(acc, 0);
-    float t = 0.0f;
-    for (uint32_t j = lane; j < C; j += 64) t += expf(xr[j] - mx);
-    S = wave_sum(t);
-    l = logf(S);
-    bool b = false;
-    for (uint32_t j = lane; j < C; j += 64) {
-      const float ls = (xr[j] - mx) - l;
-      if (int32_t(j) != y) b = b || !(fabsf(ls) <= FLT_MAX);
-    }
-    bad = __any(b);
-  }
-  if (lane == 0) {
-    float t;
-    if (bad) t = __builtin_nanf("");
-    else if (y >= 0 && uint32_t(y) < C) t = 0.0f + ((xr[y] - mx) - l);
-    else t = 0.0f;
-    loss[row] = row < simd_end ? 0.0f - t : -t;
-    stats[2 * row] = mx;
-    stats[2 * row + 1] = l;
-  }
+  // a NaN logit reaches the sum (fmaxf skips NaN, exp(NaN - m) does not); an infinite one makes M
+  // or the minimum non-finite
+  if (ce_needs_exact(M, S, mn, l)) ce_wave_exact(xr, C, y, lane, mx, l, bad);
+  if (lane == 0) ce_row_out(xr, C, y, mx, l, bad, row, simd_end, loss, stats);
 }
-
-// Backward, any alignment: the scalar kernel's chunk of a row is kBwdUnroll * 4 * kCeBlock
-// elements.
-constexpr int kBwdUnroll = PLAST_CE_BWD_UNROLL;
 
 // Backward, float4 path over the flattened [N, C] gradient: one float4 per lane, its row found by
 // magic division; the per-row constants are cached vector loads shared by the wave.
@@ -326,27 +452,54 @@ __global__ __launch_bounds__(kCeFlatBlock) void ce_bwd_flat_kernel(const float *
   store_stream<PLAST_CE_NT_STORE>(r, reinterpret_cast<f4 *>(dx) + q);
 }
 
-// Backward, any alignment: one element per lane per step.
+// The same over rows that are no whole float4: a unit's elements fall in the row of its first one and
+// in those after it. [60000, 10]: 18.7 us with a workgroup per row.
 template <bool OVERWRITE>
-__global__ __launch_bounds__(kCeBlock) void ce_bwd_scalar_kernel(const float *__restrict__ x,
+__global__ __launch_bounds__(kCeFlatBlock) void ce_bwd_ragged_kernel(const float *__restrict__ x,
                                                                  const int32_t *__restrict__ lab,
                                                                  const float *__restrict__ stats,
                                                                  const float *__restrict__ dloss,
-                                                                 float *dx, uint32_t C,
-                                                                 uint32_t chunks) {
-  const uint64_t row = blockIdx.x / chunks;
-  const uint32_t chunk = blockIdx.x - uint32_t(row) * chunks;
-  const float m = stats[2 * row], l = stats[2 * row + 1], g = dloss[row];
-  const int32_t y = lab[row];
-  const float *xr = x + row * C;
-  float *dr = dx + row * C;
-  const uint32_t j0 = chunk * (kCeBlock * kBwdUnroll * 4);
-  const uint32_t j1 = j0 + kCeBlock * kBwdUnroll * 4 < C ? j0 + kCeBlock * kBwdUnroll * 4 : C;
-  for (uint32_t j = j0 + threadIdx.x; j < j1; j += kCeBlock) {
-    const float sm = exp_le0((xr[j] - m) - l);
-    const float oh = int32_t(j) == y ? 1.0f : 0.0f;
+                                                                 float *dx, MagicDiv dc, uint32_t n) {
+  const uint32_t q = (PLAST_CE_BWD_XCD ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) * kCeFlatBlock + threadIdx.x;
+  const uint64_t at = uint64_t(q) * 4;
+  if (at >= n) return;
+  const bool whole = at + 4 <= n;
+  f4 xv = f4(0.0f), dv = f4(0.0f);
+  if (whole) {
+    xv = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(x + at));
+    if constexpr (!OVERWRITE) dv = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(dx + at));
+  } else {
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c) {
+      if (at + c >= n) continue;
+      xv[c] = x[at + c];
+      if constexpr (!OVERWRITE) dv[c] = dx[at + c];
+    }
+  }
+  uint32_t row = dc.div(uint32_t(at));
+  uint32_t col = uint32_t(at) - row * dc.d;
+  float m = stats[2 * uint64_t(row)], l = stats[2 * uint64_t(row) + 1], g = dloss[row];
+  int32_t y = lab[row];
+  f4 r;
+#pragma unroll
+  for (uint32_t c = 0; c < 4; ++c) {
+    const float sm = exp_le0((xv[c] - m) - l);
+    const float oh = int32_t(col) == y ? 1.0f : 0.0f;
     const float gv = g * (sm - oh);
-    dr[j] = OVERWRITE ? gv : dr[j] + gv;
+    r[c] = OVERWRITE ? gv : dv[c] + gv;
+    if (++col == dc.d && at + c + 1 < n) {  // the next element starts a row
+      col = 0;
+      ++row;
+      m = stats[2 * uint64_t(row)], l = stats[2 * uint64_t(row) + 1], g = dloss[row];
+      y = lab[row];
+    }
+  }
+  if (whole) {
+    store_unit<PLAST_CE_NT_STORE>(r, dx + at);
+  } else {
+#pragma unroll
+    for (uint32_t c = 0; c < 3; ++c)
+      if (at + c < n) dx[at + c] = r[c];
   }
 }
 
@@ -469,7 +622,9 @@ __device__ void ce_row_exact(const float *row, uint32_t C, int32_t y, float *lds
   bad = block_any<W>(b, lds);
 }
 
-template <int V, bool DYN>
+// RAGGED: rows of any length and alignment. A row's last unit is then partial: it is read from four
+// elements before the row's end and owns its last C % 4 (a lane past the row reads it too).
+template <int V, bool DYN, bool RAGGED>
 __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
     const float *__restrict__ x, const int32_t *__restrict__ lab, const float *__restrict__ dloss,
     float *__restrict__ stats, float *__restrict__ loss, float *__restrict__ dx,
@@ -484,6 +639,9 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
   // row indices are 32-bit (the host checks N < 2^32): a 64-bit bound compare would be made in
   // vector registers, which the loop head may find still tied to an in-flight memory operation
   const uint32_t G = gridDim.x;
+  const uint32_t rem = RAGGED ? C % 4 : 0;
+  // the first element of unit q that the unit owns (4: none)
+  const auto own = [&](uint32_t q) -> uint32_t { return q < C4 ? 0 : q == C4 ? 4 - rem : 4; };
   const float ninf = -__builtin_huge_valf(), pinf = __builtin_huge_valf();
 #pragma unroll
   for (int u = 0; u < V; ++u) colsum[t + uint32_t(u) * BS] = f4(0.0f);
@@ -513,8 +671,13 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
 #pragma unroll
     for (int u = 0; u < V; ++u) {
       const uint32_t q = ti + uint32_t(u) * BS;
-      const uint32_t off = (q < C4 ? q : C4 - 1) * 16u;
-      v[u] = load_row_unit<PLAST_CE_STEP_NT_LOAD>(reinterpret_cast<const f4 *>(xr + off));
+      if constexpr (RAGGED) {
+        const uint32_t off = q < C4 ? q * 16u : (C - 4) * 4u;
+        v[u] = __builtin_nontemporal_load(reinterpret_cast<const f4u *>(xr + off));
+      } else {
+        const uint32_t off = (q < C4 ? q : C4 - 1) * 16u;
+        v[u] = load_row_unit<PLAST_CE_STEP_NT_LOAD>(reinterpret_cast<const f4 *>(xr + off));
+      }
     }
     pin_loads();
   };
@@ -555,6 +718,8 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
     // the label's logit, taken by the lane that holds it before the sum pass overwrites v
     const bool live = y >= 0 && uint32_t(y) < C;
     const uint32_t yq = live ? uint32_t(y) >> 2 : 0;
+    // the label's element of its unit
+    const int yc = RAGGED && yq == C4 ? int(uint32_t(y) - (C - 4)) : int(y & 3);
     const bool owner = ti == yq % BS;
     float xy = 0.0f;
     if (owner) {
@@ -562,7 +727,7 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
       for (int u = 0; u < V; ++u)
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          if (uint32_t(u) == yq / BS && c == int(y & 3)) xy = v[u][c];
+          if (uint32_t(u) == yq / BS && c == yc) xy = v[u][c];
     }
     __syncthreads();
     if (next) *next = tk;
@@ -579,11 +744,12 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
 #pragma unroll
     for (int u = 0; u < V; ++u) {
       const bool in = uint32_t(u) < full || ti + uint32_t(u) * BS < C4;
+      const uint32_t lo = RAGGED ? own(ti + uint32_t(u) * BS) : 0;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
+      for (uint32_t c = 0; c < 4; ++c) {
         const float e = exp_le0_finite(v[u][c] - M);
         v[u][c] = e;
-        sl += in ? e : 0.0f;
+        sl += (RAGGED ? c >= lo : in) ? e : 0.0f;
       }
     }
     sl = wave_sum(sl);
@@ -626,10 +792,18 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
         if (owner && uint32_t(u) == yq / BS && live) {
 #pragma unroll
           for (int c = 0; c < 4; ++c)
-            if (c == int(y & 3)) o[c] = g * (v[u][c] * inv - 1.0f);
+            if (c == yc) o[c] = g * (v[u][c] * inv - 1.0f);
         }
-        if (uint32_t(u) < full || q < C4)
-          store_stream<PLAST_CE_NT_STORE>(o, reinterpret_cast<f4 *>(dr + q * 16u));
+        if (uint32_t(u) < full || q < C4) {
+          if constexpr (RAGGED) store_unit<PLAST_CE_NT_STORE>(o, reinterpret_cast<float *>(dr + q * 16u));
+          else store_stream<PLAST_CE_NT_STORE>(o, reinterpret_cast<f4 *>(dr + q * 16u));
+        } else if (RAGGED && q == C4) {
+#pragma unroll
+          for (uint32_t c = 0; c < 4; ++c) {
+            if (c >= 4 - rem) reinterpret_cast<float *>(dr)[C - 4 + c] = o[c];
+            else o[c] = 0.0f;  // the unit before's column
+          }
+        }
         v[u] = o;
       }
 #pragma unroll
@@ -643,17 +817,25 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
 #pragma unroll
       for (int u = 0; u < V; ++u) {
         const uint32_t q = ti + uint32_t(u) * BS;
-        if (q >= C4) continue;
-        const f4 xv = x4[q];
+        if (RAGGED ? q * 4 >= C : q >= C4) continue;
+        const uint32_t pos = RAGGED && q == C4 ? C - 4 : q * 4;
+        const f4 xv = RAGGED ? f4(*reinterpret_cast<const f4u *>(x + uint64_t(r) * C + pos)) : x4[q];
+        const uint32_t lo = RAGGED ? own(q) : 0;
         f4 o;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
+        for (uint32_t c = 0; c < 4; ++c) {
           const float sm = exp_le0((xv[c] - mx) - l);
-          const float oh = int32_t(q * 4 + c) == y ? 1.0f : 0.0f;
-          o[c] = g * (sm - oh);
+          const float oh = int32_t(pos + c) == y ? 1.0f : 0.0f;
+          o[c] = c >= lo ? g * (sm - oh) : 0.0f;
         }
         colsum[q] = colsum[q] + o;
-        store_stream<PLAST_CE_NT_STORE>(o, d4 + q);
+        if constexpr (!RAGGED) {
+          store_stream<PLAST_CE_NT_STORE>(o, d4 + q);
+        } else {
+#pragma unroll
+          for (uint32_t c = 0; c < 4; ++c)
+            if (c >= lo) dx[uint64_t(r) * C + pos + c] = o[c];
+        }
       }
     }
   };
@@ -704,11 +886,18 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
   // the workgroup's column sums: partial row b of part, in dispatch order under the dynamic
   // order (the rows each workgroup took vary from run to run) and by the static schedule's
   // numbering otherwise
-  f4 *p4 = reinterpret_cast<f4 *>(part + uint64_t(DYN ? blockIdx.x : row_block()) * C);
+  float *pb = part + uint64_t(DYN ? blockIdx.x : row_block()) * C;
 #pragma unroll
   for (int u = 0; u < V; ++u) {
     const uint32_t q = t + uint32_t(u) * BS;
-    if (q < C4) p4[q] = colsum[q];
+    if (q < C4) {
+      if constexpr (RAGGED) store_unit<false>(colsum[q], pb + 4 * q);
+      else reinterpret_cast<f4 *>(pb)[q] = colsum[q];
+    } else if (RAGGED && q == C4) {
+#pragma unroll
+      for (uint32_t c = 0; c < 4; ++c)
+        if (c >= 4 - rem) pb[C - 4 + c] = colsum[q][c];
+    }
   }
 }
 
@@ -801,6 +990,145 @@ __global__ __launch_bounds__(kCeBlock) void ce_step_tail(const float *__restrict
   dbias[c] = u;
 }
 
+// The step for rows of at most 4 * L * U floats (kWaveRow): L lanes hold a row in registers, 64 / L
+// rows per wave, and persistent workgroups of W waves walk the row groups with the next group's loads
+// in flight. A lane always holds the same columns, so their gradient sums stay in its registers
+// until the end, when the workgroup's waves add up through LDS in a fixed tree and write part[b]:
+// the bias gradient is the same bits on every call in either mode. One read and one write per logit
+// and no barrier per row (the workgroup-per-row kernel above takes 450 us for 60000 rows of 12 to
+// 1024 logits, all of it barriers and idle lanes).
+// Waves per workgroup, one workgroup per CU: 16, or 8 where two sets of eight units want more than the
+// 128 registers that 16 leave a lane. [60000, 128] / [60000, 512] / [60000, 1024]: 22.4 / 53.6 / 95.8 us
+// with 16, 25.2 / 63.2 / 116.5 with 8, 31.6 / 96.1 / 188 with 4.
+template <int U>
+constexpr int kStepRowsWaves = U == 8 ? 8 : 16;
+
+template <int L, int U>
+__global__ __launch_bounds__(64 * kStepRowsWaves<U>) void ce_step_rows_kernel(
+    const float *__restrict__ x, const int32_t *__restrict__ lab, const float *__restrict__ dloss,
+    float *__restrict__ stats, float *__restrict__ loss, float *__restrict__ dx,
+    float *__restrict__ part, uint32_t N, uint32_t C, uint32_t simd_end) {
+  constexpr int W = kStepRowsWaves<U>, P = 64 / L;  // rows per wave
+  __shared__ f4 sh[W / 2][L * U];
+  const int lane = threadIdx.x & 63, l = lane % L;
+  const uint32_t wave = threadIdx.x >> 6, groups = (N + P - 1) / P;
+  f4 acc[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) acc[u] = f4(0.0f);
+  // group `gr`'s row of this lane (the last row again past the end), its label and upstream gradient
+  const auto load = [&](uint32_t gr, f4 (&v)[U], int32_t &y, float &g) {
+    const uint32_t r = gr * P + lane / L < N && gr < groups ? gr * P + lane / L : N - 1;
+    y = lab[r];
+    g = dloss[r];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = load_row_part(x + uint64_t(r) * C, row_unit(uint32_t(l) + u * L, C), C);
+    pin_loads();
+  };
+  const auto process = [&](uint32_t gr, f4 (&v)[U], const int32_t y, const float g) {
+    const uint32_t r = gr * P + lane / L;
+    const bool valid = r < N;
+    float M = -__builtin_huge_valf(), mn = __builtin_huge_valf();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        M = fmaxf(M, v[u][c]);
+        mn = fminf(mn, v[u][c]);
+      }
+    M = group_max<L>(M);
+    mn = group_min<L>(mn);
+    float S = 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const RowUnit ru = row_unit(uint32_t(l) + u * L, C);
+#pragma unroll
+      for (uint32_t c = 0; c < 4; ++c) {
+        const float e = exp_le0(v[u][c] - M);
+        v[u][c] = e;
+        S += c >= ru.lo && c < ru.hi ? e : 0.0f;
+      }
+    }
+    S = group_sum<L>(S);
+    float mx = M, lg = logf(S);
+    bool bad = false, exact = valid && ce_needs_exact(M, S, mn, lg);
+    for (uint64_t todo = __ballot(exact && l == 0); todo; todo &= todo - 1) {
+      const int first = __ffsll((unsigned long long)todo) - 1;  // the row's first lane
+      float m1, l1;
+      bool b1;
+      ce_wave_exact(x + uint64_t(gr * P + first / L) * C, C, __shfl(y, first), lane, m1, l1, b1);
+      if (lane / L == first / L) mx = m1, lg = l1, bad = b1;
+    }
+    if (!valid) return;
+    const float *xr = x + uint64_t(r) * C;
+    float *dr = dx + uint64_t(r) * C;
+    if (l == 0) ce_row_out(xr, C, y, mx, lg, bad, r, simd_end, loss, stats);
+    const float inv = 1.0f / S, gs = g * inv;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const RowUnit ru = row_unit(uint32_t(l) + u * L, C);
+      f4 o;
+      if (exact) {  // from memory, as the backward op computes it
+        const f4 xv = load_row_part(xr, ru, C);
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+          const float sm = exp_le0((xv[c] - mx) - lg);
+          o[c] = g * (sm - (int32_t(ru.pos + c) == y ? 1.0f : 0.0f));
+        }
+      } else {
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c)
+          o[c] = int32_t(ru.pos + c) == y ? g * (v[u][c] * inv - 1.0f) : v[u][c] * gs;
+      }
+      store_row_part(o, dr, ru);
+#pragma unroll
+      for (uint32_t c = 0; c < 4; ++c) acc[u][c] += c >= ru.lo && c < ru.hi ? o[c] : 0.0f;
+    }
+  };
+  // wave w of workgroup b takes groups (w, b), (w + W, b), ... numbered w * G + b: the first G groups
+  // go to the workgroups' first waves
+  const uint32_t G = gridDim.x, step = G * W;
+  f4 va[U], vb[U];
+  int32_t ya, yb;
+  float ga, gb;
+  uint32_t gr = wave * G + blockIdx.x;
+  load(gr, va, ya, ga);
+  for (; gr < groups; gr += 2 * step) {
+    load(gr + step, vb, yb, gb);
+    process(gr, va, ya, ga);
+    load(gr + 2 * step, va, ya, ga);
+    if (gr + step < groups) process(gr + step, vb, yb, gb);
+  }
+  // the wave's rows: lanes with the same l
+#pragma unroll
+  for (int m = L; m < 64; m <<= 1)
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) acc[u][c] += __shfl_xor(acc[u][c], m);
+  // the workgroup's waves: the upper half hands its sums to the lower half, which halves again
+#pragma unroll
+  for (uint32_t h = W / 2; h >= 1; h /= 2) {
+    if (wave >= h && wave < 2 * h && lane < L) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) sh[wave - h][l + u * L] = acc[u];
+    }
+    __syncthreads();
+    if (wave < h && lane < L) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) acc[u] = acc[u] + sh[wave][l + u * L];
+    }
+    __syncthreads();
+  }
+  if (wave != 0 || lane >= L) return;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const RowUnit ru = row_unit(uint32_t(l) + u * L, C);
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c)
+      if (c >= ru.lo && c < ru.hi) part[uint64_t(blockIdx.x) * C + ru.pos + c] = acc[u][c];
+  }
+}
+
 // Whether ce_step_kernel<V> may be launched with its dynamic LDS (raising its limit once: beyond
 // the default the kernel has to opt in).
 template <int V>
@@ -808,8 +1136,10 @@ bool ce_step_lds_ok() {
   static bool granted = false;
   if (granted) return true;
   const int bytes = kStepBlock * V * int(sizeof(f4));
-  for (const void *k : {reinterpret_cast<const void *>(&ce_step_kernel<V, true>),
-                        reinterpret_cast<const void *>(&ce_step_kernel<V, false>)})
+  for (const void *k : {reinterpret_cast<const void *>(&ce_step_kernel<V, true, false>),
+                        reinterpret_cast<const void *>(&ce_step_kernel<V, false, false>),
+                        reinterpret_cast<const void *>(&ce_step_kernel<V, true, true>),
+                        reinterpret_cast<const void *>(&ce_step_kernel<V, false, true>)})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
       (void)hipGetLastError();  // not an error of the call: the caller takes the three passes
       return false;
@@ -841,13 +1171,17 @@ void ce_step_launch_v(int want, unsigned grid, float *part, const float *logits,
       return;
     }
     const size_t lds = size_t(kStepBlock) * V * sizeof(f4);
+    const auto run = [&](auto dynamic, auto ragged) {
+      ce_step_kernel<V, decltype(dynamic)::value, decltype(ragged)::value>
+          <<<grid, kStepBlock, lds, stream()>>>(logits, labels, dloss, stats, loss, dlogits, part, N, C,
+                                                uint32_t(simd_end(N)));
+    };
     // the dynamic row order unless results must not depend on timing (plast_hip_set_deterministic)
-    if (deterministic())
-      ce_step_kernel<V, false><<<grid, kStepBlock, lds, stream()>>>(
-          logits, labels, dloss, stats, loss, dlogits, part, N, C, uint32_t(simd_end(N)));
-    else
-      ce_step_kernel<V, true><<<grid, kStepBlock, lds, stream()>>>(
-          logits, labels, dloss, stats, loss, dlogits, part, N, C, uint32_t(simd_end(N)));
+    const bool ragged = C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits);
+    if (deterministic() && ragged) run(std::false_type{}, std::true_type{});
+    else if (deterministic()) run(std::false_type{}, std::false_type{});
+    else if (ragged) run(std::true_type{}, std::true_type{});
+    else run(std::true_type{}, std::false_type{});
   }
 }
 
@@ -870,8 +1204,8 @@ int ce_step_form(const float *logits, const int32_t *labels, const float *dloss,
   }
   // the column sums live in LDS (one float4 slot per lane and unit, the row's plus padding): the
   // kernel must be allowed that much of it
-  if (C % 4 == 0 && C <= kStepMaxC && aligned16(logits) && aligned16(dlogits))
-    return ce_step_units<1>(C);
+  if (C <= kWaveRow) return 1;  // ce_step_rows_kernel
+  if (C <= kStepMaxC) return ce_step_units<1>(C);
   return 0;
 }
 
@@ -881,6 +1215,13 @@ int ce_step_form(const float *logits, const int32_t *labels, const float *dloss,
 // sums for (kScratchFloats / C; on MI355X, 256 CUs of rows up to 32768 floats, never binding).
 uint64_t ce_step_grid(uint64_t N, uint64_t C) {
   uint64_t grid = uint64_t(num_cus()) * PLAST_CE_STEP_WPC;
+  if (C <= kWaveRow) {
+    // four row groups per workgroup before another one is added: each adds a row to the tail's sum
+    uint64_t rows = 1;
+    with_row_lanes<kWaveRow>(uint32_t(C), [&](auto lanes, auto) { rows = 4 * (64 / decltype(lanes)::value); });
+    const uint64_t need = (N + rows - 1) / rows;
+    return need < grid ? need : grid;
+  }
   if (grid > kScratchFloats / C) grid = kScratchFloats / C;
   return N < grid ? N : grid;
 }
@@ -902,7 +1243,14 @@ void ce_step_launch(int V, unsigned grid, float *part, const float *logits, cons
                     const float *dloss, float *stats, float *loss, float *dlogits, float *dbias,
                     float *mean_loss, uint64_t N, uint64_t C) {
   const uint32_t c32 = uint32_t(C);
-  ce_step_launch_v<1>(V, grid, part, logits, labels, dloss, stats, loss, dlogits, uint32_t(N), c32);
+  if (C <= kWaveRow)
+    with_row_lanes<kWaveRow>(c32, [&](auto lanes, auto units) {
+      constexpr int L = decltype(lanes)::value, U = decltype(units)::value;
+      ce_step_rows_kernel<L, U><<<grid, 64 * kStepRowsWaves<U>, 0, stream()>>>(
+          logits, labels, dloss, stats, loss, dlogits, part, uint32_t(N), c32, uint32_t(simd_end(N)));
+    });
+  else
+    ce_step_launch_v<1>(V, grid, part, logits, labels, dloss, stats, loss, dlogits, uint32_t(N), c32);
   step_tail(part, dbias, C, grid, loss, mean_loss, N);
 }
 
@@ -957,23 +1305,79 @@ __global__ __launch_bounds__(kCeBlock) void softmax_fwd_kernel(const float *__re
   }
 }
 
+// Softmax / log-softmax forward over rows of at most 4 * L * U floats in a wave's registers, L lanes
+// each: the operations of softmax_fwd_kernel, with the row's sum in the lanes' fixed tree. No
+// barrier, and a wave's loads fill its lanes whatever the row length.
+template <bool LOG, int L, int U>
+__global__ __launch_bounds__(kCeBlock) void softmax_fwd_rows_kernel(const float *__restrict__ x,
+                                                                    float *__restrict__ y, uint64_t N,
+                                                                    uint32_t C) {
+  const int lane = threadIdx.x & 63, l = lane % L;
+  const uint64_t row0 = (uint64_t(blockIdx.x) * kCeWaves + (threadIdx.x >> 6)) * (64 / L);
+  if (row0 >= N) return;  // whole wave
+  const uint64_t row = row0 + lane / L;
+  const bool valid = row < N;
+  const float *xr = x + (valid ? row : N - 1) * C;
+  f4 v[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) v[u] = load_row_part(xr, row_unit(uint32_t(l) + u * L, C), C);
+  float M = -__builtin_huge_valf(), nan = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      M = fmaxf(M, v[u][c]);
+      nan = v[u][c] != v[u][c] ? 1.0f : nan;
+    }
+  M = group_max<L>(M);
+  nan = group_max<L>(nan);
+  float mx = M > -FLT_MAX ? M : -FLT_MAX;
+  for (uint64_t todo = __ballot(valid && l == 0 && (nan != 0.0f || M == 0.0f)); todo; todo &= todo - 1) {
+    const int first = __ffsll((unsigned long long)todo) - 1;  // the row's first lane
+    const float m1 = wave_max_fold(x + (row0 + first / L) * C, C, lane);
+    if (lane / L == first / L) mx = m1;
+  }
+  float s = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const RowUnit r = row_unit(uint32_t(l) + u * L, C);
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c) {
+      const float t = v[u][c] - mx;
+      const float e = expf(t);
+      v[u][c] = LOG ? t : e;
+      s += c >= r.lo && c < r.hi ? e : 0.0f;
+    }
+  }
+  s = group_sum<L>(s);
+  const float lg = LOG ? logf(s) : 0.0f;
+  if (!valid) return;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const RowUnit r = row_unit(uint32_t(l) + u * L, C);
+    f4 o;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) o[c] = LOG ? v[u][c] - lg : v[u][c] / s;
+    store_row_part(o, y + row * C, r);
+  }
+}
+
 constexpr int kSoftmaxBlock = PLAST_SOFTMAX_BLOCK;
 
-// The same with the row held in registers, for rows of up to BS * 4 * V floats in whole
-// float4 (C % 4 == 0, 16-byte aligned rows): one read and one write per element. Each lane keeps V
-// float4 of the row; lanes past the row hold -inf, which adds exp(-inf) = 0 to no sum (they are
-// masked) and never wins the max. Same operations and order as softmax_fwd_kernel's three passes
-// but the exp-sum's grouping (per lane, then the block's fixed tree).
-template <bool LOG, int V, int BS = kSoftmaxBlock>
+// The same with the row held in registers, for rows of up to BS * 4 * V floats: one read and one
+// write per element. Each lane keeps V units of the row; lanes past the row hold -inf, which adds
+// exp(-inf) = 0 to no sum (they are masked) and never wins the max. Same operations and order as
+// softmax_fwd_kernel's three passes but the exp-sum's grouping (per lane, then the block's fixed
+// tree). RAGGED: rows of any length and alignment (RowUnit; [30000, 1500] forward and backward 180 us
+// with it, 164 without).
+template <bool LOG, int V, bool RAGGED, int BS = kSoftmaxBlock>
 __global__ __launch_bounds__(BS) void softmax_fwd_reg_kernel(const float *__restrict__ x,
                                                              float *__restrict__ y, uint32_t C) {
   constexpr int W = BS / 64;
   __shared__ float lds[W + 1];
   const uint64_t row = blockIdx.x;
   const float *xr = x + row * C;
-  const uint32_t C4 = C / 4;
-  const f4 *x4 = reinterpret_cast<const f4 *>(xr);
-  f4 *y4 = reinterpret_cast<f4 *>(y + row * C);
+  const uint32_t C4 = (C + 3) / 4;
   const float ninf = -__builtin_huge_valf();
   f4 v[V];
   float m = ninf;
@@ -981,7 +1385,8 @@ __global__ __launch_bounds__(BS) void softmax_fwd_reg_kernel(const float *__rest
 #pragma unroll
   for (int u = 0; u < V; ++u) {
     const uint32_t q = threadIdx.x + uint32_t(u) * BS;
-    v[u] = q < C4 ? __builtin_nontemporal_load(x4 + q) : f4(ninf);
+    if constexpr (RAGGED) v[u] = q < C4 ? load_row_part(xr, row_unit(q, C), C) : f4(ninf);
+    else v[u] = q < C4 ? __builtin_nontemporal_load(reinterpret_cast<const f4 *>(xr) + q) : f4(ninf);
   }
 #pragma unroll
   for (int u = 0; u < V; ++u) {
@@ -993,13 +1398,14 @@ __global__ __launch_bounds__(BS) void softmax_fwd_reg_kernel(const float *__rest
   float s = 0.0f;
 #pragma unroll
   for (int u = 0; u < V; ++u) {
-    const bool in = threadIdx.x + uint32_t(u) * BS < C4;
+    const uint32_t q = threadIdx.x + uint32_t(u) * BS;
+    const uint32_t lo = RAGGED && q < C4 ? row_unit(q, C).lo : 0;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
+    for (uint32_t c = 0; c < 4; ++c) {
       const float t = v[u][c] - mx;
       const float e = expf(t);
       v[u][c] = LOG ? t : e;
-      s += in ? e : 0.0f;
+      s += q < C4 && c >= lo ? e : 0.0f;
     }
   }
   s = block_sum<W>(s, lds);
@@ -1011,7 +1417,8 @@ __global__ __launch_bounds__(BS) void softmax_fwd_reg_kernel(const float *__rest
     f4 r;
 #pragma unroll
     for (int c = 0; c < 4; ++c) r[c] = LOG ? v[u][c] - l : v[u][c] / s;
-    y4[q] = r;
+    if constexpr (RAGGED) store_row_part(r, y + row * C, row_unit(q, C));
+    else reinterpret_cast<f4 *>(y + row * C)[q] = r;
   }
 }
 
@@ -1206,17 +1613,57 @@ __global__ __launch_bounds__(kCeBlock) void softmax_bwd_kernel(const float *__re
   }
 }
 
+// The same over rows of at most 4 * L * U floats in a wave's registers, L lanes each.
+template <bool LOG, int L, int U>
+__global__ __launch_bounds__(kCeBlock) void softmax_bwd_rows_kernel(const float *__restrict__ y,
+                                                                    const float *__restrict__ dy,
+                                                                    float *dx, uint64_t N, uint32_t C) {
+  const int lane = threadIdx.x & 63, l = lane % L;
+  const uint64_t row0 = (uint64_t(blockIdx.x) * kCeWaves + (threadIdx.x >> 6)) * (64 / L);
+  if (row0 >= N) return;  // whole wave
+  const bool valid = row0 + lane / L < N;
+  const uint64_t row = valid ? row0 + lane / L : N - 1;
+  f4 yv[U], gv[U], dv[U];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const RowUnit r = row_unit(uint32_t(l) + u * L, C);
+    yv[u] = load_row_part(y + row * C, r, C);
+    gv[u] = load_row_part(dy + row * C, r, C);
+    dv[u] = load_row_part(dx + row * C, r, C);
+  }
+  float t = 0.0f;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const RowUnit r = row_unit(uint32_t(l) + u * L, C);
+#pragma unroll
+    for (uint32_t c = 0; c < 4; ++c)
+      t += c >= r.lo && c < r.hi ? (LOG ? gv[u][c] : gv[u][c] * yv[u][c]) : 0.0f;
+  }
+  t = group_sum<L>(t);
+  if (!valid) return;
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const RowUnit r = row_unit(uint32_t(l) + u * L, C);
+    f4 d = dv[u];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      d[c] = d[c] + (LOG ? gv[u][c] - expf(yv[u][c]) * t : yv[u][c] * (gv[u][c] - t));
+    store_row_part(d, dx + row * C, r);
+  }
+}
+
 // The backward with y and dy of a row held in registers (rows of whole float4 up to BS * 4 * V
 // floats): y, dy and dx are each read once and dx written once. The sum's grouping is per lane,
 // then the block's fixed tree.
-template <bool LOG, int V, int BS>
+// RAGGED: rows of any length and alignment, their last unit partial (RowUnit).
+template <bool LOG, int V, int BS, bool RAGGED>
 __global__ __launch_bounds__(BS) void softmax_bwd_reg_kernel(const float *__restrict__ y,
                                                              const float *__restrict__ dy,
                                                              float *dx, uint32_t C) {
   constexpr int W = BS / 64;
   __shared__ float lds[W + 1];
   const uint64_t row = blockIdx.x;
-  const uint32_t C4 = C / 4;
+  const uint32_t C4 = RAGGED ? (C + 3) / 4 : C / 4;
   const f4 *y4 = reinterpret_cast<const f4 *>(y + row * C);
   const f4 *g4 = reinterpret_cast<const f4 *>(dy + row * C);
   f4 *d4 = reinterpret_cast<f4 *>(dx + row * C);
@@ -1231,6 +1678,13 @@ __global__ __launch_bounds__(BS) void softmax_bwd_reg_kernel(const float *__rest
   for (int u = 0; u < V; ++u) {
     const uint32_t q = threadIdx.x + uint32_t(u) * BS;
     const uint32_t qc = q < C4 ? q : C4 - 1;
+    if constexpr (RAGGED) {
+      const RowUnit r = row_unit(qc, C);
+      yv[u] = load_row_part(y + row * C, r, C);
+      gv[u] = load_row_part(dy + row * C, r, C);
+      if (u < kPre) dv[u] = load_row_part(dx + row * C, r, C);
+      continue;
+    }
     yv[u] = __builtin_nontemporal_load(y4 + qc);
     gv[u] = __builtin_nontemporal_load(g4 + qc);
     if (u < kPre) dv[u] = PLAST_SOFTMAX_BWD_NT ? __builtin_nontemporal_load(d4 + qc) : d4[qc];
@@ -1238,9 +1692,10 @@ __global__ __launch_bounds__(BS) void softmax_bwd_reg_kernel(const float *__rest
   float t = 0.0f;
 #pragma unroll
   for (int u = 0; u < V; ++u) {
-    const bool in = threadIdx.x + uint32_t(u) * BS < C4;
+    const uint32_t q = threadIdx.x + uint32_t(u) * BS;
+    const uint32_t lo = RAGGED && q < C4 ? row_unit(q, C).lo : 0;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) t += in ? (LOG ? gv[u][c] : gv[u][c] * yv[u][c]) : 0.0f;
+    for (uint32_t c = 0; c < 4; ++c) t += q < C4 && c >= lo ? (LOG ? gv[u][c] : gv[u][c] * yv[u][c]) : 0.0f;
   }
   t = block_sum<W>(t, lds);
 #pragma unroll
@@ -1249,11 +1704,13 @@ __global__ __launch_bounds__(BS) void softmax_bwd_reg_kernel(const float *__rest
     if (q >= C4) continue;
     f4 d;
     if (u < kPre) d = dv[u < kPre ? u : 0];
+    else if constexpr (RAGGED) d = load_row_part(dx + row * C, row_unit(q, C), C);
     else d = PLAST_SOFTMAX_BWD_NT ? __builtin_nontemporal_load(d4 + q) : d4[q];
 #pragma unroll
     for (int c = 0; c < 4; ++c)
       d[c] = d[c] + (LOG ? gv[u][c] - expf(yv[u][c]) * t : yv[u][c] * (gv[u][c] - t));
-    store_stream<PLAST_SOFTMAX_BWD_NT>(d, d4 + q);
+    if constexpr (RAGGED) store_row_part(d, dx + row * C, row_unit(q, C));
+    else store_stream<PLAST_SOFTMAX_BWD_NT>(d, d4 + q);
   }
 }
 
@@ -1287,28 +1744,32 @@ void softmax_forward(const Tensor **inputs, Tensor *output, KernelParams params,
   const uint32_t C = uint32_t(x->shape[x->ndim - 1]);
   const uint64_t N = C ? numel(x) / C : 0;
   const uint64_t R = max_blocks(kCeBlock);
+  const float *px0 = static_cast<const float *>(x->data);
+  float *py0 = static_cast<float *>(output->data);
+  if (C <= kSoftmaxWaveRow) {
+    for (uint64_t r0 = 0; r0 < N; r0 += R) {
+      const uint64_t n = N - r0 < R ? N - r0 : R;
+      with_row_lanes<kSoftmaxWaveRow>(C, [&](auto lanes, auto units) {
+        constexpr int L = decltype(lanes)::value, U = decltype(units)::value;
+        softmax_fwd_rows_kernel<LOG, L, U>
+            <<<unsigned(ceil_div(n, kCeWaves * (64 / L))), kCeBlock, 0, stream()>>>(
+                px0 + r0 * C, py0 + r0 * C, n, C);
+      });
+    }
+    finish(where);
+    return;
+  }
   // float4 units per lane for a register-resident row (0: the three-pass kernel)
   int V = 0;
-  if (C % 4 == 0 && aligned16(x->data) && aligned16(output->data))
-    for (int v = 1; v <= 32 && !V; v *= 2)
-      if (uint64_t(C) <= uint64_t(kSoftmaxBlock) * 4 * v) V = v;
-  // rows of 2048..32768 floats: the persistent form (rows at a time below 2^31)
-  int SV = 0;
-  if (V && C >= 2048 && N < (uint64_t(1) << 31))
-    for (int v = 1; v <= 8 && !SV; v *= 2)
-      if (uint64_t(C) <= uint64_t(kStepBlock) * 4 * v) SV = v;
-  if (SV) {
+  const bool ragged = C % 4 != 0 || !aligned16(px0) || !aligned16(py0);
+  for (int v = 1; v <= 32 && !V; v *= 2)
+    if (uint64_t(C) <= uint64_t(kSoftmaxBlock) * 4 * v) V = v;
+  // long rows of whole float4: the persistent form (rows at a time below 2^31)
+  constexpr int SV = 8;
+  if (!ragged && C >= PLAST_SOFTMAX_PERSISTENT && C <= uint32_t(kStepBlock) * 4 * SV &&
+      N < (uint64_t(1) << 31)) {
     const unsigned G = unsigned(N < uint64_t(num_cus()) ? N : uint64_t(num_cus()));
-    const float *px = static_cast<const float *>(x->data);
-    float *py = static_cast<float *>(output->data);
-    const uint32_t n32 = uint32_t(N);
-    constexpr bool D = PLAST_ROW_DYNAMIC;
-    switch (SV) {
-      case 1: softmax_fwd_step_kernel<LOG, 1, D><<<G, kStepBlock, 0, stream()>>>(px, py, n32, C); break;
-      case 2: softmax_fwd_step_kernel<LOG, 2, D><<<G, kStepBlock, 0, stream()>>>(px, py, n32, C); break;
-      case 4: softmax_fwd_step_kernel<LOG, 4, D><<<G, kStepBlock, 0, stream()>>>(px, py, n32, C); break;
-      default: softmax_fwd_step_kernel<LOG, 8, D><<<G, kStepBlock, 0, stream()>>>(px, py, n32, C); break;
-    }
+    softmax_fwd_step_kernel<LOG, SV, PLAST_ROW_DYNAMIC><<<G, kStepBlock, 0, stream()>>>(px0, py0, uint32_t(N), C);
     finish(where);
     return;
   }
@@ -1316,13 +1777,17 @@ void softmax_forward(const Tensor **inputs, Tensor *output, KernelParams params,
     const unsigned n = unsigned(N - r0 < R ? N - r0 : R);
     const float *px = static_cast<const float *>(x->data) + r0 * C;
     float *py = static_cast<float *>(output->data) + r0 * C;
+    const auto reg = [&](auto units) {
+      constexpr int U = decltype(units)::value;
+      if (ragged) softmax_fwd_reg_kernel<LOG, U, true><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C);
+      else softmax_fwd_reg_kernel<LOG, U, false><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C);
+    };
     switch (V) {
-      case 1: softmax_fwd_reg_kernel<LOG, 1><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C); break;
-      case 2: softmax_fwd_reg_kernel<LOG, 2><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C); break;
-      case 4: softmax_fwd_reg_kernel<LOG, 4><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C); break;
-      case 8: softmax_fwd_reg_kernel<LOG, 8><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C); break;
-      case 16: softmax_fwd_reg_kernel<LOG, 16><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C); break;
-      case 32: softmax_fwd_reg_kernel<LOG, 32><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C); break;
+      case 2: reg(std::integral_constant<int, 2>{}); break;
+      case 4: reg(std::integral_constant<int, 4>{}); break;
+      case 8: reg(std::integral_constant<int, 8>{}); break;
+      case 16: reg(std::integral_constant<int, 16>{}); break;
+      case 32: reg(std::integral_constant<int, 32>{}); break;
       default: softmax_fwd_kernel<LOG><<<n, kCeBlock, 0, stream()>>>(px, py, C); break;
     }
   }
@@ -1346,24 +1811,34 @@ void softmax_backward(Tensor **inputs, const Tensor *output, KernelParams params
   constexpr int BS = PLAST_SOFTMAX_BWD_BLOCK;  // y and dy in registers: 512 lanes keep V at 16
                                               // for 32768-float rows
   int V = 0;
-  if (C % 4 == 0 && aligned16(output->data) && aligned16(output->grad->data) &&
-      aligned16(x->grad->data))
-    for (int v = 1; v <= 16 && !V && v * BS <= 8192; v *= 2)
-      if (uint64_t(C) <= uint64_t(BS) * 4 * v) V = v;
+  const bool ragged = C % 4 != 0 || !aligned16(output->data) || !aligned16(output->grad->data) ||
+                      !aligned16(x->grad->data);
+  for (int v = 1; v <= 16 && !V && v * BS <= 8192; v *= 2)
+    if (uint64_t(C) <= uint64_t(BS) * 4 * v) V = v;
   for (uint64_t r0 = 0; r0 < N; r0 += R) {
     const unsigned n = unsigned(N - r0 < R ? N - r0 : R);
     const float *py = static_cast<const float *>(output->data) + r0 * C;
     const float *pg = static_cast<const float *>(output->grad->data) + r0 * C;
     float *pd = static_cast<float *>(x->grad->data) + r0 * C;
+    if (C <= kSoftmaxBwdWaveRow) {
+      with_row_lanes<kSoftmaxWaveRow>(C, [&](auto lanes, auto units) {
+        constexpr int L = decltype(lanes)::value, U = decltype(units)::value;
+        softmax_bwd_rows_kernel<LOG, L, U>
+            <<<unsigned(ceil_div(n, kCeWaves * (64 / L))), kCeBlock, 0, stream()>>>(py, pg, pd, n, C);
+      });
+      continue;
+    }
+    const auto reg = [&](auto units) {
+      constexpr int U = decltype(units)::value;
+      if (ragged) softmax_bwd_reg_kernel<LOG, U, BS, true><<<n, BS, 0, stream()>>>(py, pg, pd, C);
+      else softmax_bwd_reg_kernel<LOG, U, BS, false><<<n, BS, 0, stream()>>>(py, pg, pd, C);
+    };
     switch (V) {
-      case 1: softmax_bwd_reg_kernel<LOG, 1, BS><<<n, BS, 0, stream()>>>(py, pg, pd, C); break;
-      case 2: softmax_bwd_reg_kernel<LOG, 2, BS><<<n, BS, 0, stream()>>>(py, pg, pd, C); break;
-      case 4: softmax_bwd_reg_kernel<LOG, 4, BS><<<n, BS, 0, stream()>>>(py, pg, pd, C); break;
-      case 8: softmax_bwd_reg_kernel<LOG, 8, BS><<<n, BS, 0, stream()>>>(py, pg, pd, C); break;
-      case 16:
-        if constexpr (16 * BS <= 8192)
-          softmax_bwd_reg_kernel<LOG, 16, BS><<<n, BS, 0, stream()>>>(py, pg, pd, C);
-        break;
+      case 1: reg(std::integral_constant<int, 1>{}); break;
+      case 2: reg(std::integral_constant<int, 2>{}); break;
+      case 4: reg(std::integral_constant<int, 4>{}); break;
+      case 8: reg(std::integral_constant<int, 8>{}); break;
+      case 16: reg(std::integral_constant<int, 16>{}); break;
       default: softmax_bwd_kernel<LOG><<<n, kCeBlock, 0, stream()>>>(py, pg, pd, C); break;
     }
   }
@@ -1392,8 +1867,7 @@ void softmax_cross_entropy_hip_forward(const Tensor **inputs, Tensor *output, Ke
   if (N == 0) return;
   // The NEG node of the reference chain runs over the [N] (or [N,1]) loss tensor.
   const uint64_t se = simd_end(N);
-  const bool vec = C % 4 == 0 && aligned16(static_cast<const float *>(x->data)) && C > 0;
-  // rows per launch: one workgroup per row (generic) or one wave per row (vectorised)
+  // rows per launch: at most one workgroup for each
   const uint64_t R = max_blocks(kCeBlock);
   for (uint64_t r0 = 0; r0 < N; r0 += R) {
     const uint64_t n = N - r0 < R ? N - r0 : R;
@@ -1402,11 +1876,15 @@ void softmax_cross_entropy_hip_forward(const Tensor **inputs, Tensor *output, Ke
     float *ps = static_cast<float *>(st->data) + 2 * r0;
     float *po = static_cast<float *>(output->data) + r0;
     const uint64_t ser = se > r0 ? se - r0 : 0;  // the rule's boundary, relative to this range
-    if (vec)
+    if (C > 0 && C <= kCeWaveRow)
+      with_row_lanes<kCeWaveRow>(C, [&](auto lanes, auto units) {
+        constexpr int L = decltype(lanes)::value, U = decltype(units)::value;
+        ce_fwd_rows_kernel<L, U><<<unsigned(ceil_div(n, kCeWaves * (64 / L))), kCeBlock, 0, stream()>>>(
+            px, pl, ps, po, n, C, ser);
+      });
+    else
       ce_fwd_wave_kernel<<<unsigned(ceil_div(n, kCeFwdWaves)), 64 * kCeFwdWaves, 0, stream()>>>(
           px, pl, ps, po, n, C, ser);
-    else
-      ce_fwd_generic_kernel<<<unsigned(n), kCeBlock, 0, stream()>>>(px, pl, ps, po, C, ser);
   }
   finish(where);
 }
@@ -1429,16 +1907,11 @@ void softmax_cross_entropy_hip_backward(Tensor **inputs, const Tensor *output, K
   if (N == 0 || C == 0) return;
 
   const bool vec = C % 4 == 0 && aligned16(x->data) && aligned16(x->grad->data);
-  // each workgroup covers kBwdUnroll float4 per lane of one row
-  const uint32_t per_block = kCeBlock * kBwdUnroll * 4;
-  const uint32_t chunks = ceil_div(C, per_block);
   const bool over = params.keepdim == 1;
-  const uint64_t C4 = C / 4;
-  // rows per launch, so that every grid below stays within the dispatch limit
-  uint64_t R = max_blocks(kCeBlock) / chunks;
-  if (vec && C4 && R > max_blocks(kCeBlock) * kCeBlock / C4) R = max_blocks(kCeBlock) * kCeBlock / C4;
-  if (vec && C4 && R > max_blocks(kCeFlatBlock) * kCeFlatBlock / C4)
-    R = max_blocks(kCeFlatBlock) * kCeFlatBlock / C4;
+  // rows per launch, so that every grid below stays within the dispatch limit and element numbers
+  // within 32 bits
+  uint64_t R = (vec ? max_blocks(kCeFlatBlock) * kCeFlatBlock : (uint64_t(1) << 32) - 4) /
+               (vec ? C / 4 : C);
   if (R == 0) R = 1;
   for (uint64_t r0 = 0; r0 < N; r0 += R) {
     const uint64_t n = N - r0 < R ? N - r0 : R;
@@ -1447,19 +1920,17 @@ void softmax_cross_entropy_hip_backward(Tensor **inputs, const Tensor *output, K
     const int32_t *pl = static_cast<const int32_t *>(lab->data) + r0;
     const float *ps = static_cast<const float *>(st->data) + 2 * r0;
     const float *pg = static_cast<const float *>(output->grad->data) + r0;
-    const unsigned grid = unsigned(uint64_t(chunks) * n);
-    const uint64_t units = n * C4;
-    if (vec) {
-      const MagicDiv dc4 = MagicDiv::make(uint32_t(C4));
-      const unsigned g = unsigned(ceil_div(units, kCeFlatBlock));
-      if (over)
-        ce_bwd_flat_kernel<true><<<g, kCeFlatBlock, 0, stream()>>>(px, pl, ps, pg, pd, dc4, uint32_t(units));
-      else
-        ce_bwd_flat_kernel<false><<<g, kCeFlatBlock, 0, stream()>>>(px, pl, ps, pg, pd, dc4, uint32_t(units));
-    } else if (over)
-      ce_bwd_scalar_kernel<true><<<grid, kCeBlock, 0, stream()>>>(px, pl, ps, pg, pd, C, chunks);
+    const uint64_t units = (n * C + 3) / 4;
+    const MagicDiv dc = MagicDiv::make(vec ? C / 4 : C);
+    const unsigned g = unsigned(ceil_div(units, kCeFlatBlock));
+    if (vec && over)
+      ce_bwd_flat_kernel<true><<<g, kCeFlatBlock, 0, stream()>>>(px, pl, ps, pg, pd, dc, uint32_t(units));
+    else if (vec)
+      ce_bwd_flat_kernel<false><<<g, kCeFlatBlock, 0, stream()>>>(px, pl, ps, pg, pd, dc, uint32_t(units));
+    else if (over)
+      ce_bwd_ragged_kernel<true><<<g, kCeFlatBlock, 0, stream()>>>(px, pl, ps, pg, pd, dc, uint32_t(n * C));
     else
-      ce_bwd_scalar_kernel<false><<<grid, kCeBlock, 0, stream()>>>(px, pl, ps, pg, pd, C, chunks);
+      ce_bwd_ragged_kernel<false><<<g, kCeFlatBlock, 0, stream()>>>(px, pl, ps, pg, pd, dc, uint32_t(n * C));
   }
   finish(where);
 }
@@ -1530,7 +2001,7 @@ void softmax_cross_entropy_step_noalloc_hip(const float *logits, const int32_t *
   }
   const int V = ce_step_form(logits, labels, dloss, stats, loss, dlogits, N, C, where);
   if (V < 0) return;
-  if (V == 0) {
+  if (V == 0 || C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits)) {
     report_error(where, "rows of %llu floats are not one-pass rows (whole float4, 16-byte aligned "
                  "logits and dlogits, at most %llu floats): the three-pass form allocates",
                  (unsigned long long)C, (unsigned long long)kStepMaxC);

@@ -1,0 +1,106 @@
+"""Cross-entropy and softmax over short rows (2, 8, 32 or 64 lanes a row in a wave's registers) and over
+rows of any length and alignment, on each side of the lengths where the kernel changes, against the
+oracle at the bars of tests/test_gpu_ce_step.py and tests/test_gpu_softmax.py: clean rows and the
+special ones (NaN, infinities, zero maxima, extreme spreads), more rows than the step's workgroups
+hold at once, and results that repeat bit for bit. A gradient's scale has the floor 1e-2 * g: its
+bar is then at least 1e-7 * g, the rounding of g * (p - 1) for p next to 1 (an ulp of p is 6e-8; the
+same floor as 1e-2 / N where g = 1 / N)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cases import assert_bits, check_ce_rows
+from test_gpu_ce_step import _oracle, _special_rows, _step
+from test_gpu_ce_step import test_step_matches_oracle as step_case
+from test_gpu_softmax import test_softmax_forward_and_backward as softmax_case
+
+pytestmark = pytest.mark.gpu
+
+ROW = [1, 2, 3, 4, 5, 10, 31, 32, 33, 127, 128, 129, 511, 512, 513, 1001, 1024, 1025, 2047, 2048, 2049,
+       2050, 4097, 8191]
+
+
+@pytest.mark.parametrize("C", ROW)
+def test_cross_entropy_op(C):
+    """The op's forward and its accumulating and overwriting backward; the special rows need C > 3."""
+    from plast_amd import ops, runtime as rt
+    from plast_amd.abi import KernelParams
+    N = 203
+    print(f"ce op {N}x{C}", flush=True)
+    rng = np.random.RandomState(C)
+    x = (rng.randn(N, C) * 2).astype(np.float32)
+    if C > 3:
+        _special_rows(x)
+    lab = rng.randint(0, C, N).astype(np.int32)
+    g = rng.uniform(0.1, 1.0, N).astype(np.float32)
+    X, Lb = rt.DeviceTensor.from_numpy(x, requires_grad=True), rt.DeviceTensor.from_numpy(lab)
+    loss, stats = ops.softmax_cross_entropy(X, Lb, requires_grad=True)
+    rt.lib().arena_memcpy_h2d_hip(loss.grad.ptr, g.ctypes.data, g.nbytes)
+    rt.backward("softmax_cross_entropy", [X, Lb, stats], loss)
+    wst, wloss, wdx = _oracle(x, lab, g)
+    first = X.grad.numpy()
+    check_ce_rows(x, lab, g, stats.numpy(), loss.numpy(), first, wst, wloss, wdx, 1e-2 * g)
+    assert_bits(np.isnan(first), np.isnan(wdx), "NaN positions of dlogits")
+    rt.backward("softmax_cross_entropy", [X, Lb, stats], loss)
+    assert_bits(X.grad.numpy(), first + first, "accumulated gradient")
+    rt.backward("softmax_cross_entropy", [X, Lb, stats], loss, KernelParams(0, 1, 0.0))
+    assert_bits(X.grad.numpy(), first, "overwritten gradient")
+
+
+@pytest.mark.parametrize("special", [False, True], ids=["clean", "special_rows"])
+@pytest.mark.parametrize("N, C", [(1, 4), (9, 5), (700, 10), (301, 31), (77, 33), (130, 128), (41, 300),
+                                  (25, 513), (19, 1025), (300, 2046), (21, 2049), (33, 4099), (12, 9001),
+                                  (10, 32767)])
+def test_step(N, C, special):
+    step_case(N, C, special)
+
+
+@pytest.mark.parametrize("N, C", [(40000, 12), (20000, 77), (6000, 700), (3000, 2000), (1100, 2051)])
+def test_step_many_rows(N, C):
+    """Several row groups per wave: every row against the oracle, the same bits twice for short rows."""
+    from plast_amd import runtime as rt
+    print(f"ce step {N}x{C}", flush=True)
+    rng = np.random.RandomState(C)
+    x = (rng.randn(N, C) * 2).astype(np.float32)
+    x[N // 2, :] = 0.0     # a zero maximum, and an infinite logit, in later groups
+    x[N - 3, 1] = -np.inf
+    lab = rng.randint(0, C, N).astype(np.int32)
+    g = rng.uniform(0.1, 1.0, N).astype(np.float32)
+    X, Lb = rt.DeviceTensor.from_numpy(x), rt.DeviceTensor.from_numpy(lab)
+    st, loss, dx, db = _step(rt, X, Lb, g)
+    wst, wloss, wdx = _oracle(x, lab, g)
+    check_ce_rows(x, lab, g, st, loss, dx, wst, wloss, wdx, 1e-2 * g)
+    ok = np.isfinite(wdx).all(0)
+    want = wdx.astype(np.float64).sum(0)
+    bar = 1e-5 * np.abs(wdx.astype(np.float64)).sum(0) + 1e-12
+    assert np.all(np.abs(db - want)[ok] <= bar[ok])
+    if C <= 2048:
+        for a, b in zip(_step(rt, X, Lb, g), (st, loss, dx, db)):
+            assert_bits(a, b, "a second call")
+
+
+@pytest.mark.parametrize("log", [False, True], ids=["softmax", "log_softmax"])
+@pytest.mark.parametrize("C", ROW + [16381, 16388, 20001])
+def test_softmax_rows(C, log):
+    softmax_case((23, C), log)
+
+
+@pytest.mark.parametrize("off", [1, 2])
+@pytest.mark.parametrize("C", [100, 2052, 17000])
+def test_misaligned_rows(C, off):
+    """Rows of whole float4 in a buffer that does not start on one: the bits of the aligned call for
+    short rows, the fp64 softmax for the others (a longer row's kernel differs)."""
+    from plast_amd import runtime as rt
+    from plast_amd.abi import KernelParams
+    N = 7
+    print(f"softmax {N}x{C} offset {off}", flush=True)
+    x = np.random.RandomState(C + off).randn(N * C + off).astype(np.float32)
+    X, Y = rt.DeviceTensor.from_numpy(x), rt.DeviceTensor((N * C + 4,), zero=False)
+    vx = rt.DeviceTensor((N, C), base=X, offset=off, zero=False)
+    vy = rt.DeviceTensor((N, C), base=Y, offset=4 - off, zero=False)
+    rt.forward("softmax", [vx], vy, KernelParams(1, 0, 0.0))
+    h = x[off:].reshape(N, C).astype(np.float64)
+    e = np.exp(h - h.max(1, keepdims=True))
+    want = e / e.sum(1, keepdims=True)
+    assert np.all(np.abs(vy.numpy() - want) <= 1e-5 * want)
