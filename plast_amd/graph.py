@@ -22,6 +22,7 @@ class Graph:
         self._arena_bufs = []
         self._alloc_cb = abi.ArenaAllocFn(self._alloc)
         self.dag = None
+        self._run = None      # the DAG's calls, bound by build()
 
     # --- construction
     def node(self, op: str, inputs, output: DeviceTensor, p: KernelParams | None = None) -> DeviceTensor:
@@ -79,25 +80,41 @@ class Graph:
         if fuse:
             fused = lib().plast_hip_fuse_elementwise_chains(C.byref(dag), self._alloc_cb)
             lib().check("plast_hip_fuse_elementwise_chains")
+        self._run = None
         return int(fused)
 
     def op_types(self) -> list[str]:
         return [abi.OP_NAMES[self.dag.nodes[i].contents.op_type] for i in range(self.dag.count)]
 
-    def forward(self) -> None:
-        """dag_forward (graph.c:57-60): each node's GPU forward slot in order."""
-        L = lib()
+    def _calls(self):
+        """(forward slot, backward slot, inputs, output, params) of every node of the DAG, in order:
+        the objects ctypes would otherwise make anew for each field on every pass (2 us a node of
+        the 5 a small pass took). `inputs`, `output` and `params` read the node itself, so a node
+        changed after build() is run as changed; its slots are taken at build()."""
+        calls = []
         for i in range(self.dag.count):
             n = self.dag.nodes[i].contents
-            f = C.cast(n.op.gpu_forward, abi.ForwardKernel)
-            f(n.inputs, n.output, n.params)
-        L.check("dag forward")
+            calls.append((C.cast(n.op.gpu_forward, abi.ForwardKernel),
+                          C.cast(n.op.gpu_backward, abi.BackwardKernel), n.inputs, n.output, n.params))
+        return calls
+
+    def _bound(self):
+        if self._run is None or len(self._run) != self.dag.count:
+            self._run = self._calls()
+        return self._run
+
+    def forward(self) -> None:
+        """dag_forward (graph.c:57-60): each node's GPU forward slot in order."""
+        for f, _, inputs, output, p in self._bound():
+            f(inputs, output, p)
+        L = lib()
+        if L.error_count():
+            L.raise_error("dag forward")
 
     def backward(self) -> None:
         """dag_backward (graph.c:62-65): GPU backward slots in reverse order."""
+        for _, f, inputs, output, p in reversed(self._bound()):
+            f(inputs, output, p)
         L = lib()
-        for i in range(self.dag.count - 1, -1, -1):
-            n = self.dag.nodes[i].contents
-            f = C.cast(n.op.gpu_backward, abi.BackwardKernel)
-            f(n.inputs, n.output, n.params)
-        L.check("dag backward")
+        if L.error_count():
+            L.raise_error("dag backward")

@@ -42,11 +42,17 @@ class Library:
         # (kind, op name) -> bound entry point, looked up once: the per-call path does no
         # attribute lookups or string formatting
         self.entry = {}
+        # the same entry points taking addresses: an array of c_void_p and a byref cost half of the
+        # pointer objects a call otherwise makes (2.7 -> 1.4 us for two inputs and an output)
+        self.by_address = {}
         for name in OP_NAMES:
             for kind in ("forward", "backward"):
                 f = getattr(L, f"{name}_hip_{kind}")
                 f.argtypes, f.restype = [TensorPP, TensorP, KernelParams], None
                 self.entry[kind, name] = f
+                f = L[f"{name}_hip_{kind}"]  # a function object of its own
+                f.argtypes, f.restype = [C.c_void_p, C.c_void_p, KernelParams], None
+                self.by_address[kind, name] = f
         sig = {
             "plast_hip_init": ([C.c_int], C.c_int),
             "plast_hip_set_sync": ([C.c_int], None),
@@ -262,33 +268,41 @@ class DeviceTensor:
             pass
 
 
-_PTR_ARRAY = [TensorP * n for n in range(17)]
+_ADDR_ARRAY = [C.c_void_p * n for n in range(17)]
+_NO_PARAMS = KernelParams(0, 0, 0.0)
 
 
-def _ptr(x) -> TensorP:
-    return x.p if isinstance(x, DeviceTensor) else C.pointer(x)
+def _struct(x) -> Tensor:
+    """The Tensor struct of a DeviceTensor, or the struct itself; nothing else is a tensor."""
+    if isinstance(x, DeviceTensor):
+        return x.t
+    if isinstance(x, Tensor):
+        return x
+    raise TypeError(f"expected a DeviceTensor or a Tensor struct, got {type(x).__name__}")
 
 
 def _call(kind: str, name: str, inputs, output, p: KernelParams):
     L = lib()
     n = len(inputs)
-    arr = (_PTR_ARRAY[n] if n < len(_PTR_ARRAY) else TensorP * n)(*map(_ptr, inputs))
-    fn = L.entry.get((kind, name))
+    # the structs stay referenced by `inputs` for the call's duration
+    arr = (_ADDR_ARRAY[n] if n < len(_ADDR_ARRAY) else C.c_void_p * n)(
+        *[C.addressof(_struct(x)) for x in inputs])
+    fn = L.by_address.get((kind, name))
     if fn is None:
         raise PlastHipError(f"no entry point {name}_hip_{kind}")
-    fn(arr, _ptr(output), p)
+    fn(arr, C.byref(_struct(output)), p)
     if L.error_count():
         L.raise_error(f"{name}_hip_{kind}")
 
 
 def forward(name: str, inputs, output, p: KernelParams | None = None) -> None:
     """Call `<name>_hip_forward(inputs, output, params)`."""
-    _call("forward", name, inputs, output, p or KernelParams(0, 0, 0.0))
+    _call("forward", name, inputs, output, p or _NO_PARAMS)
 
 
 def backward(name: str, inputs, output, p: KernelParams | None = None) -> None:
     """Call `<name>_hip_backward(inputs, output, params)`."""
-    _call("backward", name, inputs, output, p or KernelParams(0, 0, 0.0))
+    _call("backward", name, inputs, output, p or _NO_PARAMS)
 
 
 def synchronize() -> None:
