@@ -110,6 +110,58 @@ void grad_into(const Tensor *x, const Tensor *out, const Tensor *a, const Tensor
   }
 }
 
+// Both gradients of a binary op over contiguous operands of one shape in one pass: g and the operands
+// are read once (28 bytes an element for mul where two launches moved 32, 20 for add and 24), and a
+// small op is one launch. Each element's operations are those of the two launches. One float4 unit
+// a lane in XCD order, as the vector kernel streams. leaky_relu(a * b + c) and its gradients node by
+// node, eight launches to six: [4096, 4096] 300 -> 275 us, [93, 24] 37 -> 29.
+template <Bin OP>
+__global__ __launch_bounds__(PLAST_EW_BLOCK) void bin_grad_pair_kernel(const float *g, const float *a,
+                                                                       const float *b, float *da,
+                                                                       float *db, uint64_t n,
+                                                                       uint64_t simd_end) {
+  constexpr bool kA = kGradUsesA<OP, false> || kGradUsesA<OP, true>;
+  constexpr bool kB = kGradUsesB<OP, false> || kGradUsesB<OP, true>;
+  const uint64_t e = (uint64_t(xcd_block(blockIdx.x, gridDim.x)) * PLAST_EW_BLOCK + threadIdx.x) * 4;
+  if (e >= n) return;
+  const uint32_t m = n - e < 4 ? uint32_t(n - e) : 4u;
+  const f4 gv = load_part<false>(g + e, m);
+  f4 av = f4(0.0f), bv = f4(0.0f);
+  if constexpr (kA) av = load_part<false>(a + e, m);
+  if constexpr (kB) bv = load_part<false>(b + e, m);
+  f4 dav = load_part<false>(da + e, m), dbv = load_part<false>(db + e, m);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const bool simd = e + c < simd_end;
+    dav[c] = dav[c] + grad_a<OP>(gv[c], av[c], bv[c]);
+    dbv[c] = dbv[c] + grad_b<OP>(gv[c], av[c], bv[c], simd);
+  }
+  store_part<false>(dav, da + e, m);
+  store_part<false>(dbv, db + e, m);
+}
+
+// Launches it where it applies: every operand, gradient and the output's gradient contiguous fp32 of
+// one shape, and neither gradient's buffer shared with anything else the op touches (x * x has one
+// gradient for both operands); false (launching nothing) otherwise.
+template <Bin OP>
+bool grad_pair(const Tensor *a, const Tensor *b, const Tensor *g, uint64_t simd) {
+  const Tensor *t[5] = {a->grad, b->grad, g, a, b};
+  for (const Tensor *x : t)
+    if (!same_shape(x, g) || !contiguous(x)) return false;
+  const uint64_t n = numel(g), blocks = ((n + 3) / 4 + PLAST_EW_BLOCK - 1) / PLAST_EW_BLOCK;
+  if (n == 0 || blocks > max_blocks(PLAST_EW_BLOCK)) return false;
+  for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < 5; ++j) {
+      const float *p = static_cast<const float *>(t[i]->data), *q = static_cast<const float *>(t[j]->data);
+      if (i != j && p < q + n && q < p + n) return false;
+    }
+  bin_grad_pair_kernel<OP><<<unsigned(blocks), PLAST_EW_BLOCK, 0, stream()>>>(
+      static_cast<const float *>(g->data), static_cast<const float *>(a->data),
+      static_cast<const float *>(b->data), static_cast<float *>(a->grad->data),
+      static_cast<float *>(b->grad->data), n, simd);
+  return true;
+}
+
 template <Bin OP>
 void binary_backward(Tensor **in, const Tensor *out, const char *where) {
   if (!ensure_init()) return;
@@ -124,8 +176,13 @@ void binary_backward(Tensor **in, const Tensor *out, const char *where) {
   // The reference's contiguous same-shape path (kernel_macros.h:306-311) rounds the B-gradient of
   // sub/div from 0 - g inside its SIMD blocks.
   const bool ref_contig = contiguous(a) && contiguous(b) && contiguous(out) && same_shape(a, b);
+  const uint64_t simd = ref_contig ? simd_end(n) : 0;
+  if (da && db && grad_pair<OP>(a, b, out->grad, simd)) {
+    finish(where);
+    return;
+  }
   if (da) grad_into<OP, false>(a, out, a, b, 0, where);
-  if (db) grad_into<OP, true>(b, out, a, b, ref_contig ? simd_end(n) : 0, where);
+  if (db) grad_into<OP, true>(b, out, a, b, simd, where);
   finish(where);
 }
 
