@@ -89,6 +89,11 @@ constexpr int kBlock = 256;  // threads per workgroup for streaming kernels (4 w
 // 1536 and fewer leave CUs idle.
 #define PLAST_ROW_WAVES 2048
 #endif
+// The same where several axes are reduced, whose runs are shorter and decoded one by one: config 3's
+// B gradient (512 outputs, 268 MB) 54.6 us with 2048 segments, 45.0 with 4096, 45.7 with 8192.
+#ifndef PLAST_MULTI_WAVES
+#define PLAST_MULTI_WAVES 4096
+#endif
 // Rows in flight per lane, leading-axis reductions, for one-, two- and three-operand producers.
 // Measured (two alternating runs): one operand with 2 rather than 4 rows, the axis-0 sum of
 // [4096, 65536] 6.60-6.64 -> 6.72-6.74 TB/s, config 5's bias gradient 6.24-6.26 -> 6.41-6.42, the

@@ -81,6 +81,7 @@ struct ScalarBody {
   static constexpr bool kTape = false;             // selects the vectorised launch shape
   static constexpr bool kTileFixed3 = false;       // fixed-role tile kernels for 3 operands
   static constexpr int kTileRows = 1;              // tile rows per evaluation
+  static constexpr uint32_t kStreamed = 0;         // bit k: operand k is read once by any launch
   // host: whether no element's value depends on its linear index (the NEG rule), so that the axes
   // may be walked in another order
   bool index_free() const { return true; }
@@ -164,6 +165,10 @@ __device__ __forceinline__ float bin_grad_term(const float *v, bool simd) {
 template <Bin OP, bool B>
 struct BinGradBody : ScalarBody<BinGradBody<OP, B>> {
   static constexpr int NIN = 2 + int(kGradUsesA<OP, B>) + int(kGradUsesB<OP, B>);
+  // d and g cover the space: where an operand is broadcast they keep nontemporal loads (mul's gradient
+  // of the unbroadcast operand, 67M elements: 158 us with every load ordinary, 128 so; with ordinary
+  // stores 138)
+  static constexpr uint32_t kStreamed = 3;
   uint64_t simd_end;
   bool index_free() const { return simd_end == 0; }
   __device__ __forceinline__ float eval(const float *v, uint64_t i) const {
@@ -237,6 +242,7 @@ template <int N, uint32_t OPS>
 struct TapeBody {
   static constexpr int NIN = N;
   static constexpr bool kTape = true;
+  static constexpr uint32_t kStreamed = 0;
   static constexpr bool kTileFixed3 = true;
   static constexpr int kTileRows = PLAST_TAPE_TILE_ROWS;
   static constexpr bool kExp = (OPS & kTapeExp) != 0;

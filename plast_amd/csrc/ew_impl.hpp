@@ -67,6 +67,13 @@ __device__ __forceinline__ f4 load4(const EwArgs<NIN> &A, int k, int64_t off) {
   return load_operand<REUSE>(A.in[k] + off);
 }
 
+// Whether a launch that re-reads some operand re-reads operand k (always-streamed operands of a body
+// keep their nontemporal loads there).
+template <class Body>
+__device__ __forceinline__ constexpr bool reread(int k) {
+  return (Body::kStreamed >> k & 1u) == 0;
+}
+
 // Vectorised kernel: innermost axis has stride 1 (output, streamed inputs) or 0 (broadcast
 // inputs) and a multiple-of-4 extent; the other ORANK axes (ORANK < 0: runtime count) are decoded
 // from the unit index with magic division. A workgroup owns kEwBlock * kEwUnroll consecutive units,
@@ -124,7 +131,8 @@ __global__ __launch_bounds__((VecLaunch<Body, REUSE>::block)) void ew_vec_kernel
       }
     }
 #pragma unroll
-    for (int k = 0; k < NIN; ++k) x[u][k] = load4<REUSE>(A, k, off[k]);
+    for (int k = 0; k < NIN; ++k)
+      x[u][k] = REUSE && reread<Body>(k) ? load4<true>(A, k, off[k]) : load4<false>(A, k, off[k]);
     oo[u] = ooff;
   }
   uint64_t idx[kEwUnroll];

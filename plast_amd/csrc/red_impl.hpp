@@ -1382,7 +1382,7 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       const uint64_t span = multi && vec ? A.vlen : A.len;  // what segments divide
       // enough waves to cover the machine: split long rows when there are few of them
       uint32_t segs = 1;
-      const uint64_t want_waves = PLAST_ROW_WAVES;
+      const uint64_t want_waves = multi ? PLAST_MULTI_WAVES : PLAST_ROW_WAVES;
       if (A.rows < want_waves && span >= 8192) {
         uint64_t sg = (want_waves + A.rows - 1) / A.rows;
         const uint64_t max_sg = span / 4096;
