@@ -19,8 +19,18 @@ class Graph:
     def __init__(self):
         self.nodes: list[abi.Node] = []
         self._keep = []       # ctypes objects the C side points into
-        self._arena_bufs = []
-        self._alloc_cb = abi.ArenaAllocFn(self._alloc)
+        self._arena_bufs = bufs = []
+
+        # the fusion pass allocates its nodes and tapes through this callback; it refers to the list
+        # alone, so that a dropped graph (and the tensors it keeps) goes at once and not at the next
+        # garbage collection
+        def alloc(arena, size, align):
+            buf = C.create_string_buffer(int(size) + int(align))
+            bufs.append(buf)
+            addr = C.addressof(buf)
+            return (addr + align - 1) // align * align
+
+        self._alloc_cb = abi.ArenaAllocFn(alloc)
         self.dag = None
         self._run = None      # the DAG's calls, bound by build()
 
@@ -43,13 +53,6 @@ class Graph:
         self.nodes.append(n)
         output.t.creator = C.addressof(n)
         return output
-
-    # --- the fusion pass allocates its nodes and tapes through this callback
-    def _alloc(self, arena, size, align):
-        buf = C.create_string_buffer(int(size) + int(align))
-        self._arena_bufs.append(buf)
-        addr = C.addressof(buf)
-        return (addr + align - 1) // align * align
 
     def build(self, root: DeviceTensor, fuse: bool = False) -> int:
         """Topologically order the nodes reachable from root's creator (graph.c:30-39); with
