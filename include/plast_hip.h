@@ -200,10 +200,11 @@ void relu_grad_modulate_bias_grad_hip(const float *dout, const float *out_data, 
  * the gradient of a bias broadcast-added to the logits (the reference's ADD backward into a [C]
  * operand, kernel_macros.h:283-299). dloss [N] is the upstream gradient of each row's loss (1/N
  * for a mean), known before the step. Each logit is read once and each gradient written once
- * (16-byte aligned rows of whole float4 up to 32768 floats; other rows run the three passes).
- * stats, loss and dlogits are the same bits on every call; dbias, a sum over rows, is split over
- * the GPU's workgroups by the rows each one took, which varies from call to call (its last bits
- * may too) unless plast_hip_set_deterministic(1) fixes the split. No counterpart in the
+ * (rows up to 32768 floats; longer rows run the three passes). stats, loss and dlogits are the same
+ * bits on every call; dbias, a sum over rows, is too for rows up to 2048 floats and for rows that are
+ * no whole float4 or not 16-byte aligned. For others it is split over the GPU's workgroups by the
+ * rows each one took, which varies from call to call (its last bits may too) unless
+ * plast_hip_set_deterministic(1) fixes the split. No counterpart in the
  * reference, which runs the op chain of src/api/loss.c:97-169, its backward and the bias's ADD
  * backward as separate passes (its ADD backward accumulates the bias gradient with omp atomics,
  * kernel_macros.h:292-297, in no fixed order either); for callers that train with a

@@ -1286,6 +1286,10 @@ void launch_cols_finalize(const RedArgs<Prod::NIN> &A, const Prod &prod, uint64_
     red_cols_finalize<Prod, Comb><<<ceil_div(nout, kBlock), kBlock, 0, stream()>>>(A, prod);
 }
 
+// Whether slot 0 can hold `bytes` of partials now: a capture cannot grow it, and a launch that once
+// needed none there then runs unsplit instead of failing.
+inline bool partials_fit(uint64_t bytes) { return !capturing() || bytes <= plast_hip_workspace_bytes(0); }
+
 // Reduce over every axis where operand NIN (the target) has stride 0 and extent > 1.
 // `post` and `divisor` describe the epilogue; `out` is float* or int64_t* per Comb::Out.
 template <class Prod, class Comb>
@@ -1390,6 +1394,7 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
         if (sg > 65535) sg = 65535;
         segs = uint32_t(sg < 1 ? 1 : sg);
       }
+      if (multi && !partials_fit(sizeof(Part) * A.rows * segs)) segs = 1;
       uint64_t seglen = (span + segs - 1) / segs;
       seglen = (seglen + 255) / 256 * 256;
       segs = uint32_t((span + seglen - 1) / seglen);
@@ -1473,6 +1478,7 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       if (chunks > 65535) chunks = 65535;
       if (chunks < 1) chunks = 1;
     }
+    if (multi && !partials_fit(sizeof(Part) * nout * chunks)) chunks = 1;
     uint64_t seglen = (A.len + chunks - 1) / chunks;
     chunks = (A.len + seglen - 1) / seglen;
     A.segs = uint32_t(chunks);
@@ -1511,7 +1517,11 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       const uint64_t most = (PLAST_COL_BLOCKS + A.rows - 1) / A.rows, least = (256 + A.rows - 1) / A.rows;
       if (fc > most) fc = most;
       if (fc < least) fc = steps / 2 < least ? steps / 2 : least;
-      if (steps <= 8) fc = 1;
+      // one chunk needs no partials, as neither a short axis nor a small sum of whole float4 columns
+      // does in slices
+      const bool slices_fit = chunks == 1 || (std::is_same<Comb, SumComb>::value && in % 4 == 0 && vec &&
+                                              A.len * nout <= PLAST_COL_SMALL_MAX);
+      if (steps <= 8 || (slices_fit && !partials_fit(sizeof(Part) * nout * fc))) fc = 1;
       if (fc > 65535) fc = 65535;
       if (fc < 1) fc = 1;
       A.seglen = (steps + fc - 1) / fc * F.R;

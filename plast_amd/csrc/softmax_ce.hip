@@ -1138,7 +1138,6 @@ bool ce_step_lds_ok() {
   const int bytes = kStepBlock * V * int(sizeof(f4));
   for (const void *k : {reinterpret_cast<const void *>(&ce_step_kernel<V, true, false>),
                         reinterpret_cast<const void *>(&ce_step_kernel<V, false, false>),
-                        reinterpret_cast<const void *>(&ce_step_kernel<V, true, true>),
                         reinterpret_cast<const void *>(&ce_step_kernel<V, false, true>)})
     if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) {
       (void)hipGetLastError();  // not an error of the call: the caller takes the three passes
@@ -1176,11 +1175,11 @@ void ce_step_launch_v(int want, unsigned grid, float *part, const float *logits,
           <<<grid, kStepBlock, lds, stream()>>>(logits, labels, dloss, stats, loss, dlogits, part, N, C,
                                                 uint32_t(simd_end(N)));
     };
-    // the dynamic row order unless results must not depend on timing (plast_hip_set_deterministic)
-    const bool ragged = C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits);
-    if (deterministic() && ragged) run(std::false_type{}, std::true_type{});
+    // the dynamic row order unless results must not depend on timing (plast_hip_set_deterministic);
+    // rows that are no whole float4 always keep the static one, as their bias gradient has been the
+    // same bits on every call
+    if (C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits)) run(std::false_type{}, std::true_type{});
     else if (deterministic()) run(std::false_type{}, std::false_type{});
-    else if (ragged) run(std::true_type{}, std::true_type{});
     else run(std::true_type{}, std::false_type{});
   }
 }
@@ -1945,8 +1944,13 @@ void softmax_cross_entropy_step_hip(const float *logits, const int32_t *labels, 
     if (mean_loss) finish(where);
     return;
   }
-  const int V = ce_step_form(logits, labels, dloss, stats, loss, dlogits, N, C, where);
+  int V = ce_step_form(logits, labels, dloss, stats, loss, dlogits, N, C, where);
   if (V < 0) return;
+  // rows of no whole float4 while a capture holds too little workspace for their column sums, which
+  // the three passes do not need
+  if ((C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits)) && capturing() &&
+      sizeof(float) * ce_step_grid(N, C) * C > plast_hip_workspace_bytes(0))
+    V = 0;
   if (V == 0) {
     // any other row: the forward, the overwriting backward and the column sum as three passes
     Tensor tx, tl, ts, to, tg, tdx;
