@@ -1487,9 +1487,11 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
     A.divisor = divisor;
     if constexpr (std::is_same<Comb, SumComb>::value) {
       // small: one launch over narrow column slices instead of chunks plus a finalize, while a lane's
-      // share of the rows stays a few batches (narrow columns leave few workgroups)
+      // share of the rows stays a few batches (narrow columns leave few workgroups). Below 128 rows
+      // only where slices of 256 columns leave most of the chip idle: config 1's step at [32, 568]
+      // 10.8 us in slices, 6.4 so, at [60, 3000] 15.6 and 7.5, at [16, 4096] 6.9 and 6.3.
       const uint64_t few_rows = uint64_t(2) * kColSmallU<Prod> * (kBlock / kColSmallS4<Prod>);
-      if ((A.len >= 128 || (A.len >= 64 && base_blocks < 64)) && vec && !multi && A.len * nout <= PLAST_COL_SMALL_MAX &&
+      if ((A.len >= 128 || (A.len >= 16 && base_blocks < 64)) && vec && !multi && A.len * nout <= PLAST_COL_SMALL_MAX &&
           (!flat || A.len <= few_rows) && (NIN < 3 || PLAST_COL_SMALL3 != 0)) {
         const uint32_t sblocks = ceil_div(A.inner, uint64_t(4) * kColSmallS4<Prod>);
         const uint64_t sgrid = uint64_t(sblocks) * A.rows;

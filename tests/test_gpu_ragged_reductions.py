@@ -20,7 +20,7 @@ ROWS = [(1, 1), (5, 2), (7, 3), (64, 5), (33, 31), (70, 32), (9, 33), (65, 77), 
 # (outer, len, inner): narrow columns, then wide ones
 COLS = [(1, 1, 3), (1, 700, 1), (3, 40, 2), (1, 5000, 3), (1, 60000, 10), (2, 300, 77), (1, 9000, 77),
         (1, 64, 129), (1, 3000, 171), (1, 40, 255), (1, 6000, 254), (2, 100, 256), (1, 90, 257),
-        (1, 1000, 261), (2, 30, 1027), (1, 5000, 515)]
+        (1, 1000, 261), (2, 30, 1027), (1, 5000, 515), (1, 17, 300), (2, 63, 1003)]
 
 
 def _cases():
