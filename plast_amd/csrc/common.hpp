@@ -9,6 +9,7 @@
 #include <cstring>
 
 #include "../../include/plast_hip.h"
+#include "launch_rules.hpp"
 
 namespace plast {
 
@@ -301,10 +302,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 // The same at any float's address: one 16-byte access of a lane, which gfx950 takes at 4-byte
 // alignment (a wave still covers one contiguous 1 KiB, at most one line more).
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-
-// The dispatch packet's grid size is 32-bit: a launch holds fewer than 2^32 work-items per
-// dimension, i.e. at most max_blocks(threads) workgroups of `threads` lanes along x.
-constexpr uint64_t max_blocks(uint64_t threads) { return (uint64_t(1) << 32) / threads - 1; }
 
 // Workgroups are dispatched round-robin over the 8 XCDs. xcd_block renumbers the first
 // 8 * (grid / 8) of them (a permutation) so that XCD x owns the x-th contiguous range of workgroup

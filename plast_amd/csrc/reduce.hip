@@ -208,14 +208,15 @@ __global__ __launch_bounds__(T > 64 ? T : kBlock) void ext_bwd_rows_kernel(RedAr
 }
 
 // Launches ext_bwd_rows_kernel when a and its gradient are unit-stride along the reduced axis `dim`,
-// the last one, and the rows fill the chip or are short; false (launching nothing) otherwise. `ost`:
-// the output's strides over a's axes.
+// the last one, and ext_row_threads takes the rows; false (launching nothing) otherwise. `ost`: the
+// output's strides over a's axes.
 bool ext_backward_rows(const Tensor *a, const Tensor *out, uint64_t dim, const int64_t *ost) {
   const uint64_t n = numel(a), len = a->shape[dim];
   if (dim + 1 != a->ndim || n == 0 || n >= (uint64_t(1) << 32)) return false;
   if (len > 1 && (a->strides[dim] != 1 || a->grad->strides[dim] != 1)) return false;
   const uint64_t rows = n / len;
-  if (len > 32768 && rows < 256) return false;
+  const uint32_t threads = ext_row_threads(rows, len);
+  if (!threads) return false;
   Space s;
   s.rank = int(a->ndim);
   s.nops = 4;
@@ -240,9 +241,8 @@ bool ext_backward_rows(const Tensor *a, const Tensor *out, uint64_t dim, const i
     for (int k = 0; k < 4; ++k) A.ost[k][d] = s.st[k][d];
   }
   A.nouter = s.rank;
-  // threads per row: about four float4 units each
-  if (len <= 128) ext_bwd_rows_kernel<8><<<ceil_div(rows, kBlock / 8), kBlock, 0, stream()>>>(A);
-  else if (len <= 2048) ext_bwd_rows_kernel<64><<<ceil_div(rows, kBlock / 64), kBlock, 0, stream()>>>(A);
+  if (threads == 8) ext_bwd_rows_kernel<8><<<ceil_div(rows, kBlock / 8), kBlock, 0, stream()>>>(A);
+  else if (threads == 64) ext_bwd_rows_kernel<64><<<ceil_div(rows, kBlock / 64), kBlock, 0, stream()>>>(A);
   else ext_bwd_rows_kernel<kExtBlock><<<unsigned(rows), kExtBlock, 0, stream()>>>(A);
   return true;
 }

@@ -138,3 +138,29 @@ def test_sgd_tensor_split_over_launch_entries():
     idx = [0, piece - 1, piece, 2 * piece - 1, 2 * piece, n - 1]
     assert (_read(p.ptr, idx) == 0.5).all()
     p.free()
+
+
+def test_max_backward_rows_beyond_one_launch():
+    """max's backward over 2^29 rows of 4: eight threads a row would be 2^32 work-items, so the two
+    passes run. The rows around the ends and the middle against numpy."""
+    from plast_amd.abi import KernelParams
+    rt = _rt()
+    L = rt.lib()
+    rows, cols = 1 << 29, 4
+    _need(4 * (2 * rows * cols + 4 * rows))
+    print(f"max backward {rows}x{cols}", flush=True)
+    a = rt.DeviceTensor((rows, cols), requires_grad=True, zero=False)
+    o = rt.DeviceTensor((rows,), requires_grad=True, zero=False)
+    a.fill_("uniform", 5, -1.0, 1.0)
+    L.ones_hip(C.byref(a.grad.t), rows * cols)
+    L.ones_hip(C.byref(o.grad.t), rows)
+    p = KernelParams(1, 0, 0.0)
+    rt.forward("max", [a], o, p)
+    rt.backward("max", [a], o, p)
+    r = np.array([0, 1, 2, rows // 2 - 1, rows // 2, rows - 2, rows - 1])
+    idx = (r[:, None] * cols + np.arange(cols)).ravel()
+    x, g = _read(a.ptr, idx).reshape(-1, cols), _read(a.grad.ptr, idx).reshape(-1, cols)
+    tie = x == x.max(1, keepdims=True)
+    assert np.array_equal(g, 1.0 + tie / tie.sum(1, keepdims=True, dtype=np.float32))
+    a.free()
+    o.free()
