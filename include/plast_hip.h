@@ -225,7 +225,8 @@ void softmax_cross_entropy_step_hip(const float *logits, const i32 *labels, cons
  * 32768, logits and dlogits 16-byte aligned, N below 2^31; anything else is reported as an error
  * (the three-pass form allocates). The results are softmax_cross_entropy_step_hip's (the same
  * kernels over the same grid; bit-identical in deterministic mode). Calls that overlap on one GPU
- * (other streams, other threads) share the array and race. No counterpart in the reference. */
+ * (other streams, other threads) share the array and race; so do replays, on a stream of the
+ * caller's, of a graph captured before the workspace its partial sums need (plast_hip_capture_begin). No counterpart in the reference. */
 void softmax_cross_entropy_step_noalloc_hip(const float *logits, const i32 *labels,
                                             const float *dloss, float *stats, float *loss,
                                             float *dlogits, float *dbias, float *mean_loss, u64 N,
@@ -344,8 +345,10 @@ int plast_hip_synchronize(void);
  * instantiated graph (a hipGraphExec_t) that plast_hip_graph_launch() replays with the same
  * pointers and shapes, reading whatever the buffers hold at replay time; plast_hip_graph_destroy()
  * frees it. Only device work can be captured: run each op once before capturing so that the
- * library's workspaces are already sized (a capture that would grow one fails with an error), and
- * keep host transfers and allocation outside. The library records fills as kernels, never as
+ * library's workspaces are already sized (a capture that would grow one fails with an error, but
+ * for sums over several axes, sums and extremes of narrow columns and the cross-entropy step of
+ * rows that are no whole float4, whose partial sums then lie in the library's fixed device array:
+ * the bits are the same either way), and keep host transfers and allocation outside. The library records fills as kernels, never as
  * memset nodes. A workspace that eager work outgrows while a graph is alive is kept (retired)
  * until the last graph the library made is destroyed, so a replay never reaches freed memory.
  * Returns 0 / a non-null graph on success. No counterpart in the reference, which launches and

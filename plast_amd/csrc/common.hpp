@@ -343,6 +343,16 @@ bool ensure_init();
 // the reduction engine's partial summaries; slot 1 an op's own temporaries (tie counts, extremes);
 // slot 2 the staging buffer of host transfers of strided tensors.
 void *workspace(size_t bytes, int slot = 0);
+// A fixed device array of kScratchFloats floats (32 MiB: the column sums of 256 workgroups over rows
+// of up to 32768 floats), each GPU's own until the process ends: its address on the library's device
+// (null, after reporting, when the lookup fails).
+constexpr uint64_t kScratchFloats = uint64_t(1) << 23;
+float *fixed_scratch(const char *where);
+// At least `bytes` for the partials of a launch that needs none in its unsplit form: slot 0's, or,
+// while a capture that cannot grow the slot is open, the fixed array (the library's launches are
+// ordered on its stream, so they never overlap in it). The launch is then split the same way,
+// and gives the same bits, whatever ran before the capture.
+void *partials(size_t bytes, const char *where);
 
 #define PLAST_HIP_TRY(where, expr)                                                                 \
   do {                                                                                             \

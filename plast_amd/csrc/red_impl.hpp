@@ -1286,10 +1286,6 @@ void launch_cols_finalize(const RedArgs<Prod::NIN> &A, const Prod &prod, uint64_
     red_cols_finalize<Prod, Comb><<<ceil_div(nout, kBlock), kBlock, 0, stream()>>>(A, prod);
 }
 
-// Whether slot 0 can hold `bytes` of partials now: a capture cannot grow it, and a launch that once
-// needed none there then runs unsplit instead of failing.
-inline bool partials_fit(uint64_t bytes) { return !capturing() || bytes <= plast_hip_workspace_bytes(0); }
-
 // Reduce over every axis where operand NIN (the target) has stride 0 and extent > 1.
 // `post` and `divisor` describe the epilogue; `out` is float* or int64_t* per Comb::Out.
 template <class Prod, class Comb>
@@ -1394,7 +1390,6 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
         if (sg > 65535) sg = 65535;
         segs = uint32_t(sg < 1 ? 1 : sg);
       }
-      if (multi && !partials_fit(sizeof(Part) * A.rows * segs)) segs = 1;
       uint64_t seglen = (span + segs - 1) / segs;
       seglen = (seglen + 255) / 256 * 256;
       segs = uint32_t((span + seglen - 1) / seglen);
@@ -1403,7 +1398,8 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       A.post = int(post);
       A.divisor = divisor;
       if (segs > 1) {
-        A.part = workspace(sizeof(Part) * A.rows * segs);
+        A.part = multi ? partials(sizeof(Part) * A.rows * segs, where)
+                       : workspace(sizeof(Part) * A.rows * segs);
         if (!A.part) return false;
       }
       // short rows: 2, 8 or 32 lanes each. [50000, 77] a wave per row / 8 lanes: see the kernel.
@@ -1478,7 +1474,6 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       if (chunks > 65535) chunks = 65535;
       if (chunks < 1) chunks = 1;
     }
-    if (multi && !partials_fit(sizeof(Part) * nout * chunks)) chunks = 1;
     uint64_t seglen = (A.len + chunks - 1) / chunks;
     chunks = (A.len + seglen - 1) / seglen;
     A.segs = uint32_t(chunks);
@@ -1523,14 +1518,15 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       // does in slices
       const bool slices_fit = chunks == 1 || (std::is_same<Comb, SumComb>::value && in % 4 == 0 && vec &&
                                               A.len * nout <= PLAST_COL_SMALL_MAX);
-      if (steps <= 8 || (slices_fit && !partials_fit(sizeof(Part) * nout * fc))) fc = 1;
+      if (steps <= 8) fc = 1;
       if (fc > 65535) fc = 65535;
       if (fc < 1) fc = 1;
       A.seglen = (steps + fc - 1) / fc * F.R;
       chunks = (A.len + A.seglen - 1) / A.seglen;
       A.segs = uint32_t(chunks);
       if (chunks > 1) {
-        A.part = workspace(sizeof(Part) * nout * chunks);
+        A.part = slices_fit ? partials(sizeof(Part) * nout * chunks, where)
+                            : workspace(sizeof(Part) * nout * chunks);
         if (!A.part) return false;
       }
       const dim3 grid{unsigned(A.rows), unsigned(chunks), 1u};
@@ -1540,7 +1536,8 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
     }
     if (base_blocks <= max_blocks(kBlock)) {
       if (chunks > 1) {
-        A.part = workspace(sizeof(Part) * nout * chunks);
+        A.part = multi ? partials(sizeof(Part) * nout * chunks, where)
+                       : workspace(sizeof(Part) * nout * chunks);
         if (!A.part) return false;
       }
       const dim3 grid{unsigned(base_blocks), unsigned(chunks), 1u};

@@ -1,11 +1,16 @@
 // runtime.hip — library state (device, stream, errors, workspace), the arena / fill hooks of the
 // reference's L0/L1 layer, timing marks, deterministic input generation and the copy ceiling.
+#include <atomic>
 #include <cstdarg>
 #include <cstdlib>
 #include <vector>
 
 #include "common.hpp"
 #include "ws_ledger.hpp"
+
+// The fixed device array (fixed_scratch). Host code never passes this name to a kernel (it is a
+// host-side stand-in there): its device address is looked up once per device.
+static __device__ __align__(256) float scratch[uint64_t(1) << 23];
 
 namespace plast {
 
@@ -110,6 +115,38 @@ void *workspace(size_t bytes, int slot) {
         return p;
       },
       release_workspace);
+}
+
+static_assert(sizeof(scratch) == kScratchFloats * sizeof(float), "scratch size");
+
+// Looked up with hipGetSymbolAddress, with the library's device current, on the first call there.
+float *fixed_scratch(const char *where) {
+  static std::atomic<float *> addr[64] = {};
+  const int dev = library_device();
+  if (dev < 0 || dev >= 64) {
+    report_error(where, "device %d is out of range", dev);
+    return nullptr;
+  }
+  float *a = addr[dev].load(std::memory_order_acquire);
+  if (a) return a;
+  int cur = -1;
+  hipError_t e = hipGetDevice(&cur);
+  if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
+  void *p = nullptr;
+  if (e == hipSuccess) e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
+  if (cur >= 0 && cur != dev) (void)hipSetDevice(cur);
+  if (e != hipSuccess || !p) {
+    report_error(where, "hipGetSymbolAddress(scratch) on device %d: %s", dev, hipGetErrorString(e));
+    return nullptr;
+  }
+  a = static_cast<float *>(p);
+  addr[dev].store(a, std::memory_order_release);
+  return a;
+}
+
+void *partials(size_t bytes, const char *where) {
+  const bool fixed = g_capturing && bytes > g_ws.bytes(0) && bytes <= kScratchFloats * sizeof(float);
+  return fixed ? static_cast<void *>(fixed_scratch(where)) : workspace(bytes);
 }
 
 // ------------------------------------------------------------------------- metadata helpers

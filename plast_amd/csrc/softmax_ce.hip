@@ -17,45 +17,8 @@
 
 #include "common.hpp"
 
-// Device scratch of the allocation-free one-pass step (softmax_cross_entropy_step_noalloc_hip):
-// the workgroups' column sums, kScratchFloats floats (32 MiB: 256 workgroups of rows up to 32768
-// floats, the widest one-pass row of 1024-lane workgroups; wider ones, of a build with narrower
-// workgroups, run on fewer workgroups). Each GPU the library runs on holds its own copy until the
-// process ends. Host code never passes this name to a kernel (it
-// is a host-side stand-in there): noalloc_scratch() looks the device address up once per device.
-static __device__ __align__(256) float scratch[uint64_t(1) << 23];
-
 namespace plast {
 namespace {
-
-constexpr uint64_t kScratchFloats = uint64_t(1) << 23;
-static_assert(sizeof(scratch) == kScratchFloats * sizeof(float), "scratch size");
-
-// The device address of `scratch` on the library's device, found with hipGetSymbolAddress, with
-// that device current, on the first call there (null, after reporting, when the lookup fails).
-float *noalloc_scratch(const char *where) {
-  static std::atomic<float *> addr[64] = {};
-  const int dev = library_device();
-  if (dev < 0 || dev >= 64) {
-    report_error(where, "device %d is out of range", dev);
-    return nullptr;
-  }
-  float *a = addr[dev].load(std::memory_order_acquire);
-  if (a) return a;
-  int cur = -1;
-  hipError_t e = hipGetDevice(&cur);
-  if (e == hipSuccess && cur != dev) e = hipSetDevice(dev);
-  void *p = nullptr;
-  if (e == hipSuccess) e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
-  if (cur >= 0 && cur != dev) (void)hipSetDevice(cur);
-  if (e != hipSuccess || !p) {
-    report_error(where, "hipGetSymbolAddress(scratch) on device %d: %s", dev, hipGetErrorString(e));
-    return nullptr;
-  }
-  a = static_cast<float *>(p);
-  addr[dev].store(a, std::memory_order_release);
-  return a;
-}
 
 constexpr int kCeBlock = 256;
 constexpr int kCeWaves = kCeBlock / 64;
@@ -1944,13 +1907,8 @@ void softmax_cross_entropy_step_hip(const float *logits, const int32_t *labels, 
     if (mean_loss) finish(where);
     return;
   }
-  int V = ce_step_form(logits, labels, dloss, stats, loss, dlogits, N, C, where);
+  const int V = ce_step_form(logits, labels, dloss, stats, loss, dlogits, N, C, where);
   if (V < 0) return;
-  // rows of no whole float4 while a capture holds too little workspace for their column sums, which
-  // the three passes do not need
-  if ((C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits)) && capturing() &&
-      sizeof(float) * ce_step_grid(N, C) * C > plast_hip_workspace_bytes(0))
-    V = 0;
   if (V == 0) {
     // any other row: the forward, the overwriting backward and the column sum as three passes
     Tensor tx, tl, ts, to, tg, tdx;
@@ -1985,7 +1943,10 @@ void softmax_cross_entropy_step_hip(const float *logits, const int32_t *labels, 
   }
   const uint64_t grid = ce_step_grid(N, C);
   // the workgroups' column sums (written even when no bias gradient is wanted; then unread)
-  float *part = static_cast<float *>(workspace(sizeof(float) * grid * C));
+  const bool whole = C % 4 == 0 && aligned16(logits) && aligned16(dlogits);
+  // (rows that are no whole float4 were three passes once, which a capture took without workspace)
+  float *part = static_cast<float *>(whole ? workspace(sizeof(float) * grid * C)
+                                           : partials(sizeof(float) * grid * C, where));
   if (!part) return;
   ce_step_launch(V, unsigned(grid), part, logits, labels, dloss, stats, loss, dlogits, dbias,
                  mean_loss, N, C);
@@ -2011,7 +1972,7 @@ void softmax_cross_entropy_step_noalloc_hip(const float *logits, const int32_t *
                  (unsigned long long)C, (unsigned long long)kStepMaxC);
     return;
   }
-  float *part = noalloc_scratch(where);
+  float *part = fixed_scratch(where);
   if (!part) return;
   const uint64_t grid = ce_step_grid(N, C);
   ce_step_launch(V, unsigned(grid), part, logits, labels, dloss, stats, loss, dlogits, dbias,

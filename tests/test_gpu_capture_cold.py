@@ -1,6 +1,6 @@
 """Calls recorded into a graph by a library whose workspace is still empty: the launches that split
-their work over partials elsewhere run unsplit there, and give the eager call's results. The library
-is a copy of the build with a state of its own."""
+their work over partials keep the split there, and give the eager call's results bit for bit. The
+library is a copy of the build with a state of its own."""
 from __future__ import annotations
 
 import shutil
@@ -25,18 +25,38 @@ def cold(tmp_path):
 
 
 def _replayed(L, call, outs):
-    """The outputs after two replays of the captured call, with eager work between."""
-    assert L.plast_hip_capture_begin() == 0
-    call()
-    g = L.plast_hip_capture_end()
-    L.check("capture")
-    for _ in range(2):
+    """The outputs of the captured call, the same bits from two replays, from the eager call and from
+    a second capture, with the workspace that the eager call left."""
+    def clear():
         for t in outs:
             L.zeros_hip(t.p, int(np.prod(t.shape)))
+
+    def capture():
+        assert L.plast_hip_capture_begin() == 0
+        call()
+        g = L.plast_hip_capture_end()
+        L.check("capture")
+        return g
+
+    def replay(g):
+        clear()
         assert L.plast_hip_graph_launch(g) == 0
-        got = [t.numpy() for t in outs]
-    L.plast_hip_graph_destroy(g)
-    return got
+        return [t.numpy() for t in outs]
+
+    g = capture()
+    assert L.plast_hip_workspace_bytes(0) == 0
+    got = [replay(g), replay(g)]
+    clear()
+    call()
+    got.append([t.numpy() for t in outs])
+    warm = capture()
+    got += [replay(warm), replay(g)]
+    for h in (g, warm):
+        L.plast_hip_graph_destroy(h)
+    for other in got[1:]:
+        for a, b in zip(got[0], other):
+            assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    return got[0]
 
 
 @pytest.mark.parametrize("shape, small", [((300, 2, 1028), (1, 2, 1)), ((200, 2, 100, 12), (1, 2, 1, 12)),
@@ -79,8 +99,9 @@ def test_step_of_ragged_rows(cold):
     g = np.full(N, np.float32(1 / N), np.float32)
     X, Y, G = (rt.DeviceTensor.from_numpy(v) for v in (x, lab, g))
     st, loss, dx = rt.DeviceTensor((N, 2)), rt.DeviceTensor((N,)), rt.DeviceTensor((N, C))
+    db, mean = rt.DeviceTensor((C,)), rt.DeviceTensor((1,))
     got = _replayed(cold, lambda: cold.softmax_cross_entropy_step_hip(
-        X.ptr, Y.ptr, G.ptr, st.ptr, loss.ptr, dx.ptr, None, None, N, C), [loss, dx])
+        X.ptr, Y.ptr, G.ptr, st.ptr, loss.ptr, dx.ptr, db.ptr, mean.ptr, N, C), [loss, dx, st, db, mean])
     x64 = x.astype(np.float64)
     m = x64.max(1, keepdims=True)
     lse = np.log(np.exp(x64 - m).sum(1))
