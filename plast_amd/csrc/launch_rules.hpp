@@ -21,4 +21,110 @@ inline uint32_t ext_row_threads(uint64_t rows, uint64_t len) {
   return blocks <= max_blocks(t > 64 ? kLongBlock : kRowsBlock) ? t : 0;
 }
 
+// ------------------------------------------------------------------------- leading-axis reductions
+// A reduction of [rows, len, inner] over len, the `inner` columns kept.
+
+inline uint64_t div_up(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
+
+// Row chunks of the column kernel with lanes of `width` columns: slices of 64 lanes, and the reduced
+// axis in chunks of at least `min_rows` rows until the grid has about `blocks` workgroups.
+struct ColChunks {
+  uint64_t slices;  // of one row's columns
+  uint64_t chunks, seglen;
+};
+inline ColChunks col_chunks(uint64_t rows, uint64_t len, uint64_t inner, uint64_t width,
+                            uint64_t min_rows, uint64_t blocks) {
+  ColChunks c;
+  c.slices = div_up(inner, 64 * width);
+  const uint64_t base = c.slices * rows;
+  c.chunks = 1;
+  if (base < blocks && len >= 2 * min_rows) {
+    c.chunks = div_up(blocks, base);
+    if (c.chunks > len / min_rows) c.chunks = len / min_rows;
+    if (c.chunks > 65535) c.chunks = 65535;
+  }
+  c.seglen = div_up(len, c.chunks);
+  c.chunks = div_up(len, c.seglen);
+  return c;
+}
+
+// Narrow columns read as one flat array: T of kFlatBlock lanes take consecutive float4 units, 4 T
+// floats being R whole rows (a step). Chunks of whole steps: one up to eight of them, else eight
+// steps each up to about `blocks` workgroups, down to two where that leaves the chip idle (sum and
+// max of [60000, 10]: 16.0 us with chunks of eight, 13.4 of two; the bias gradient of [16384, 250]:
+// 28.3 and 30.6).
+constexpr uint32_t kFlatBlock = 512, kFlatInner = 256;  // inner is below kFlatInner
+struct FlatCols {
+  uint32_t T, R;
+  uint64_t chunks, seglen;
+};
+inline FlatCols flat_cols(uint64_t rows, uint64_t len, uint64_t inner, uint64_t blocks) {
+  const uint32_t in = uint32_t(inner);
+  const uint32_t units = in % 4 == 0 ? in / 4 : in % 2 == 0 ? in / 2 : in;  // of the shortest whole rows
+  FlatCols f;
+  f.T = kFlatBlock / units * units;
+  f.R = uint32_t(uint64_t(4) * f.T / in);
+  const uint64_t steps = div_up(len, f.R);
+  const uint64_t most = div_up(blocks, rows), least = div_up(256, rows);
+  uint64_t c = steps / 8;
+  if (c > most) c = most;
+  if (c < least) c = steps / 2 < least ? steps / 2 : least;
+  if (c > 65535) c = 65535;
+  if (steps <= 8 || c < 1) c = 1;
+  f.seglen = div_up(steps, c) * f.R;
+  f.chunks = div_up(len, f.seglen);
+  return f;
+}
+
+// Whether the flat array beats the column kernel at one column a lane (`w`: its chunks). A flat
+// workgroup is 512 lanes and pays its merge through LDS however little it reads (an argmax, whose
+// partials are 16 bytes of value and index, twice that), so over many outer rows of a short axis
+// the column kernel's small workgroups win: sum of [20000, 8, 10] over the 8 16 us against 64,
+// argmax 20 and 200, sum of [1024, 100, 10] 5.4 and 6.7. The flat array wins where it needs one
+// launch and the chunks two (sum of [256, 512, 10] 4.4 us, 8.3 in chunks), where each column
+// workgroup would walk more than some 64 rows (max of [256, 2048, 8] 7.9 and 27.7, of [16, 6000, 10]
+// 8.4 and 9.5), where the partials of many chunks are left to merge (sum of [60000, 10] 7.1 and
+// 8.9), over a few rows of nearly the chunks' 128 (max of [100, 10] 4.8 and 5.3), and, at widths of which a wave's slice leaves a part idle, on large inputs (sum of [16384, 250]
+// 8.4 and 9.6; of [8192, 250] 7.5 and 7.2).
+inline bool flat_pays(const ColChunks &w, const FlatCols &f, uint64_t rows, uint64_t len, uint64_t inner,
+                      bool argmax) {
+  const uint64_t steps = div_up(len, f.R);
+  if (w.chunks == 1)
+    return len >= 256 || (!argmax && ((len >= 128 && rows <= 1024) ||
+                                      (len >= 96 && rows <= 256 && inner >= 8 && inner < 128)));
+  if (f.chunks == 1 && steps <= (!argmax ? 8 : inner < 64 ? 4 : 7)) return true;
+  if (inner < 128) return w.seglen >= 80 || w.chunks > 320;
+  return w.seglen >= 128 || (inner > 192 && !argmax && rows * len * inner >= uint64_t(7) << 19);
+}
+
+// Columns a lane of the column kernel owns where rows allow float4 units: 4 only where the launch is
+// bound by its loads or by its workgroup count. Below some 5.8 million elements it is bound by
+// the rows each wave walks one after the other, and one column a lane makes four times the
+// waves (max of [2048, 1001] 7.9 us, 11 with four, of [8192, 1001] 14.4 and 13.1; sum of [4096, 513]
+// 7.3 and 10.1). Rows of at most 64 columns would leave most of a wave idle with four. Sums of many
+// short columns are bound by the workgroups (sum of [4096, 8, 250] 14.1 us, 7.9 with four; argmax
+// does more per column: of [4096, 8, 77] 10.3 and 15.3).
+inline uint32_t col_width(uint64_t rows, uint64_t len, uint64_t inner, bool argmax) {
+  if (inner <= 64) return 1;
+  if (!argmax && rows * div_up(inner, 64) >= 4096) return 4;
+  return rows * len * inner >= uint64_t(11) << 19 ? 4 : 1;
+}
+
+// Whether a sum of whole float4 columns (partial at a row's end) goes to the one-launch slices, each
+// lane walking its share of the rows: from a few rows on, below 128 only where the slices are few
+// (they read 16 or 32 bytes a row: sum of [256, 100, 77] 6.9 us, 5.2 in columns), up to what one
+// workgroup walks in the time of the second launch it saves. Producers of one operand: sum of
+// [6000, 64] 6.0 us, in chunks 7.3, of [12000, 64] 8.6 and 7.4. Of two and three: the gradient of a
+// multiplied [4000, 64] 7.2 and 8.0, of [6000, 64] 9.0 and 7.8, of [4096, 301] 13.7 and 8.2. Storing
+// ones, whose stores off a 16-byte boundary cost more: the one-pass epilogue at [2048, 64] 6.5 and
+// 7.9, at [1500, 301] 7.1 and 8.2, at [2048, 30] 8.2 and 7.6; config 1's step at [2048, 256] 8.3
+// and 9.4, at [2048, 64] 10.3 and 8.6, at [2048, 8] 6.3 and 7.5.
+inline bool col_slices(uint64_t rows, uint64_t len, uint64_t inner, int nin, bool stores) {
+  const uint64_t n = rows * len * inner;
+  if (len < (stores ? 24 : 48) || (len < 128 && rows * div_up(inner, 64) >= 128)) return false;
+  if (!stores) return len <= (nin == 1 ? 6144 : n <= (uint64_t(1) << 19) ? 4096 : 2048);
+  if (n <= (uint64_t(1) << 15)) return len <= 2048;
+  return len <= (inner % 4 == 0 && (nin == 2 || inner >= 256) ? 2048 : 1536);
+}
+
 }  // namespace plast

@@ -196,6 +196,7 @@ struct ArgmaxComb {
 
 template <int NIN>
 struct RedArgs {
+  static constexpr bool kMulti = false;
   const float *in[NIN];
   void *out;
   int64_t ost[NIN][kMaxRank];  // operand strides on the kept (output) axes, innermost excluded
@@ -215,13 +216,24 @@ struct RedArgs {
   void *part;                  // partial summaries [segs][outputs] when segs > 1
   int post;                    // Post
   float divisor;               // Mean
-  int nx;                      // reduced axes outside the innermost reduced one (MULTI kernels)
-  MagicDiv drun;               // extent of the innermost reduced axis (nx > 0)
+};
+
+// The same with further reduced axes outside the innermost reduced one (the MULTI kernels'). A type of
+// its own: the serial refolds of every other reduction need not ask for each element whether such
+// axes are there (min over the leading axis of [4096, 1024] with a zero in every column: 63 us, 72
+// asking).
+template <int NIN>
+struct RedMultiArgs : RedArgs<NIN> {
+  static constexpr bool kMulti = true;
+  int nx;                      // number of those axes
+  MagicDiv drun;               // extent of the innermost reduced axis
   MagicDiv dunits;             // float4 units of one run of it, the last one partial
-  uint64_t vlen;               // 4 * the units of every run (what MULTI rows with VEC segment)
+  uint64_t vlen;               // 4 * the units of every run (what the rows kernel with VEC segments)
   MagicDiv xdv[kMaxRank];      // extents of the outer reduced axes, outermost first
   int64_t xst[NIN][kMaxRank];  // operand strides along them
 };
+template <int NIN, bool MULTI>
+using RedArgsOf = typename std::conditional<MULTI, RedMultiArgs<NIN>, RedArgs<NIN>>::type;
 
 // Outer-axis decode: index -> per-operand base offsets and the target offset.
 template <int NIN>
@@ -257,12 +269,12 @@ __device__ __forceinline__ void store_final(void *out, int64_t off, const typena
 
 // ------------------------------------------------------------------------- rows kernel
 
-// Offset of the i-th reduced position in every operand: i * rst for one reduced axis (MULTI false),
-// else the coordinates of flattened index i over the outer reduced axes and the position in the
-// innermost one's run (the space has fewer than 2^32 elements there).
-template <bool MULTI, int NIN>
-__device__ __forceinline__ void reduced_offset(const RedArgs<NIN> &A, uint64_t i, int64_t *off) {
-  if constexpr (!MULTI) {
+// Offset of the i-th reduced position in every operand: i * rst for one reduced axis, else the
+// coordinates of flattened index i over the outer reduced axes and the position in the innermost
+// one's run (the space has fewer than 2^32 elements there).
+template <int NIN, class Args>
+__device__ __forceinline__ void reduced_offset(const Args &A, uint64_t i, int64_t *off) {
+  if constexpr (!Args::kMulti) {
 #pragma unroll
     for (int k = 0; k < NIN; ++k) off[k] = int64_t(i) * A.rst[k];
   } else {
@@ -287,11 +299,12 @@ __device__ __forceinline__ void reduced_offset(const RedArgs<NIN> &A, uint64_t i
 // term of the column): its inputs may have been overwritten by those stores (dc written over
 // dout). One with kRefoldInputs stores something other than its terms, over none of the operands
 // its terms read, and recomputes them.
-template <bool MULTI, class Prod, int NIN>
-__device__ __forceinline__ float value_at_as(const RedArgs<NIN> &A, const Prod &prod,
-                                             const int64_t *base, uint64_t i) {
+template <class Prod, class Args>
+__device__ __forceinline__ float value_at(const Args &A, const Prod &prod, const int64_t *base,
+                                          uint64_t i) {
+  constexpr int NIN = Prod::NIN;
   int64_t off[NIN];
-  reduced_offset<MULTI>(A, i, off);
+  reduced_offset<NIN>(A, i, off);
   if constexpr (kStores<Prod> && !StoresOther<Prod>::value) {
     return prod.dst[base[0] + off[0]];
   } else {
@@ -300,11 +313,6 @@ __device__ __forceinline__ float value_at_as(const RedArgs<NIN> &A, const Prod &
     for (int k = 0; k < NIN; ++k) v[k] = A.in[k][base[k] + off[k]];
     return prod.eval(v);
   }
-}
-template <class Prod, int NIN>
-__device__ __forceinline__ float value_at(const RedArgs<NIN> &A, const Prod &prod,
-                                          const int64_t *base, uint64_t i) {
-  return A.nx ? value_at_as<true>(A, prod, base, i) : value_at_as<false>(A, prod, base, i);
 }
 
 template <class T>
@@ -327,8 +335,8 @@ __device__ __forceinline__ float wave_fmax(float v, bool is_max) {
 __device__ __forceinline__ bool wave_any(bool b) { return __any(b); }
 
 // Exact fold summary of [b, e) by one wave, used when the fast path saw a NaN or a zero extreme.
-template <bool IS_MAX, class Prod, int NIN>
-__device__ ExtPart exact_range(const RedArgs<NIN> &A, const Prod &prod, const int64_t *base,
+template <bool IS_MAX, class Prod, class Args>
+__device__ ExtPart exact_range(const Args &A, const Prod &prod, const int64_t *base,
                                uint64_t b, uint64_t e, int lane) {
   // last NaN
   int64_t last_nan = -1;
@@ -369,8 +377,8 @@ constexpr bool kSerialSum = std::is_same<Comb, SumComb>::value;
 __device__ __forceinline__ bool finite_sum(float p) { return fabsf(p) <= FLT_MAX; }
 
 // By one lane: the serial sum of elements [0, len) at base.
-template <class Prod, int NIN>
-__device__ float serial_sum_lane(const RedArgs<NIN> &A, const Prod &prod, const int64_t *base,
+template <class Prod, class Args>
+__device__ float serial_sum_lane(const Args &A, const Prod &prod, const int64_t *base,
                                  uint64_t len) {
   float s = 0.0f;
   for (uint64_t i = 0; i < len; ++i) s = s + value_at(A, prod, base, i);
@@ -380,8 +388,8 @@ __device__ float serial_sum_lane(const RedArgs<NIN> &A, const Prod &prod, const 
 // By a wave, for a whole row: a NaN operand makes every order's sum NaN, so the wave first looks
 // for one (in parallel) and only a row without one is refolded, by lane 0; every lane returns the
 // result.
-template <class Prod, int NIN>
-__device__ float serial_sum_wave(const RedArgs<NIN> &A, const Prod &prod, const int64_t *base,
+template <class Prod, class Args>
+__device__ float serial_sum_wave(const Args &A, const Prod &prod, const int64_t *base,
                                  uint64_t len, float p, int lane) {
   bool nan = false;
   for (uint64_t i = lane; i < len; i += 64) {
@@ -400,9 +408,10 @@ constexpr int kRowUnroll = PLAST_ROW_UNROLL;  // float4 loads in flight per lane
 // value splatted. MULTI: i / 4 counts units of runs whose last unit may be partial; that one is read
 // from four elements before the run's end. Returns the reduced index of the unit's first element;
 // the first `skip` elements belong to the unit before.
-template <bool MULTI, int NIN>
-__device__ __forceinline__ uint64_t load_unit(const RedArgs<NIN> &A, const int64_t *base, uint64_t i,
-                                              f4 *x, uint32_t &skip) {
+template <int NIN, class Args>
+__device__ __forceinline__ uint64_t load_unit(const Args &A, const int64_t *base, uint64_t i, f4 *x,
+                                              uint32_t &skip) {
+  constexpr bool MULTI = Args::kMulti;
   int64_t off[NIN];
   if constexpr (MULTI) {
     const uint32_t run = A.dunits.div(uint32_t(i / 4));
@@ -410,7 +419,7 @@ __device__ __forceinline__ uint64_t load_unit(const RedArgs<NIN> &A, const int64
     const uint32_t pos = at + 4 <= A.drun.d ? at : A.drun.d - 4;
     skip = at - pos;
     i = uint64_t(run) * A.drun.d + pos;
-    reduced_offset<true>(A, i, off);
+    reduced_offset<NIN>(A, i, off);
   } else {
     skip = 0;
   }
@@ -428,13 +437,13 @@ __device__ __forceinline__ uint64_t load_unit(const RedArgs<NIN> &A, const int64
 
 // The reduced index at which MULTI position i (a multiple of 4) starts.
 template <int NIN>
-__device__ __forceinline__ uint64_t run_index(const RedArgs<NIN> &A, uint64_t i) {
+__device__ __forceinline__ uint64_t run_index(const RedMultiArgs<NIN> &A, uint64_t i) {
   const uint32_t run = A.dunits.div(uint32_t(i / 4));
   return uint64_t(run) * A.drun.d + 4 * (uint32_t(i / 4) - run * A.dunits.d);
 }
 
 template <class Prod, class Comb, bool VEC, bool MULTI>
-__global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, Prod prod) {
+__global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgsOf<Prod::NIN, MULTI> A, Prod prod) {
   constexpr int NIN = Prod::NIN;
   using Part = typename Comb::Part;
   const int lane = threadIdx.x & 63;
@@ -446,7 +455,8 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
   int64_t base[NIN], tbase;
   decode_outer(A, row, base, tbase);
   const uint64_t b = uint64_t(seg) * A.seglen;
-  const uint64_t total = VEC && MULTI ? A.vlen : A.len;
+  uint64_t total = A.len;
+  if constexpr (VEC && MULTI) total = A.vlen;
   const uint64_t e = b + A.seglen < total ? b + A.seglen : total;
   // end of the whole float4 units; the up to three elements left are lanes 0 to 2's
   const uint64_t eu = MULTI ? e : e - (e & 3);
@@ -469,7 +479,7 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
           const uint64_t i = i0 + uint64_t(u) * 256;
-          if (i < eu) at[u] = load_unit<MULTI>(A, base, i, x[u], skip[u]);
+          if (i < eu) at[u] = load_unit<NIN>(A, base, i, x[u], skip[u]);
         }
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
@@ -484,9 +494,9 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
           }
         }
       }
-      if (!MULTI && eu + lane < e) take(value_at_as<false>(A, prod, base, eu + lane));
+      if (!MULTI && eu + lane < e) take(value_at(A, prod, base, eu + lane));
     } else {
-      for (uint64_t i = b + lane; i < e; i += 64) take(value_at_as<MULTI>(A, prod, base, i));
+      for (uint64_t i = b + lane; i < e; i += 64) take(value_at(A, prod, base, i));
     }
     m = wave_fmax(m, IS_MAX);
     nan = wave_any(nan);
@@ -511,7 +521,7 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
           const uint64_t i = i0 + uint64_t(u) * 256;
-          if (i < eu) at[u] = load_unit<MULTI>(A, base, i, x[u], skip[u]);
+          if (i < eu) at[u] = load_unit<NIN>(A, base, i, x[u], skip[u]);
         }
 #pragma unroll
         for (int u = 0; u < kRowUnroll; ++u) {
@@ -527,11 +537,11 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgs<Prod::NIN> A, 
         }
       }
       if (!MULTI && eu + lane < e)
-        Comb::next(acc[0], value_at_as<false>(A, prod, base, eu + lane), int64_t(eu + lane));
+        Comb::next(acc[0], value_at(A, prod, base, eu + lane), int64_t(eu + lane));
       p = Comb::merge(Comb::merge(acc[0], acc[1]), Comb::merge(acc[2], acc[3]));
     } else {
       for (uint64_t i = b + lane; i < e; i += 64) {
-        Comb::next(p, value_at_as<MULTI>(A, prod, base, i), int64_t(i));
+        Comb::next(p, value_at(A, prod, base, i), int64_t(i));
       }
     }
 #pragma unroll
@@ -573,7 +583,7 @@ __global__ __launch_bounds__(kBlock) void red_rows_short_kernel(RedArgs<Prod::NI
       // a lane past the row reads its last unit: the loads take no branch
       const uint32_t q = uint32_t(l) + u * L;
       uint32_t skip;
-      load_unit<false>(A, base, uint64_t(q < units ? q : units - 1) * 4, x[u], skip);
+      load_unit<NIN>(A, base, uint64_t(q < units ? q : units - 1) * 4, x[u], skip);
     }
   }
   const auto each = [&](auto &&take) {
@@ -592,7 +602,7 @@ __global__ __launch_bounds__(kBlock) void red_rows_short_kernel(RedArgs<Prod::NI
       }
     }
     for (uint32_t i = units * 4 + l; i < len; i += L)
-      take(0, value_at_as<false>(A, prod, base, i), int64_t(i));
+      take(0, value_at(A, prod, base, i), int64_t(i));
   };
   Part p = Comb::empty();
   bool redo;
@@ -682,8 +692,8 @@ __device__ __forceinline__ P shfl_down_part(const P &p, int off) {
 // runs merge pairwise, always earlier run on the left (every combiner's merge is associative over
 // ordered ranges; for sums this fixes a different, still deterministic, rounding order than one
 // serial pass). A row of 4096 partials took one thread 50 us to merge serially.
-template <class Prod, class Comb>
-__global__ __launch_bounds__(kBlock) void red_rows_finalize(RedArgs<Prod::NIN> A, Prod prod) {
+template <class Prod, class Comb, class Args>
+__global__ __launch_bounds__(kBlock) void red_rows_finalize(Args A, Prod prod) {
   using Part = typename Comb::Part;
   constexpr int NIN = Prod::NIN;
   const int lane = threadIdx.x & 63;
@@ -717,7 +727,7 @@ __global__ __launch_bounds__(kBlock) void red_rows_finalize(RedArgs<Prod::NIN> A
 
 template <class Prod>
 constexpr int kColUnroll = Prod::NIN == 1   ? PLAST_COL_UNROLL
-                           : Prod::NIN == 2 ? PLAST_COL_UNROLL2
+                           : Prod::NIN == 2 && kStores<Prod> ? PLAST_COL_UNROLL2
                                             : PLAST_COL_UNROLL3;
 
 template <class Prod>
@@ -727,10 +737,14 @@ __device__ __forceinline__ void store_col(float *p, f4 v) {
 
 template <class Prod>
 constexpr int kColMinRows = Prod::NIN >= 3 ? PLAST_COL_MIN_ROWS3 : 64;
+// Float4 columns a workgroup of the small kernel owns, and the rows a lane loads per batch: producers
+// of three operands take one column, those of one and storing ones of two take two, and two
+// operands one over narrow rows (the gradient of a multiplied [128, 64] 4.3 us, 4.6 with two) and two
+// over wide ones ([512, 4096] 5.7 us, 7.4 with one).
 template <class Prod>
-constexpr int kColSmallS4 = Prod::NIN >= 3 ? PLAST_COL_SMALL_S4_3 : PLAST_COL_SMALL_S4;
-template <class Prod>
-constexpr int kColSmallU = Prod::NIN >= 3 ? PLAST_COL_SMALL_U3 : PLAST_COL_SMALL_U;
+inline bool col_small_one(uint64_t inner) {
+  return Prod::NIN >= 3 || (Prod::NIN == 2 && !kStores<Prod> && inner < 512);
+}
 
 // Fast summary of an order-sensitive fold (exact max/min): the plain extreme and a NaN flag.
 struct ExtFast {
@@ -750,8 +764,8 @@ struct ExtFast {
 // the operand mask (a broadcast operand's splat makes the compiler wait for each load in turn).
 // RAGGED (with VEC): a row's last unit is partial, or its slices hold fewer than 64 lanes.
 template <class Prod, class Comb, bool VEC, bool ALLV, bool MULTI, bool RAGGED>
-__global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, Prod prod,
-                                                          uint32_t xblocks) {
+__global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgsOf<Prod::NIN, MULTI> A,
+                                                          Prod prod, uint32_t xblocks) {
   constexpr int NIN = Prod::NIN;
   constexpr int W = VEC ? 4 : 1;
   using Part = typename Comb::Part;
@@ -798,7 +812,7 @@ __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, 
       // a row past the chunk is clamped to its last row: loaded, not used
       const uint64_t r = r0 + 4 * u < k1 ? r0 + 4 * u : k1 - 1;
       int64_t roff[NIN];
-      reduced_offset<MULTI>(A, r, roff);
+      reduced_offset<NIN>(A, r, roff);
 #pragma unroll
       for (int k = 0; k < NIN; ++k) {
         const float *src = A.in[k] + lbase[k] + roff[k];
@@ -909,11 +923,12 @@ __global__ __launch_bounds__(kBlock) void red_cols_kernel(RedArgs<Prod::NIN> A, 
 // of float4 column c in order. The row groups of a wave then merge with a fixed butterfly, and the
 // four waves' partials in wave order: the result is deterministic. A column whose sum is not finite
 // is summed again serially in index order (the reference's order decides such sums).
-template <class Prod, bool ALLV>
+// RAGGED: a row's last unit is partial (testing for it costs 5-8% where none is).
+template <class Prod, int S4, bool ALLV, bool RAGGED>
 __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NIN> A, Prod prod,
                                                                 uint32_t xblocks) {
   constexpr int NIN = Prod::NIN;
-  constexpr int S4 = kColSmallS4<Prod>, G = kBlock / S4, kU = kColSmallU<Prod>;
+  constexpr int G = kBlock / S4, kU = S4 == PLAST_COL_SMALL_S4 ? PLAST_COL_SMALL_U : PLAST_COL_SMALL_U3;
   static_assert(64 % S4 == 0, "row groups split evenly over the waves");
   __shared__ f4 sh[kBlock / 64][S4];
   const uint32_t t = threadIdx.x, c4 = t % S4, g = t / S4, lane = t & 63, wv = t >> 6;
@@ -924,8 +939,8 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
   const uint64_t j0 = uint64_t(b - o * xblocks) * (4 * S4);  // the slice's first column
   // a partial unit at the end of a row is read from four columns before the end (see red_cols_kernel)
   const bool active = j0 + 4 * c4 < A.inner;
-  const uint64_t j = j0 + 4 * c4 + 4 <= A.inner ? j0 + 4 * c4 : A.inner - 4;
-  const int skip = active ? int(j0 + 4 * c4 - j) : 0;
+  const uint64_t j = !RAGGED || j0 + 4 * c4 + 4 <= A.inner ? j0 + 4 * c4 : A.inner - 4;
+  const int skip = RAGGED && active ? int(j0 + 4 * c4 - j) : 0;
   int64_t base0[NIN], base[NIN], lbase[NIN], tbase;
   decode_outer(A, o, base0, tbase);
 #pragma unroll
@@ -984,8 +999,8 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
   // lane t finishes one output column, element t % 4 of unit t / 4: the waves' partials in wave order
   const uint64_t ju = j0 + (t & ~3u);  // the unit's first column, before a partial one moves back
   if (ju >= A.inner) return;
-  const uint64_t jc = (ju + 4 <= A.inner ? ju : A.inner - 4) + (t & 3u);
-  if (jc < ju) return;
+  const uint64_t jc = (!RAGGED || ju + 4 <= A.inner ? ju : A.inner - 4) + (t & 3u);
+  if (RAGGED && jc < ju) return;
   float p = sh[0][t / 4][t % 4];
 #pragma unroll
   for (int w = 1; w < kBlock / 64; ++w) p = p + sh[w][t / 4][t % 4];
@@ -1004,17 +1019,16 @@ __global__ __launch_bounds__(kBlock) void red_cols_small_kernel(RedArgs<Prod::NI
 // four elements fall in are the same in every step, whatever inner is, and no lane idles over a short
 // row (a slice of 64 lanes keeps 3 of them on 10 columns). The workgroup's 4 T sums, R per column,
 // are merged through LDS eight rows at a time, in order.
-constexpr int kFlatBlock = 512;
 template <class Prod>
 constexpr int kFlatUnroll = Prod::NIN == 1 ? 4 : 2;
-struct FlatCols {
+struct FlatArgs {
   uint32_t T, R;
   MagicDiv dinner;
 };
 
 template <class Prod, class Comb>
 __global__ __launch_bounds__(kFlatBlock) void red_cols_flat_kernel(RedArgs<Prod::NIN> A, Prod prod,
-                                                                   FlatCols F) {
+                                                                   FlatArgs F) {
   constexpr int NIN = Prod::NIN, kU = kFlatUnroll<Prod>;
   using Part = typename Comb::Part;
   constexpr bool kExt = Comb::kExact;
@@ -1147,8 +1161,8 @@ __global__ __launch_bounds__(kFlatBlock) void red_cols_flat_kernel(RedArgs<Prod:
   else static_cast<Part *>(A.part)[uint64_t(blockIdx.y) * (A.rows * inner) + uint64_t(o) * inner + t] = p;
 }
 
-template <class Prod, class Comb>
-__global__ __launch_bounds__(kBlock) void red_cols_finalize(RedArgs<Prod::NIN> A, Prod prod) {
+template <class Prod, class Comb, class Args>
+__global__ __launch_bounds__(kBlock) void red_cols_finalize(Args A, Prod prod) {
   using Part = typename Comb::Part;
   constexpr int NIN = Prod::NIN;
   const uint64_t oi = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
@@ -1173,8 +1187,8 @@ __global__ __launch_bounds__(kBlock) void red_cols_finalize(RedArgs<Prod::NIN> A
 // consecutive chunks of output o in index order (lanes with the same q read consecutive outputs),
 // then the runs merge pairwise through shuffles with the earlier run always on the left, as in
 // red_rows_finalize. One batch of loads per lane instead of segs / 16 batches in sequence.
-template <class Prod, class Comb, int Q>
-__global__ __launch_bounds__(kBlock) void red_cols_finalize_q(RedArgs<Prod::NIN> A, Prod prod) {
+template <class Prod, class Comb, int Q, class Args>
+__global__ __launch_bounds__(kBlock) void red_cols_finalize_q(Args A, Prod prod) {
   using Part = typename Comb::Part;
   constexpr int NIN = Prod::NIN;
   constexpr uint32_t OPW = 64 / Q;  // outputs per wave
@@ -1277,8 +1291,8 @@ __global__ __launch_bounds__(kBlock) void red_generic_kernel(GenArgs<Prod::NIN> 
 // Merges the chunks' partials (and, for a serial refold, reads the inputs). More than one chunk is
 // planned only below PLAST_COL_BLOCKS workgroups of columns, so nout * Q lanes (at most
 // PLAST_COL_BLOCKS * 256 * Q) stay far inside one launch.
-template <class Prod, class Comb>
-void launch_cols_finalize(const RedArgs<Prod::NIN> &A, const Prod &prod, uint64_t nout, uint64_t chunks) {
+template <class Prod, class Comb, class Args>
+void launch_cols_finalize(const Args &A, const Prod &prod, uint64_t nout, uint64_t chunks) {
   if (PLAST_COL_FIN_Q > 1 && chunks >= 2 * PLAST_COL_FIN_Q)
     red_cols_finalize_q<Prod, Comb, PLAST_COL_FIN_Q>
         <<<ceil_div(nout * PLAST_COL_FIN_Q, kBlock), kBlock, 0, stream()>>>(A, prod);
@@ -1335,7 +1349,7 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
 
   const bool small_idx = s.numel() < (uint64_t(1) << 32) && nout < (uint64_t(1) << 32);
   // the innermost reduced axis, the other reduced axes' flattened walk in every kernel's arguments
-  const auto outer_reduced = [&](RedArgs<NIN> &A) {
+  const auto outer_reduced = [&](RedMultiArgs<NIN> &A) {
     uint64_t len = s.shape[red_ax];
     A.drun = MagicDiv::make(uint32_t(s.shape[red_ax]));
     for (int d = 0; d < red_ax; ++d) {
@@ -1355,8 +1369,9 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
   // are only split when there are fewer than PLAST_ROW_WAVES rows)
   if (!kStores<Prod> && !empty_space && small_idx && nred >= 1 && red_ax == r - 1 &&
       nout <= max_blocks(kBlock) * (kBlock / 64)) {
-    RedArgs<NIN> A;
+    RedMultiArgs<NIN> A;
     memset(&A, 0, sizeof A);
+    const RedArgs<NIN> &A1 = A;  // what the kernels over one reduced axis take
     for (int k = 0; k < NIN; ++k) A.in[k] = static_cast<const float *>(in[k]);
     A.out = out;
     const bool vec = !multi || s.shape[r - 1] >= 4;  // a run's partial unit is read from its end
@@ -1406,9 +1421,9 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       if (!multi && A.len <= 16 * 32) {
         const int lanes = A.len <= 16 * 2 ? 2 : A.len <= 16 * 8 ? 8 : 32;
         const unsigned sgrid = ceil_div(A.rows, (kBlock / 64) * (64 / lanes));
-        if (lanes == 2) red_rows_short_kernel<Prod, Comb, 2><<<sgrid, kBlock, 0, stream()>>>(A, prod);
-        else if (lanes == 8) red_rows_short_kernel<Prod, Comb, 8><<<sgrid, kBlock, 0, stream()>>>(A, prod);
-        else red_rows_short_kernel<Prod, Comb, 32><<<sgrid, kBlock, 0, stream()>>>(A, prod);
+        if (lanes == 2) red_rows_short_kernel<Prod, Comb, 2><<<sgrid, kBlock, 0, stream()>>>(A1, prod);
+        else if (lanes == 8) red_rows_short_kernel<Prod, Comb, 8><<<sgrid, kBlock, 0, stream()>>>(A1, prod);
+        else red_rows_short_kernel<Prod, Comb, 32><<<sgrid, kBlock, 0, stream()>>>(A1, prod);
         return true;
       }
       const uint64_t waves = A.rows * segs;
@@ -1416,21 +1431,26 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       if (vec && multi)
         red_rows_kernel<Prod, Comb, true, true><<<grid, kBlock, 0, stream()>>>(A, prod);
       else if (vec)
-        red_rows_kernel<Prod, Comb, true, false><<<grid, kBlock, 0, stream()>>>(A, prod);
+        red_rows_kernel<Prod, Comb, true, false><<<grid, kBlock, 0, stream()>>>(A1, prod);
       else
         red_rows_kernel<Prod, Comb, false, true><<<grid, kBlock, 0, stream()>>>(A, prod);
-      if (segs > 1)  // the finalize reads the partials, and the inputs for a serial refold
-        red_rows_finalize<Prod, Comb>
-            <<<ceil_div(A.rows, kBlock / 64), kBlock, 0, stream()>>>(A, prod);
+      if (segs > 1) {  // the finalize reads the partials, and the inputs for a serial refold
+        const unsigned fgrid = ceil_div(A.rows, kBlock / 64);
+        if (multi) red_rows_finalize<Prod, Comb><<<fgrid, kBlock, 0, stream()>>>(A, prod);
+        else red_rows_finalize<Prod, Comb><<<fgrid, kBlock, 0, stream()>>>(A1, prod);
+      }
       return true;
     }
   }
 
-  // ---- cols: innermost axis kept with unit target stride
-  if (!empty_space && small_idx && nred >= 1 && (!multi || !kStores<Prod>) && red_ax != r - 1 &&
+  // ---- cols: innermost axis kept with unit target stride (several reduced axes beside it: the
+  // gradient of a broadcast operand, a sum)
+  constexpr bool kMultiCols = !kStores<Prod> && std::is_same<Comb, SumComb>::value;
+  if (!empty_space && small_idx && nred >= 1 && (!multi || kMultiCols) && red_ax != r - 1 &&
       s.st[NIN][r - 1] != 0) {
-    RedArgs<NIN> A;
+    RedMultiArgs<NIN> A;
     memset(&A, 0, sizeof A);
+    const RedArgs<NIN> &A1 = A;  // what the kernels over one reduced axis take
     for (int k = 0; k < NIN; ++k) A.in[k] = static_cast<const float *>(in[k]);
     A.out = out;
     A.inner = s.shape[r - 1];
@@ -1446,7 +1466,9 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
       ++no;
     }
     A.nouter = no;
-    bool flat = !multi && A.inner < 256;  // narrow: rows read as one flat array
+    constexpr bool kArg = std::is_same<Comb, ArgmaxComb>::value;
+    // rows read as one flat array: operands contiguous over [len, inner] or constant along len
+    bool flat = !multi && A.inner < kFlatInner;
     for (int k = 0; k < NIN; ++k) {
       A.rst[k] = s.st[k][red_ax];
       A.kst[k] = s.st[k][r - 1];
@@ -1456,110 +1478,95 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
     }
     if (kStores<Prod> && A.rst[0] == 0) flat = false;
     A.rows = nout / A.inner;  // outer count
-    const bool allv = A.vec_mask == (1u << NIN) - 1;
-    const uint32_t W = vec ? 4 : 1;
-    const uint32_t xblocks = ceil_div(A.inner, uint64_t(64) * W);
-    // the slices of a row share its lanes evenly, in whole 128-byte lines
-    A.lanes = ceil_div(ceil_div(A.inner, W), xblocks);
-    A.lanes = vec && A.lanes < 56 ? (A.lanes + 7) / 8 * 8 : 64;
-    const uint64_t base_blocks = uint64_t(xblocks) * A.rows;
-    // chunk the reduced axis until the grid has ~PLAST_COL_BLOCKS workgroups, keeping at least
-    // kColMinRows rows per chunk
-    uint64_t chunks = 1;
-    constexpr uint64_t min_rows = kColMinRows<Prod>;
-    if (base_blocks < PLAST_COL_BLOCKS && A.len >= 2 * min_rows) {
-      chunks = (PLAST_COL_BLOCKS + base_blocks - 1) / base_blocks;
-      const uint64_t max_c = A.len / min_rows;
-      if (chunks > max_c) chunks = max_c;
-      if (chunks > 65535) chunks = 65535;
-      if (chunks < 1) chunks = 1;
-    }
-    uint64_t seglen = (A.len + chunks - 1) / chunks;
-    chunks = (A.len + seglen - 1) / seglen;
-    A.segs = uint32_t(chunks);
-    A.seglen = seglen;
     A.post = int(post);
     A.divisor = divisor;
+    const bool allv = A.vec_mask == (1u << NIN) - 1;
+    const uint64_t nall = A.len * nout;
+    // sums that some form takes in one launch: a capture needs no workspace for them
+    const bool one_pass = std::is_same<Comb, SumComb>::value && vec && A.inner % 4 == 0 &&
+                          nall <= PLAST_COL_SMALL_MAX;
     if constexpr (std::is_same<Comb, SumComb>::value) {
-      // small: one launch over narrow column slices instead of chunks plus a finalize, while a lane's
-      // share of the rows stays a few batches (narrow columns leave few workgroups). Below 128 rows
-      // only where slices of 256 columns leave most of the chip idle: config 1's step at [32, 568]
-      // 10.8 us in slices, 6.4 so, at [60, 3000] 15.6 and 7.5, at [16, 4096] 6.9 and 6.3.
-      const uint64_t few_rows = uint64_t(2) * kColSmallU<Prod> * (kBlock / kColSmallS4<Prod>);
-      if ((A.len >= 128 || (A.len >= 16 && base_blocks < 64)) && vec && !multi && A.len * nout <= PLAST_COL_SMALL_MAX &&
-          (!flat || A.len <= few_rows) && (NIN < 3 || PLAST_COL_SMALL3 != 0)) {
-        const uint32_t sblocks = ceil_div(A.inner, uint64_t(4) * kColSmallS4<Prod>);
-        const uint64_t sgrid = uint64_t(sblocks) * A.rows;
-        if (sgrid <= max_blocks(kBlock)) {
+      // small: one launch over narrow column slices instead of chunks plus a finalize
+      if (vec && !multi && nall <= PLAST_COL_SMALL_MAX &&
+          col_slices(A.rows, A.len, A.inner, NIN, kStores<Prod>) && (NIN < 3 || PLAST_COL_SMALL3 != 0)) {
+        const auto slices = [&](auto s4, auto every, auto ragged) {
+          constexpr int S4 = decltype(s4)::value;
+          const uint32_t sblocks = ceil_div(A.inner, uint64_t(4) * S4);
+          const uint64_t sgrid = uint64_t(sblocks) * A.rows;
+          if (sgrid > max_blocks(kBlock)) return false;
           A.segs = 1;
-          const unsigned grid = unsigned(sgrid);
-          if (allv) red_cols_small_kernel<Prod, true><<<grid, kBlock, 0, stream()>>>(A, prod, sblocks);
-          else red_cols_small_kernel<Prod, false><<<grid, kBlock, 0, stream()>>>(A, prod, sblocks);
+          red_cols_small_kernel<Prod, S4, decltype(every)::value, decltype(ragged)::value>
+              <<<unsigned(sgrid), kBlock, 0, stream()>>>(A1, prod, sblocks);
           return true;
-        }
+        };
+        const auto with_form = [&](auto s4) {
+          if (A.inner % 4 == 0)
+            return allv ? slices(s4, std::true_type{}, std::false_type{}) : slices(s4, std::false_type{}, std::false_type{});
+          return allv ? slices(s4, std::true_type{}, std::true_type{}) : slices(s4, std::false_type{}, std::true_type{});
+        };
+        bool done;
+        if constexpr (NIN == 1) done = with_form(std::integral_constant<int, PLAST_COL_SMALL_S4>{});
+        else if (col_small_one<Prod>(A.inner)) done = with_form(std::integral_constant<int, PLAST_COL_SMALL_S4_3>{});
+        else done = with_form(std::integral_constant<int, PLAST_COL_SMALL_S4>{});
+        if (done) return true;
       }
     }
     if (flat && A.rows <= max_blocks(kFlatBlock)) {
-      const uint32_t in = uint32_t(A.inner);
-      const uint32_t units = in % 4 == 0 ? in / 4 : in % 2 == 0 ? in / 2 : in;  // of the shortest
-      FlatCols F;                                                             // whole rows
-      F.T = kFlatBlock / units * units;
-      F.R = uint32_t(uint64_t(4) * F.T / in);
-      F.dinner = MagicDiv::make(in);
-      // chunks of whole steps: eight steps each up to about PLAST_COL_BLOCKS workgroups, down to two
-      // where that leaves the chip idle (sum and max of [60000, 10]: 16.0 us with chunks of eight,
-      // 13.4 of two; the bias gradient of [16384, 250]: 28.3 and 30.6)
-      const uint64_t steps = (A.len + F.R - 1) / F.R;
-      uint64_t fc = steps / 8;
-      const uint64_t most = (PLAST_COL_BLOCKS + A.rows - 1) / A.rows, least = (256 + A.rows - 1) / A.rows;
-      if (fc > most) fc = most;
-      if (fc < least) fc = steps / 2 < least ? steps / 2 : least;
-      // one chunk needs no partials, as neither a short axis nor a small sum of whole float4 columns
-      // does in slices
-      const bool slices_fit = chunks == 1 || (std::is_same<Comb, SumComb>::value && in % 4 == 0 && vec &&
-                                              A.len * nout <= PLAST_COL_SMALL_MAX);
-      if (steps <= 8) fc = 1;
-      if (fc > 65535) fc = 65535;
-      if (fc < 1) fc = 1;
-      A.seglen = (steps + fc - 1) / fc * F.R;
-      chunks = (A.len + A.seglen - 1) / A.seglen;
-      A.segs = uint32_t(chunks);
-      if (chunks > 1) {
-        A.part = slices_fit ? partials(sizeof(Part) * nout * chunks, where)
-                            : workspace(sizeof(Part) * nout * chunks);
-        if (!A.part) return false;
+      const FlatCols f = flat_cols(A.rows, A.len, A.inner, PLAST_COL_BLOCKS);
+      const ColChunks w = col_chunks(A.rows, A.len, A.inner, 1, kColMinRows<Prod>, PLAST_COL_BLOCKS);
+      if (kStores<Prod> ? A.len >= 64 : flat_pays(w, f, A.rows, A.len, A.inner, kArg)) {
+        A.segs = uint32_t(f.chunks);
+        A.seglen = f.seglen;
+        if (f.chunks > 1) {
+          const size_t bytes = sizeof(Part) * nout * f.chunks;
+          A.part = one_pass || w.chunks == 1 ? partials(bytes, where) : workspace(bytes);
+          if (!A.part) return false;
+        }
+        const FlatArgs F{f.T, f.R, MagicDiv::make(uint32_t(A.inner))};
+        const dim3 grid{unsigned(A.rows), unsigned(f.chunks), 1u};
+        red_cols_flat_kernel<Prod, Comb><<<grid, kFlatBlock, 0, stream()>>>(A1, prod, F);
+        if (f.chunks > 1) launch_cols_finalize<Prod, Comb>(A1, prod, nout, f.chunks);
+        return true;
       }
-      const dim3 grid{unsigned(A.rows), unsigned(chunks), 1u};
-      red_cols_flat_kernel<Prod, Comb><<<grid, kFlatBlock, 0, stream()>>>(A, prod, F);
-      if (chunks > 1) launch_cols_finalize<Prod, Comb>(A, prod, nout, chunks);
-      return true;
     }
+    if (!multi && col_width(A.rows, A.len, A.inner, kArg) == 1) vec = false;
+    const uint32_t W = vec ? 4 : 1;
+    const ColChunks w = col_chunks(A.rows, A.len, A.inner, W, kColMinRows<Prod>, PLAST_COL_BLOCKS);
+    const uint32_t xblocks = uint32_t(w.slices);
+    const uint64_t chunks = w.chunks;
+    A.segs = uint32_t(chunks);
+    A.seglen = w.seglen;
+    // the slices of a row share its lanes evenly, in whole 128-byte lines
+    A.lanes = ceil_div(ceil_div(A.inner, W), xblocks);
+    A.lanes = vec && A.lanes < 56 ? (A.lanes + 7) / 8 * 8 : 64;
+    const uint64_t base_blocks = w.slices * A.rows;
     if (base_blocks <= max_blocks(kBlock)) {
       if (chunks > 1) {
-        A.part = multi ? partials(sizeof(Part) * nout * chunks, where)
-                       : workspace(sizeof(Part) * nout * chunks);
+        const size_t bytes = sizeof(Part) * nout * chunks;
+        A.part = multi || one_pass ? partials(bytes, where) : workspace(bytes);
         if (!A.part) return false;
       }
       const dim3 grid{unsigned(base_blocks), unsigned(chunks), 1u};
-      bool launched = false;
-      if constexpr (!kStores<Prod>) {
-        if (multi && vec)
-          red_cols_kernel<Prod, Comb, true, false, true, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
-        else if (multi)
-          red_cols_kernel<Prod, Comb, false, false, true, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
-        launched = multi;
+      if constexpr (kMultiCols) {
+        if (multi) {
+          if (vec)
+            red_cols_kernel<Prod, Comb, true, false, true, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+          else
+            red_cols_kernel<Prod, Comb, false, false, true, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+          if (chunks > 1) launch_cols_finalize<Prod, Comb>(A, prod, nout, chunks);
+          return true;
+        }
       }
       const bool ragged = A.inner % 4 != 0 || A.lanes < 64;
-      if (launched) {
-      } else if (vec && allv && ragged)
-        red_cols_kernel<Prod, Comb, true, true, false, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+      if (vec && allv && ragged)
+        red_cols_kernel<Prod, Comb, true, true, false, true><<<grid, kBlock, 0, stream()>>>(A1, prod, xblocks);
       else if (vec && allv)
-        red_cols_kernel<Prod, Comb, true, true, false, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+        red_cols_kernel<Prod, Comb, true, true, false, false><<<grid, kBlock, 0, stream()>>>(A1, prod, xblocks);
       else if (vec)
-        red_cols_kernel<Prod, Comb, true, false, false, true><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
+        red_cols_kernel<Prod, Comb, true, false, false, true><<<grid, kBlock, 0, stream()>>>(A1, prod, xblocks);
       else
-        red_cols_kernel<Prod, Comb, false, false, false, false><<<grid, kBlock, 0, stream()>>>(A, prod, xblocks);
-      if (chunks > 1) launch_cols_finalize<Prod, Comb>(A, prod, nout, chunks);
+        red_cols_kernel<Prod, Comb, false, false, false, false><<<grid, kBlock, 0, stream()>>>(A1, prod, xblocks);
+      if (chunks > 1) launch_cols_finalize<Prod, Comb>(A1, prod, nout, chunks);
       return true;
     }
   }
