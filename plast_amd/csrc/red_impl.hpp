@@ -563,7 +563,9 @@ __global__ __launch_bounds__(kBlock) void red_rows_kernel(RedArgsOf<Prod::NIN, M
 // contiguous stretch of rows (a wave per row of 77 floats kept 20 of its 64 lanes on 308 bytes, and
 // took 15 us for 15 MB). Each lane holds up to four float4 units of its row, all loaded before the
 // first is used, and the up to three elements left. A row whose fast value could differ from the
-// reference's (max/min of a NaN or a zero extreme, a non-finite sum) is redone by the whole wave.
+// reference's (max/min of a NaN or a zero extreme, a non-finite sum) is redone by its own lanes, from
+// the same registers: min of [1000, 100] with a zero in every row 16.9 us with a wave's rows redone
+// one after the other, 4.4 with a wave per row.
 template <class Prod, class Comb, int L>
 __global__ __launch_bounds__(kBlock) void red_rows_short_kernel(RedArgs<Prod::NIN> A, Prod prod) {
   constexpr int NIN = Prod::NIN, U = 4;
@@ -631,17 +633,48 @@ __global__ __launch_bounds__(kBlock) void red_rows_short_kernel(RedArgs<Prod::NI
     redo = false;
     if constexpr (kSerialSum<Comb>) redo = !finite_sum(p);
   }
-  if constexpr (Comb::kExact || kSerialSum<Comb>) {
-    for (uint64_t todo = __ballot(redo && valid && l == 0); todo; todo &= todo - 1) {
-      const int first = __ffsll((unsigned long long)todo) - 1;  // the row's first lane
-      int64_t rb[NIN], rt;
-      decode_outer(A, uint32_t(row0 + first / L), rb, rt);
-      Part r;
-      if constexpr (Comb::kExact)
-        r = exact_range<std::is_same<Comb, ExtComb<true>>::value>(A, prod, rb, 0, A.len, lane);
-      else
-        r = serial_sum_wave(A, prod, rb, A.len, __shfl(p, first), lane);
-      if (lane == first) p = r;
+  if (__any(redo && valid)) {  // every row of the wave at once, each by its own lanes
+    if constexpr (Comb::kExact) {
+      constexpr bool IS_MAX = std::is_same<Comb, ExtComb<true>>::value;
+      const auto group_last = [](int v) {
+#pragma unroll
+        for (int s = L / 2; s >= 1; s >>= 1) {
+          const int o = __shfl_xor(v, s);
+          v = o > v ? o : v;
+        }
+        return v;
+      };
+      int last_nan = -1;
+      each([&](int, float y, int64_t i) {
+        if (y != y && int(i) > last_nan) last_nan = int(i);
+      });
+      last_nan = group_last(last_nan);
+      // the extreme after the last NaN, and the last zero there (its index and sign)
+      float m = IS_MAX ? -__builtin_huge_valf() : __builtin_huge_valf();
+      int zero = -1;
+      each([&](int, float y, int64_t i) {
+        if (int(i) <= last_nan) return;
+        m = IS_MAX ? fmaxf(m, y) : fminf(m, y);
+        const int key = 2 * int(i) + int(__float_as_uint(y) >> 31);
+        if (y == 0.0f && key > zero) zero = key;
+      });
+#pragma unroll
+      for (int s = L / 2; s >= 1; s >>= 1) {
+        const float o = __shfl_xor(m, s);
+        m = IS_MAX ? fmaxf(m, o) : fminf(m, o);
+      }
+      zero = group_last(zero);
+      if (redo) {
+        p = ExtPart{m == 0.0f ? (zero & 1 ? -0.0f : 0.0f) : m, kNonEmpty | (last_nan >= 0 ? kIndep : 0u)};
+        // a row that ends in a NaN: the fold's value is that NaN
+        if (last_nan == int(len) - 1) p.r = value_at(A, prod, base, uint64_t(last_nan));
+      }
+    } else if constexpr (kSerialSum<Comb>) {
+      uint32_t nan = 0;  // a NaN term makes every order's sum NaN
+      each([&](int, float y, int64_t) { nan |= y != y ? 1u : 0u; });
+#pragma unroll
+      for (int s = L / 2; s >= 1; s >>= 1) nan |= uint32_t(__shfl_xor(int(nan), s));
+      if (redo && !nan && l == 0) p = serial_sum_lane(A, prod, base, A.len);
     }
   }
   if (l == 0 && valid) store_final<Comb>(A.out, tbase, p, A.post, A.divisor);
@@ -1115,26 +1148,92 @@ __global__ __launch_bounds__(kFlatBlock) void red_cols_flat_kernel(RedArgs<Prod:
   }
   __syncthreads();
   // sh[r][j]: the sums of rows r, r + R, ... of column j; rows 8e .. 8e + 7 merge into row e. A round
-  // has at most T / 2 + inner of them (rounding up), two per lane.
+  // leaves ceil(R / 8) * inner sums at most, R * inner being 4 T: 448, one a lane.
   for (uint32_t rows = F.R; rows > 1;) {
     const uint32_t next = (rows + 7) / 8;
-    Fast g[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t i = t + uint32_t(h) * kFlatBlock;
-      if (i >= next * inner) continue;
-      const uint32_t e = F.dinner.div(i), j = i - e * inner;
-      g[h] = sh[8 * e * inner + j];
+    Fast g;
+    if (t < next * inner) {
+      const uint32_t e = F.dinner.div(t), j = t - e * inner;
+      g = sh[8 * e * inner + j];
 #pragma unroll
       for (uint32_t q = 1; q < 8; ++q)
-        if (8 * e + q < rows) g[h] = merge(g[h], sh[(8 * e + q) * inner + j]);
+        if (8 * e + q < rows) g = merge(g, sh[(8 * e + q) * inner + j]);
     }
     __syncthreads();
-#pragma unroll
-    for (int h = 0; h < 2; ++h)
-      if (t + uint32_t(h) * kFlatBlock < next * inner) sh[t + uint32_t(h) * kFlatBlock] = g[h];
+    if (t < next * inner) sh[t] = g;
     __syncthreads();
     rows = next;
+  }
+  if constexpr (kExt) {
+    // Columns with a zero extreme or a NaN, all of them at once: the workgroup walks its chunk again
+    // (from the caches) for the last NaN of each, the extreme after it, and the last zero after it,
+    // whose sign decides the bits. One lane a column folding its chunk in order took 93 us for max of
+    // [60000, 10] with a zero in every column.
+    static_assert(NIN == 1, "order-sensitive folds are of one operand");
+    __shared__ uint32_t last[kFlatInner], key[kFlatInner], zero[kFlatInner];
+    const bool nan = t < inner && sh[t].nan;
+    if (__syncthreads_or(nan || (t < inner && sh[t].m == 0.0f))) {
+      const bool any_nan = __syncthreads_or(nan);
+      if (t < inner) last[t] = zero[t] = 0, key[t] = IS_MAX ? 0u : ~0u;
+      __syncthreads();
+      // take(c, y, the row of the chunk + 1), then done(c, column) for the lane's four columns
+      const auto walk = [&](auto &&take, auto &&done) {
+        if (t < F.T) {
+          const float *src = A.in[0] + base[0] + k0 * inner;
+          uint32_t step = 0;
+          for (uint64_t at = 4 * t; at < nf; at += uint64_t(4) * F.T, ++step) {
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c)
+              if (at + c < nf) {
+                const float v = A.rst[0] == 0 ? fixed[0][c] : src[at + c];
+                take(c, prod.eval(&v), step * F.R + row[c] + 1);
+              }
+          }
+#pragma unroll
+          for (uint32_t c = 0; c < 4; ++c) done(c, 4 * t + c - row[c] * inner);
+        }
+        __syncthreads();
+      };
+      uint32_t best[4] = {};
+      const auto later = [&](uint32_t *to) {
+        return [&best, to](uint32_t c, uint32_t col) {
+          if (best[c]) atomicMax(&to[col], best[c]);
+        };
+      };
+      if (any_nan) {
+        walk([&](uint32_t c, float y, uint32_t r) { if (y != y) best[c] = r; }, later(last));
+        uint32_t from[4];
+        float m[4];
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+          from[c] = t < F.T ? last[4 * t + c - row[c] * inner] : 0;
+          m[c] = IS_MAX ? -__builtin_huge_valf() : __builtin_huge_valf();
+        }
+        // as unsigned integers ordered like the floats
+        walk([&](uint32_t c, float y, uint32_t r) {
+          if (r > from[c]) m[c] = IS_MAX ? fmaxf(m[c], y) : fminf(m[c], y);
+        }, [&](uint32_t c, uint32_t col) {
+          const uint32_t u = __float_as_uint(m[c]), o = u >> 31 ? ~u : u | 0x80000000u;
+          if constexpr (IS_MAX) atomicMax(&key[col], o);
+          else atomicMin(&key[col], o);
+        });
+      }
+#pragma unroll
+      for (int c = 0; c < 4; ++c) best[c] = 0;
+      walk([&](uint32_t c, float y, uint32_t r) { if (y == 0.0f) best[c] = r; }, later(zero));
+      if (t < inner) {
+        const uint32_t o = key[t];
+        float m = nan ? __uint_as_float(o >> 31 ? o & 0x7fffffffu : ~o) : sh[t].m;
+        int64_t at = base[0] + int64_t(t) * A.kst[0] + int64_t(k0) * A.rst[0];
+        // (a column that ends in a NaN: the fold's value is that NaN)
+        const uint32_t r = nan && last[t] == uint32_t(k1 - k0) ? last[t] : m == 0.0f ? zero[t] : 0;
+        if (r) {
+          const float v = A.in[0][at + int64_t(r - 1) * A.rst[0]];
+          m = prod.eval(&v);
+        }
+        sh[t].m = m;
+      }
+    }
   }
   if (t >= inner) return;
   int64_t bc[NIN];
@@ -1142,16 +1241,7 @@ __global__ __launch_bounds__(kFlatBlock) void red_cols_flat_kernel(RedArgs<Prod:
   for (int k = 0; k < NIN; ++k) bc[k] = base[k] + int64_t(t) * A.kst[k];
   Part p;
   if constexpr (kExt) {
-    if (!sh[t].nan && sh[t].m != 0.0f) {
-      p = ExtPart{sh[t].m, kNonEmpty};
-    } else {
-      p = Comb::empty();
-      for (uint64_t r = k0; r < k1; ++r) {
-        const float y = value_at(A, prod, bc, r);
-        if (r == k0) Comb::first(p, y, int64_t(r));
-        else Comb::next(p, y, int64_t(r));
-      }
-    }
+    p = ExtPart{sh[t].m, kNonEmpty | (sh[t].nan ? kIndep : 0u)};
   } else {
     p = sh[t];
     if constexpr (kSerialSum<Comb>)
