@@ -197,12 +197,36 @@ __global__ __launch_bounds__(T > 64 ? T : kBlock) void ext_bwd_rows_kernel(RedAr
   }
   if (!valid || cnt == 0) return;
   const float add = g / float(n);
-  da[pos] = da[pos] + add;
+  const float first = da[pos] + add;
+  da[pos] = first;
   if (cnt == 1) return;
-  // several ties in one thread's share (an order of its own: units, then the elements left over)
-  for (uint32_t q = pos / 4 < units ? pos / 4 : units + l; q < units; q += T)
-    for (uint32_t i = 4 * q; i < 4 * q + 4; ++i)
-      if (i > pos && a[i] == e) da[i] = da[i] + add;
+  // several ties in one thread's share: its units from the first one on, and the elements left over
+  // (an order of its own: the first tie may be among those)
+  const auto part = [&](const float *p, uint32_t q) {
+    return __builtin_nontemporal_load(reinterpret_cast<const f4u *>(p + 4 * uint64_t(q)));
+  };
+  for (uint32_t q0 = pos / 4 < units ? pos / 4 : units; q0 < units; q0 += T * U) {
+    f4 x[U], d[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t q = q0 + uint32_t(u) * T < units ? q0 + uint32_t(u) * T : units - 1;
+      x[u] = part(a, q);
+      d[u] = part(da, q);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const uint32_t q = q0 + uint32_t(u) * T;
+      if (q >= units) continue;
+      bool any = false;
+#pragma unroll
+      for (uint32_t c = 0; c < 4; ++c) {
+        // the first tie is accumulated already: its new value may not be what was loaded
+        if (4 * q + c == pos) d[u][c] = first;
+        else if (x[u][c] == e) d[u][c] = d[u][c] + add, any = true;
+      }
+      if (any) store_unit<true>(d[u], da + 4 * uint64_t(q));
+    }
+  }
   for (uint32_t i = units * 4 + l; i < len; i += T)
     if (i != pos && a[i] == e) da[i] = da[i] + add;
 }

@@ -44,6 +44,13 @@ def _cases():
         for op in REDUCE:
             out.append(Case(f"{op}_cols_bwd_{s}", op, "bwd", [Arr(s, "ties", 80 + i, requires_grad=True)],
                             _red_shape(s, 1, 0), (1, 0, 0.0)))
+    # max/min backward over rows on each thread count and loop trip of its kernel, and past them
+    for i, s in enumerate([(3, 1025), (3, 2047), (5, 2048), (3, 2049), (2, 4099), (2, 16387), (2, 32768), (2, 32769),
+                           (257, 32769), (70, 128), (70, 1024)]):
+        for op in ("max", "min"):
+            for d in ("ties", "special"):
+                out.append(Case(f"{op}_rows_bwd_{s}_{d}", op, "bwd", [Arr(s, d, 90 + i, requires_grad=True)],
+                                _red_shape(s, 1, 0), (1, 0, 0.0)))
     return out
 
 
@@ -84,3 +91,34 @@ def test_misaligned_input(shape, dim, off):
         else:
             bar = 1e-5 * np.abs(h).astype(np.float64).sum(axis=dim)
             assert np.all(np.abs(out.numpy() - h.astype(np.float64).sum(axis=dim)) <= bar)
+
+
+@pytest.mark.parametrize("op", ["max", "min"])
+@pytest.mark.parametrize("shape", [(40, 9), (20, 300), (7, 1500), (5, 3000), (2, 40000)])
+def test_extreme_backward_strided_and_constant(shape, op):
+    """Max/min backward in its one read over a window of a wider matrix whose gradient is a window of
+    another, and over rows of one value, all of it ties: every element gets dout / n, and what lies
+    between the rows stays as it was."""
+    from plast_amd import abi, runtime as rt
+    from plast_amd.abi import KernelParams
+    print(f"{op} {shape}", flush=True)
+    rows, cols = shape
+    rng = np.random.RandomState(cols)
+    x = rng.randint(-2, 3, (rows, cols + 5)).astype(np.float32)
+    x[0] = x[rows // 2] = 1.0
+    d0 = rng.randn(rows, cols + 9).astype(np.float32)
+    dout = rng.randn(rows).astype(np.float32)
+    X, D = rt.DeviceTensor.from_numpy(x), rt.DeviceTensor.from_numpy(d0)
+    gt = abi.make_tensor(D.ptr + 7 * 4, shape, (cols + 9, 1), rt.FLOAT32)
+    v = abi.make_tensor(X.ptr + 3 * 4, shape, (cols + 5, 1), rt.FLOAT32, rt.GPU, True, gt)
+    out = rt.DeviceTensor((rows,), requires_grad=True)
+    rt.lib().arena_memcpy_h2d_hip(out.grad.ptr, dout.ctypes.data, dout.nbytes)
+    p = KernelParams(1, 0, 0.0)
+    rt.forward(op, [v], out, p)
+    rt.backward(op, [v], out, p)
+    w = x[:, 3:3 + cols]
+    tie = w == getattr(w, op)(1)[:, None]
+    want = d0.copy()
+    add = (dout / tie.sum(1, dtype=np.float32)).astype(np.float32)
+    want[:, 7:7 + cols] = np.where(tie, d0[:, 7:7 + cols] + add[:, None], d0[:, 7:7 + cols])
+    assert np.array_equal(D.numpy(), want)
