@@ -84,14 +84,16 @@ inline FlatCols flat_cols(uint64_t rows, uint64_t len, uint64_t inner, uint64_t 
 // launch and the chunks two (sum of [256, 512, 10] 4.4 us, 8.3 in chunks), where each column
 // workgroup would walk more than some 64 rows (max of [256, 2048, 8] 7.9 and 27.7, of [16, 6000, 10]
 // 8.4 and 9.5), where the partials of many chunks are left to merge (sum of [60000, 10] 7.1 and
-// 8.9), over a few rows of nearly the chunks' 128 (max of [100, 10] 4.8 and 5.3), and, at widths of which a wave's slice leaves a part idle, on large inputs (sum of [16384, 250]
+// 8.9), over a few rows of nearly the chunks' 128 (max of [100, 10] 4.8 and 5.3), where its workgroups
+// have thousands of elements each of a large input (max of [1000, 100, 100] 9.2 and 13.3), and, at widths of which a wave's slice leaves a part idle, on large inputs (sum of [16384, 250]
 // 8.4 and 9.6; of [8192, 250] 7.5 and 7.2).
 inline bool flat_pays(const ColChunks &w, const FlatCols &f, uint64_t rows, uint64_t len, uint64_t inner,
                       bool argmax) {
   const uint64_t steps = div_up(len, f.R);
   if (w.chunks == 1)
-    return len >= 256 || (!argmax && ((len >= 128 && rows <= 1024) ||
-                                      (len >= 96 && rows <= 256 && inner >= 8 && inner < 128)));
+    return len >= 256 || (len >= 96 && len * inner >= 8192 && rows * len * inner >= uint64_t(11) << 19) ||
+           (!argmax && ((len >= 128 && rows <= 1024) ||
+                        (len >= 96 && rows <= 256 && inner >= 8 && inner < 128)));
   if (f.chunks == 1 && steps <= (!argmax ? 8 : inner < 64 ? 4 : 7)) return true;
   if (inner < 128) return w.seglen >= 80 || w.chunks > 320;
   return w.seglen >= 128 || (inner > 192 && !argmax && rows * len * inner >= uint64_t(7) << 19);
@@ -102,10 +104,10 @@ inline bool flat_pays(const ColChunks &w, const FlatCols &f, uint64_t rows, uint
 // the rows each wave walks one after the other, and one column a lane makes four times the
 // waves (max of [2048, 1001] 7.9 us, 11 with four, of [8192, 1001] 14.4 and 13.1; sum of [4096, 513]
 // 7.3 and 10.1). Rows of at most 64 columns would leave most of a wave idle with four. Sums of many
-// short columns are bound by the workgroups (sum of [4096, 8, 250] 14.1 us, 7.9 with four; argmax
-// does more per column: of [4096, 8, 77] 10.3 and 15.3).
+// short columns are bound by the workgroups (sum of [4096, 8, 250] 14.1 us, 7.9 with four; argmax,
+// which does more per column, is not: [20000, 16, 77] 44 and 66).
 inline uint32_t col_width(uint64_t rows, uint64_t len, uint64_t inner, bool argmax) {
-  if (inner <= 64) return 1;
+  if (inner <= 64 || (argmax && inner < kFlatInner)) return 1;
   if (!argmax && rows * div_up(inner, 64) >= 4096) return 4;
   return rows * len * inner >= uint64_t(11) << 19 ? 4 : 1;
 }

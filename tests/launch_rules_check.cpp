@@ -85,7 +85,7 @@ static void columns() {
         for (int arg = 0; arg < 2; ++arg) {
           const bool pays = plast::flat_pays(plast::col_chunks(rows, len, inner, 1, 64, blocks), f, rows, len, inner, arg);
           CHECK(!pays || len >= 96, "short axes keep the small workgroups");
-          CHECK(!pays || rows <= 1024 || len >= 256, "rows %llu len %llu inner %llu", (unsigned long long)rows,
+          CHECK(!pays || rows <= 1024 || len >= 256 || len * inner >= 8192, "rows %llu len %llu inner %llu", (unsigned long long)rows,
                 (unsigned long long)len, (unsigned long long)inner);
         }
       }
