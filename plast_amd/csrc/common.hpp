@@ -64,13 +64,6 @@ constexpr int kBlock = 256;  // threads per workgroup for streaming kernels (4 w
 #ifndef PLAST_TAPE_SMALL
 #define PLAST_TAPE_SMALL (1u << 18)
 #endif
-// Spaces of whole 64x64 tiles always take the fixed-role tile kernel; with ragged extents, from this
-// many elements on. Config 3's chain, ragged tile / generic: [8, 301, 150] 5.82 / 4.12 us,
-// [8, 200, 301] 5.82 / 5.22, [8, 301, 301] 5.95 / 6.58, [12, 301, 301] 6.56 / 9.91,
-// [64, 513, 301] 22 / 56 us.
-#ifndef PLAST_TILE_RAGGED_MIN
-#define PLAST_TILE_RAGGED_MIN (1u << 19)
-#endif
 // Workgroup size of a tape launch that re-reads an operand (a broadcast one) from cache. Measured
 // in one process on relu(X + b) over [16384, 4096]: 256 lanes 6372 GB/s, 512 6539, 1024 6593
 // (every tape instantiation stays under 128 VGPRs, no spills); config 1's call unchanged.

@@ -152,15 +152,15 @@ __global__ __launch_bounds__((VecLaunch<Body, REUSE>::block)) void ew_vec_kernel
 // Flat kernel: the output is contiguous over the whole space, of any extents, and a lane takes four
 // consecutive elements of it wherever a row ends. Inputs contiguous the same way are read as one
 // 16-byte access; any other input (a broadcast row or column, a strided view) is gathered element
-// by element, its coordinates decoded for each with magic division. What bounds it is the
-// streaming: about 10 instructions an element and decoded axis are far under the 5 a byte the
-// issue rate allows. The generic kernel's one element per lane ran the same spaces at a quarter of
-// the copy's rate.
+// by element, its coordinates decoded for each with magic division, about 10 instructions an element
+// and decoded axis, 64-bit multiplies among them, for every operand (one that is then read as a unit
+// too: which are is only known at run time). Small spaces stay with the generic kernel
+// (flat_elementwise_pays); large ones it runs at half the copy's rate or less ([50000, 77] += a row's
+// constant: 15.4 us on the generic kernel, 9.3 here, 4.7 at the copy's rate).
 //
 // ORANK: axes outside the innermost one (0: every input contiguous; < 0: run-time count). A constant
-// count keeps the decode short and its scalar loads independent: a launch of a few thousand elements
-// lasts as long as its instruction fetches and scalar loads in series (5.4 us with a run-time
-// count unrolled to the maximum rank, measured on 646 elements, against the generic kernel's 2.8).
+// count keeps the decode short and its scalar loads independent; a run-time one costs about 1 us a
+// launch, instruction fetches and scalar loads in series.
 template <class Body, int ORANK>
 struct FlatLaunch {
   static constexpr int block = Body::kTape ? PLAST_TAPE_BLOCK : PLAST_EW_BLOCK;
@@ -667,11 +667,13 @@ bool try_tile(const Body &body, const void *const *in, void *out, const Space &s
   A.dtq = MagicDiv::make(A.tq);
   A.dtp = MagicDiv::make(A.tp);
   const bool full = A.eq % kTile == 0 && A.ep % kTile == 0;
-  if (!full && batch * A.eq * A.ep < PLAST_TILE_RAGGED_MIN) return false;
+  const bool quads = A.eq % 4 == 0 && A.ep % 4 == 0;
+  if (!tile_pays(batch * A.eq * A.ep, Body::kTape, slots, full, quads && !direct, A.eq < A.ep ? A.eq : A.ep))
+    return false;
   // the tile kernels apply the NEG rule's SIMD form to every element (a whole number of blocks)
   if (!body.index_free() && batch * A.eq * A.ep % 8 != 0) return false;
   if (full && launch_tile_fixed(A, body, roles, unsigned(blocks), lds_bytes)) return true;
-  const bool ragged = A.eq % 4 != 0 || A.ep % 4 != 0;
+  const bool ragged = !quads;
   const unsigned grid = unsigned(blocks);
   if (direct && ragged) ew_tile_kernel<Body, true, true><<<grid, kBlock, lds_bytes, stream()>>>(A, body);
   else if (direct) ew_tile_kernel<Body, true, false><<<grid, kBlock, lds_bytes, stream()>>>(A, body);
@@ -784,7 +786,7 @@ bool launch_elementwise(const Body &body, const void *const *in, void *out, Spac
   if (!small && n < (uint64_t(1) << 32) && transposed && try_tile(body, in, out, s)) return true;
 
   // --- flat path: rows that are no whole float4, over a contiguous output
-  if (!small && !transposed && n < (uint64_t(1) << 32)) {
+  if (!small && !transposed && n < (uint64_t(1) << 32) && flat_elementwise_pays(n, Body::kTape, in_ax)) {
     uint64_t want = 1;
     uint32_t contig = (2u << NIN) - 1;  // operands (output last) contiguous over the whole space
     for (int d = in_ax; d >= 0; --d) {

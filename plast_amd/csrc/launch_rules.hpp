@@ -21,6 +21,31 @@ inline uint32_t ext_row_threads(uint64_t rows, uint64_t len) {
   return blocks <= max_blocks(t > 64 ? kLongBlock : kRowsBlock) ? t : 0;
 }
 
+// ------------------------------------------------------------------------- elementwise launches
+
+// Whether a space of n elements with a transposed operand goes to the 64x64 tiles rather than to one
+// element a lane. `staged`: operands read through LDS. One, whole tiles: always. Several: a workgroup
+// stages them one after the other, 5.6 us however small the space (d += g * b, both transposed:
+// [128, 128] 5.6 us in tiles, 3.6 so, [512, 512] 5.8 and 4.9, [512, 1024] 5.9 and 6.9). Partial tiles:
+// config 3's chain [8, 301, 150] 5.82 and 4.12, [8, 301, 301] 5.95 and 6.58, [64, 513, 301] 22 and
+// 56; of whole float4 units with nothing read past LDS (`quads`), over extents that fill a tile: exp
+// of [600, 600] 4.5 and 4.6, of [700, 700] 4.6 and 5.0, but of [100000, 4] 5.6 and 3.1.
+inline bool tile_pays(uint64_t n, bool tape, uint32_t staged, bool full, bool quads, uint64_t least_extent) {
+  if (staged > 1 && !tape) return n >= uint64_t(1) << 19;
+  return full || n >= (quads && !tape && least_extent >= 64 ? uint64_t(3) << 17 : uint64_t(1) << 19);
+}
+
+// Whether a contiguous output whose rows are no whole float4 goes to the flat kernel rather than to one
+// element a lane, `outer` axes decoded outside the innermost one. Fixed bodies, a row added:
+// [30000, 77] 3.5 us flat and 3.4, [400000 / 77, 77] 3.7 and 3.8, [1.2M / 77, 77] 4.4 and 5.1; three
+// outer axes: 0.3M elements 4.6 and 3.7, 1.2M 6.0 and 5.8, 4.9M 13.9 and 15.4. Fused chains beyond the
+// smallest (which never come here) gain from it at once, with three outer axes from 1.3M elements:
+// 0.4M 6.9 and 4.9, 1.1M 8.5 and 7.9, 1.5M 8.8 and 9.5.
+inline bool flat_elementwise_pays(uint64_t n, bool tape, int outer) {
+  if (tape) return outer < 3 || n >= uint64_t(5) << 18;
+  return n >= (outer < 3 ? uint64_t(3) << 17 : uint64_t(3) << 20);
+}
+
 // ------------------------------------------------------------------------- leading-axis reductions
 // A reduction of [rows, len, inner] over len, the `inner` columns kept.
 

@@ -91,8 +91,33 @@ static void columns() {
       }
 }
 
+// Elementwise launches: a small space never pays for a workgroup's staging, a large one always leaves
+// the one-element-a-lane kernel, and each rule keeps its side once a space has grown past it.
+static void elementwise() {
+  for (int tape = 0; tape < 2; ++tape) {
+    for (int outer = 0; outer < 6; ++outer) {
+      bool was = false;
+      for (u64 n = 1; n < k32; n = n * 5 / 4 + 1) {
+        const bool pays = plast::flat_elementwise_pays(n, tape, outer);
+        CHECK(pays || !was, "n %llu", (unsigned long long)n);
+        CHECK(tape || !pays || n > 300000, "n %llu", (unsigned long long)n);
+        CHECK(pays || n < 4000000, "n %llu", (unsigned long long)n);
+        was = pays;
+      }
+    }
+    for (uint32_t staged = 1; staged < 4; ++staged)
+      for (int form = 0; form < 4; ++form)
+        for (u64 n = 1; n < k32; n = n * 5 / 4 + 1) {
+          const bool pays = plast::tile_pays(n, tape, staged, form & 1, form & 2, n < 64 ? n : 64);
+          CHECK(pays || n < 600000, "n %llu", (unsigned long long)n);
+          CHECK(!pays || n > 390000 || ((form & 1) && (staged == 1 || tape)), "n %llu", (unsigned long long)n);
+        }
+  }
+}
+
 int main() {
   ext_rows();
+  elementwise();
   columns();
   if (!g_fail) std::printf("ok\n");
   return g_fail;
