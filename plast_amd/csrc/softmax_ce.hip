@@ -203,6 +203,16 @@ constexpr uint32_t kWaveRow = 2048;  // the longest: 64 lanes of 8 units
 // [16384, 1000] 66.5 / 69.8, and with both in 8 units [30000, 1500] 185 / 163; backward [60000, 600]
 // 145 / 157, [60000, 700] 169 / 171, [16384, 1000] 70.2 / 66.5.
 constexpr uint32_t kSoftmaxWaveRow = 1024, kSoftmaxBwdWaveRow = 768;
+// and with fewer rows than these, which leave the chip idle: a lane of a wave's row has 16 elements to
+// exponentiate one after the other, of a workgroup's four (one where a short row is no whole float4:
+// the three-pass kernel, its row in the caches). Wave / workgroup per row: forward [64, 300] 4.8 / 4.0 us,
+// [1500, 300] 5.3 / 5.0, [3000, 300] 5.8 / 6.6, [2048, 1000] 6.4 / 6.3, [3000, 1000] 7.4 / 8.3; log-softmax
+// [1024, 300] 5.0 / 4.5, [2048, 300] 5.1 / 5.5; backward [64, 128] 3.9 / 3.5, [1500, 128] 4.2 / 4.3,
+// [64, 3] 4.2 / 3.5, [1500, 256] 4.3 / 4.7; log-softmax's [64, 512] 4.4 / 3.5, [2048, 512] 5.3 / 5.8.
+template <bool LOG>
+constexpr uint64_t kSoftmaxFewRows = LOG ? 1536 : 2048;
+template <bool LOG>
+constexpr uint64_t kSoftmaxBwdFewRows = LOG ? 1700 : 1280;
 template <uint32_t MAX_ROW, class F>
 void with_row_lanes(uint32_t C, F &&f) {
   using std::integral_constant;
@@ -1708,7 +1718,7 @@ void softmax_forward(const Tensor **inputs, Tensor *output, KernelParams params,
   const uint64_t R = max_blocks(kCeBlock);
   const float *px0 = static_cast<const float *>(x->data);
   float *py0 = static_cast<float *>(output->data);
-  if (C <= kSoftmaxWaveRow) {
+  if (C <= kSoftmaxWaveRow && N >= kSoftmaxFewRows<LOG>) {
     for (uint64_t r0 = 0; r0 < N; r0 += R) {
       const uint64_t n = N - r0 < R ? N - r0 : R;
       with_row_lanes<kSoftmaxWaveRow>(C, [&](auto lanes, auto units) {
@@ -1724,8 +1734,9 @@ void softmax_forward(const Tensor **inputs, Tensor *output, KernelParams params,
   // float4 units per lane for a register-resident row (0: the three-pass kernel)
   int V = 0;
   const bool ragged = C % 4 != 0 || !aligned16(px0) || !aligned16(py0);
-  for (int v = 1; v <= 32 && !V; v *= 2)
-    if (uint64_t(C) <= uint64_t(kSoftmaxBlock) * 4 * v) V = v;
+  if (!ragged || C > kCeBlock)  // (else a lane has one element at most: the three-pass kernel)
+    for (int v = 1; v <= 32 && !V; v *= 2)
+      if (uint64_t(C) <= uint64_t(kSoftmaxBlock) * 4 * v) V = v;
   // long rows of whole float4: the persistent form (rows at a time below 2^31)
   constexpr int SV = 8;
   if (!ragged && C >= PLAST_SOFTMAX_PERSISTENT && C <= uint32_t(kStepBlock) * 4 * SV &&
@@ -1745,6 +1756,7 @@ void softmax_forward(const Tensor **inputs, Tensor *output, KernelParams params,
       else softmax_fwd_reg_kernel<LOG, U, false><<<n, kSoftmaxBlock, 0, stream()>>>(px, py, C);
     };
     switch (V) {
+      case 1: reg(std::integral_constant<int, 1>{}); break;
       case 2: reg(std::integral_constant<int, 2>{}); break;
       case 4: reg(std::integral_constant<int, 4>{}); break;
       case 8: reg(std::integral_constant<int, 8>{}); break;
@@ -1775,14 +1787,15 @@ void softmax_backward(Tensor **inputs, const Tensor *output, KernelParams params
   int V = 0;
   const bool ragged = C % 4 != 0 || !aligned16(output->data) || !aligned16(output->grad->data) ||
                       !aligned16(x->grad->data);
-  for (int v = 1; v <= 16 && !V && v * BS <= 8192; v *= 2)
-    if (uint64_t(C) <= uint64_t(BS) * 4 * v) V = v;
+  if (!ragged || C > kCeBlock)
+    for (int v = 1; v <= 16 && !V && v * BS <= 8192; v *= 2)
+      if (uint64_t(C) <= uint64_t(BS) * 4 * v) V = v;
   for (uint64_t r0 = 0; r0 < N; r0 += R) {
     const unsigned n = unsigned(N - r0 < R ? N - r0 : R);
     const float *py = static_cast<const float *>(output->data) + r0 * C;
     const float *pg = static_cast<const float *>(output->grad->data) + r0 * C;
     float *pd = static_cast<float *>(x->grad->data) + r0 * C;
-    if (C <= kSoftmaxBwdWaveRow) {
+    if (C <= kSoftmaxBwdWaveRow && N >= kSoftmaxBwdFewRows<LOG>) {
       with_row_lanes<kSoftmaxWaveRow>(C, [&](auto lanes, auto units) {
         constexpr int L = decltype(lanes)::value, U = decltype(units)::value;
         softmax_bwd_rows_kernel<LOG, L, U>
