@@ -859,6 +859,7 @@ __global__ __launch_bounds__(kStepBlock) void ce_step_kernel(
   // the workgroup's column sums: partial row b of part, in dispatch order under the dynamic
   // order (the rows each workgroup took vary from run to run) and by the static schedule's
   // numbering otherwise
+  if (!part) return;
   float *pb = part + uint64_t(DYN ? blockIdx.x : row_block()) * C;
 #pragma unroll
   for (int u = 0; u < V; ++u) {
@@ -1071,6 +1072,7 @@ __global__ __launch_bounds__(64 * kStepRowsWaves<U>) void ce_step_rows_kernel(
     load(gr + 2 * step, va, ya, ga);
     if (gr + step < groups) process(gr + step, vb, yb, gb);
   }
+  if (!part) return;
   // the wave's rows: lanes with the same l
 #pragma unroll
   for (int m = L; m < 64; m <<= 1)
@@ -1149,12 +1151,19 @@ void ce_step_launch_v(int want, unsigned grid, float *part, const float *logits,
                                                 uint32_t(simd_end(N)));
     };
     // the dynamic row order unless results must not depend on timing (plast_hip_set_deterministic);
-    // rows that are no whole float4 always keep the static one, as their bias gradient has been the
-    // same bits on every call
+    // rows that are no whole float4 and short ones always keep the static one, as their bias gradient
+    // has been the same bits on every call
     if (C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits)) run(std::false_type{}, std::true_type{});
-    else if (deterministic()) run(std::false_type{}, std::false_type{});
+    else if (deterministic() || C <= kWaveRow) run(std::false_type{}, std::false_type{});
     else run(std::true_type{}, std::false_type{});
   }
+}
+
+// Whether the step's rows share waves (ce_step_rows_kernel): rows up to kWaveRow, but for so few that
+// each CU has one at most, which a workgroup per row does in one round ([64, 10] 7.4 us, 9.7 in
+// waves, [256, 1000] 9.0 and 9.8, [16, 2048] 7.2 and 11.7; [400, 300] 10.2 and 9.9).
+bool step_in_waves(uint64_t N, uint64_t C) {
+  return C <= kWaveRow && (C < 4 || N > uint64_t(num_cus()));
 }
 
 // The one-pass step's arguments: -1 (after reporting) when unusable, 0 when the rows need the three
@@ -1176,7 +1185,7 @@ int ce_step_form(const float *logits, const int32_t *labels, const float *dloss,
   }
   // the column sums live in LDS (one float4 slot per lane and unit, the row's plus padding): the
   // kernel must be allowed that much of it
-  if (C <= kWaveRow) return 1;  // ce_step_rows_kernel
+  if (step_in_waves(N, C)) return 1;
   if (C <= kStepMaxC) return ce_step_units<1>(C);
   return 0;
 }
@@ -1187,7 +1196,7 @@ int ce_step_form(const float *logits, const int32_t *labels, const float *dloss,
 // sums for (kScratchFloats / C; on MI355X, 256 CUs of rows up to 32768 floats, never binding).
 uint64_t ce_step_grid(uint64_t N, uint64_t C) {
   uint64_t grid = uint64_t(num_cus()) * PLAST_CE_STEP_WPC;
-  if (C <= kWaveRow) {
+  if (step_in_waves(N, C)) {
     // four row groups per workgroup before another one is added: each adds a row to the tail's sum
     uint64_t rows = 1;
     with_row_lanes<kWaveRow>(uint32_t(C), [&](auto lanes, auto) { rows = 4 * (64 / decltype(lanes)::value); });
@@ -1215,7 +1224,8 @@ void ce_step_launch(int V, unsigned grid, float *part, const float *logits, cons
                     const float *dloss, float *stats, float *loss, float *dlogits, float *dbias,
                     float *mean_loss, uint64_t N, uint64_t C) {
   const uint32_t c32 = uint32_t(C);
-  if (C <= kWaveRow)
+  if (!dbias) part = nullptr;  // the kernels then leave their sums where they are
+  if (step_in_waves(N, C))
     with_row_lanes<kWaveRow>(c32, [&](auto lanes, auto units) {
       constexpr int L = decltype(lanes)::value, U = decltype(units)::value;
       ce_step_rows_kernel<L, U><<<grid, 64 * kStepRowsWaves<U>, 0, stream()>>>(
@@ -1922,6 +1932,7 @@ void softmax_cross_entropy_step_hip(const float *logits, const int32_t *labels, 
   }
   const int V = ce_step_form(logits, labels, dloss, stats, loss, dlogits, N, C, where);
   if (V < 0) return;
+  const bool whole = C % 4 == 0 && aligned16(logits) && aligned16(dlogits);
   if (V == 0) {
     // any other row: the forward, the overwriting backward and the column sum as three passes
     Tensor tx, tl, ts, to, tg, tdx;
@@ -1955,8 +1966,7 @@ void softmax_cross_entropy_step_hip(const float *logits, const int32_t *labels, 
     return;
   }
   const uint64_t grid = ce_step_grid(N, C);
-  // the workgroups' column sums (written even when no bias gradient is wanted; then unread)
-  const bool whole = C % 4 == 0 && aligned16(logits) && aligned16(dlogits);
+  // the workgroups' column sums
   // (rows that are no whole float4 were three passes once, which a capture took without workspace)
   float *part = static_cast<float *>(whole ? workspace(sizeof(float) * grid * C)
                                            : partials(sizeof(float) * grid * C, where));

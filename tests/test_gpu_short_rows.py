@@ -56,6 +56,28 @@ def test_step(N, C, special):
     step_case(N, C, special)
 
 
+@pytest.mark.parametrize("special", [False, True], ids=["clean", "special_rows"])
+@pytest.mark.parametrize("N, C", [(255, 10), (256, 10), (257, 10), (258, 4), (259, 5), (260, 33), (261, 130),
+                                  (262, 300), (263, 513), (264, 1025), (256, 2048), (257, 2048)])
+def test_step_row_counts(N, C, special):
+    """Each side of one row per CU (256), beyond which short rows share waves."""
+    step_case(N, C, special)
+
+
+def test_short_step_repeats():
+    """The bias gradient of short rows is the same bits on every call, with a workgroup per row too."""
+    from plast_amd import runtime as rt
+    rng = np.random.RandomState(9)
+    for N, C in ((200, 2048), (37, 12)):
+        x, lab = (rng.randn(N, C) * 2).astype(np.float32), rng.randint(0, C, N).astype(np.int32)
+        X, Lb = rt.DeviceTensor.from_numpy(x), rt.DeviceTensor.from_numpy(lab)
+        g = np.full(N, 1.0 / N, np.float32)
+        first = _step(rt, X, Lb, g)
+        for _ in range(20):
+            for a, b in zip(_step(rt, X, Lb, g), first):
+                assert_bits(a, b, "a later call")
+
+
 @pytest.mark.parametrize("N, C", [(40000, 12), (20000, 77), (6000, 700), (3000, 2000), (1100, 2051)])
 def test_step_many_rows(N, C):
     """Several row groups per wave: every row against the oracle, the same bits twice for short rows."""
@@ -86,21 +108,85 @@ def test_softmax_rows(C, log):
     softmax_case((23, C), log)
 
 
-@pytest.mark.parametrize("off", [1, 2])
-@pytest.mark.parametrize("C", [100, 2052, 17000])
-def test_misaligned_rows(C, off):
-    """Rows of whole float4 in a buffer that does not start on one: the bits of the aligned call for
-    short rows, the fp64 softmax for the others (a longer row's kernel differs)."""
-    from plast_amd import runtime as rt
+@pytest.mark.parametrize("log", [False, True], ids=["softmax", "log_softmax"])
+@pytest.mark.parametrize("C", [c for c in ROW if c <= 1025] + [767, 768, 769])
+def test_softmax_many_rows(C, log):
+    """Rows enough for a wave each, or a share of one."""
+    softmax_case((2101, C), log)
+
+
+@pytest.mark.parametrize("log", [False, True], ids=["softmax", "log_softmax"])
+@pytest.mark.parametrize("N", [1279, 1280, 1535, 1536, 1699, 1700, 2047, 2048])
+def test_softmax_row_counts(N, log):
+    """Each side of the row counts where a wave takes over from a workgroup."""
+    softmax_case((N, 77), log)
+    softmax_case((N, 300), log)
+
+
+def _offset(rt, x, off):
+    """x at `off` floats past a 16-byte boundary."""
+    base = rt.DeviceTensor.from_numpy(np.concatenate([np.zeros(off, np.float32), x.ravel()]))
+    return rt.DeviceTensor(x.shape, base=base, offset=off, zero=False)
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+@pytest.mark.parametrize("N, C", [(7, 100), (2100, 100), (7, 2052), (7, 17000)])
+def test_misaligned_rows(N, C, off):
+    """Rows of whole float4 in buffers that do not start on one, forward and backward: the bits of the
+    aligned call where the rows are a wave's or share one (any alignment is the same kernel), the fp64
+    softmax for the others (1e-5 of each value and of its gradient's terms)."""
+    from plast_amd import abi, runtime as rt
     from plast_amd.abi import KernelParams
-    N = 7
     print(f"softmax {N}x{C} offset {off}", flush=True)
-    x = np.random.RandomState(C + off).randn(N * C + off).astype(np.float32)
-    X, Y = rt.DeviceTensor.from_numpy(x), rt.DeviceTensor((N * C + 4,), zero=False)
-    vx = rt.DeviceTensor((N, C), base=X, offset=off, zero=False)
-    vy = rt.DeviceTensor((N, C), base=Y, offset=4 - off, zero=False)
-    rt.forward("softmax", [vx], vy, KernelParams(1, 0, 0.0))
-    h = x[off:].reshape(N, C).astype(np.float64)
+    rng = np.random.RandomState(C + off)
+    x, dy, d0 = (rng.randn(N, C).astype(np.float32) for _ in range(3))
+    p = KernelParams(1, 0, 0.0)
+
+    def run(at):
+        X, Y, DY, D = _offset(rt, x, at), _offset(rt, np.zeros_like(x), (4 - at) % 4), _offset(rt, dy, at), _offset(rt, d0, at)
+        tx = abi.make_tensor(X.ptr, x.shape, None, rt.FLOAT32, rt.GPU, True, D.t)
+        ty = abi.make_tensor(Y.ptr, x.shape, None, rt.FLOAT32, rt.GPU, True, DY.t)
+        rt.forward("softmax", [tx], ty, p)
+        rt.backward("softmax", [tx], ty, p)
+        return Y.numpy(), D.numpy()
+    y, d = run(off)
+    h = x.astype(np.float64)
     e = np.exp(h - h.max(1, keepdims=True))
     want = e / e.sum(1, keepdims=True)
-    assert np.all(np.abs(vy.numpy() - want) <= 1e-5 * want)
+    assert np.all(np.abs(y - want) <= 1e-5 * want)
+    t = dy * want
+    term = want * (dy - t.sum(1, keepdims=True))
+    scale = np.abs(d0) + want * (np.abs(dy) + np.abs(t).sum(1, keepdims=True))
+    assert np.all(np.abs(d - (d0 + term)) <= 1e-5 * scale)
+    if N > 2047 and C <= 768:
+        for a, b in zip((y, d), run(0)):
+            assert_bits(a, b, "aligned")
+
+
+@pytest.mark.parametrize("off", [1, 2, 3])
+@pytest.mark.parametrize("N, C", [(300, 100), (9, 100), (40, 2052), (12, 8192)])
+def test_misaligned_cross_entropy(N, C, off):
+    """The step and the op's backward over rows of whole float4 that start off a 16-byte boundary."""
+    from plast_amd import abi, runtime as rt
+    print(f"ce {N}x{C} offset {off}", flush=True)
+    rng = np.random.RandomState(C + off)
+    x = (rng.randn(N, C) * 2).astype(np.float32)
+    _special_rows(x)
+    lab = rng.randint(0, C, N).astype(np.int32)
+    g = rng.uniform(0.1, 1.0, N).astype(np.float32)
+    wst, wloss, wdx = _oracle(x, lab, g)
+    X, DX = _offset(rt, x, off), _offset(rt, np.zeros_like(x), off)
+    Lb, G = rt.DeviceTensor.from_numpy(lab), rt.DeviceTensor.from_numpy(g)
+    st, loss, db = rt.DeviceTensor((N, 2)), rt.DeviceTensor((N,)), rt.DeviceTensor((C,))
+    L = rt.lib()
+    L.softmax_cross_entropy_step_hip(X.ptr, Lb.ptr, G.ptr, st.ptr, loss.ptr, DX.ptr, db.ptr, None, N, C)
+    L.check("step")
+    check_ce_rows(x, lab, g, st.numpy(), loss.numpy(), DX.numpy(), wst, wloss, wdx, 1e-2 * g)
+    ok = np.isfinite(wdx).all(0)
+    bar = 1e-5 * np.abs(wdx.astype(np.float64)).sum(0) + 1e-12
+    assert np.all(np.abs(db.numpy() - wdx.astype(np.float64).sum(0))[ok] <= bar[ok])
+    D = _offset(rt, np.zeros_like(x), (off + 1) % 4)
+    tx = abi.make_tensor(X.ptr, x.shape, None, rt.FLOAT32, rt.GPU, True, D.t)
+    out = abi.make_tensor(loss.ptr, (N,), None, rt.FLOAT32, rt.GPU, True, G.t)
+    rt.backward("softmax_cross_entropy", [tx, Lb, st], out)
+    check_ce_rows(x, lab, g, st.numpy(), loss.numpy(), D.numpy(), wst, wloss, wdx, 1e-2 * g)
