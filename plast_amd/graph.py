@@ -32,7 +32,7 @@ class Graph:
 
         self._alloc_cb = abi.ArenaAllocFn(alloc)
         self.dag = None
-        self._run = None      # the DAG's calls, bound by build()
+        self._run = None      # what _bound() made of the DAG
 
     # --- construction
     def node(self, op: str, inputs, output: DeviceTensor, p: KernelParams | None = None) -> DeviceTensor:
@@ -92,19 +92,28 @@ class Graph:
     def _calls(self):
         """(forward slot, backward slot, inputs, output, params) of every node of the DAG, in order:
         the objects ctypes would otherwise make anew for each field on every pass (2 us a node of
-        the 5 a small pass took). `inputs`, `output` and `params` read the node itself, so a node
-        changed after build() is run as changed; its slots are taken at build()."""
+        the 5 a small pass took). Each lies over the node's own memory, its slots included, so a
+        node changed after build() is run as changed."""
+        slot = abi.Node.op.offset
         calls = []
         for i in range(self.dag.count):
             n = self.dag.nodes[i].contents
-            calls.append((C.cast(n.op.gpu_forward, abi.ForwardKernel),
-                          C.cast(n.op.gpu_backward, abi.BackwardKernel), n.inputs, n.output, n.params))
+            calls.append((abi.ForwardKernel.from_buffer(n, slot + abi.Op.gpu_forward.offset),
+                          abi.BackwardKernel.from_buffer(n, slot + abi.Op.gpu_backward.offset),
+                          n.inputs, n.output, n.params))
         return calls
 
     def _bound(self):
-        if self._run is None or len(self._run) != self.dag.count:
-            self._run = self._calls()
-        return self._run
+        """The calls, bound on the first pass and again when the DAG holds other nodes: its head (the
+        node array and the count) and the array are compared with what they held then."""
+        run = self._run
+        if run is None or run[0] is not self.dag or run[1].raw != run[2] or run[3].raw != run[4]:
+            dag = self.dag
+            head = (C.c_char * abi.DAG.capacity.offset).from_buffer(dag)
+            size = dag.count * C.sizeof(C.c_void_p)
+            nodes = (C.c_char * size).from_address(C.addressof(dag.nodes.contents)) if size else (C.c_char * 0)()
+            run = self._run = dag, head, head.raw, nodes, nodes.raw, self._calls()
+        return run[5]
 
     def forward(self) -> None:
         """dag_forward (graph.c:57-60): each node's GPU forward slot in order."""
