@@ -54,7 +54,6 @@ void fused_elementwise_hip_forward(const Tensor **inputs, Tensor *output, Kernel
   Space s;
   init_space(s, output->shape, int(output->ndim));
   const void *ins[PLAST_TAPE_MAX_INPUTS];
-  bool all_contig = contiguous(output);
   for (uint32_t k = 0; k < tape->num_inputs; ++k) {
     if (!covers(inputs[k], output->shape, int(output->ndim))) {
       // broadcast inputs are fine; shapes that do not broadcast are not
@@ -64,9 +63,7 @@ void fused_elementwise_hip_forward(const Tensor **inputs, Tensor *output, Kernel
         report_error(where, "input %u does not broadcast to the output", k);
         return;
       }
-      all_contig = false;
     }
-    all_contig = all_contig && contiguous(inputs[k]);
     set_operand(s, int(k), inputs[k]);
     ins[k] = inputs[k]->data;
   }
@@ -84,7 +81,6 @@ void fused_elementwise_hip_forward(const Tensor **inputs, Tensor *output, Kernel
     if (in_ok && out_ok) neg_simd |= 1u << i;
   }
   const uint64_t se = simd_end(n);
-  (void)all_contig;
   switch (tape_ops_class(*tape)) {
   case kTapeArith: launch_tape<kTapeArith>(*tape, se, neg_simd, nin, ins, output->data, s, where); break;
   case kTapeExp: launch_tape<kTapeExp>(*tape, se, neg_simd, nin, ins, output->data, s, where); break;

@@ -1990,8 +1990,8 @@ void softmax_cross_entropy_step_noalloc_hip(const float *logits, const int32_t *
   const int V = ce_step_form(logits, labels, dloss, stats, loss, dlogits, N, C, where);
   if (V < 0) return;
   if (V == 0 || C % 4 != 0 || !aligned16(logits) || !aligned16(dlogits)) {
-    report_error(where, "rows of %llu floats are not one-pass rows (whole float4, 16-byte aligned "
-                 "logits and dlogits, at most %llu floats): the three-pass form allocates",
+    report_error(where, "rows of %llu floats are not one-pass rows of this call, which takes whole "
+                 "float4, 16-byte aligned logits and dlogits and at most %llu floats",
                  (unsigned long long)C, (unsigned long long)kStepMaxC);
     return;
   }

@@ -48,7 +48,7 @@ def _read(ptr, index, dtype=np.float32):
     return out
 
 
-@pytest.mark.parametrize("C_", [4, 3], ids=["wave-per-row", "workgroup-per-row"])
+@pytest.mark.parametrize("C_", [4, 3], ids=["rows-of-4", "rows-of-3"])
 def test_ce_rows_beyond_one_launch(C_):
     from plast_amd import ops
     rt = _rt()
