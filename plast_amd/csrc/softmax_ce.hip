@@ -204,15 +204,38 @@ constexpr uint32_t kWaveRow = 2048;  // the longest: 64 lanes of 8 units
 // 145 / 157, [60000, 700] 169 / 171, [16384, 1000] 70.2 / 66.5.
 constexpr uint32_t kSoftmaxWaveRow = 1024, kSoftmaxBwdWaveRow = 768;
 // and with fewer rows than these, which leave the chip idle: a lane of a wave's row has 16 elements to
-// exponentiate one after the other, of a workgroup's four (one where a short row is no whole float4:
-// the three-pass kernel, its row in the caches). Wave / workgroup per row: forward [64, 300] 4.8 / 4.0 us,
-// [1500, 300] 5.3 / 5.0, [3000, 300] 5.8 / 6.6, [2048, 1000] 6.4 / 6.3, [3000, 1000] 7.4 / 8.3; log-softmax
-// [1024, 300] 5.0 / 4.5, [2048, 300] 5.1 / 5.5; backward [64, 128] 3.9 / 3.5, [1500, 128] 4.2 / 4.3,
-// [64, 3] 4.2 / 3.5, [1500, 256] 4.3 / 4.7; log-softmax's [64, 512] 4.4 / 3.5, [2048, 512] 5.3 / 5.8.
+// exponentiate one after the other, of a workgroup's four. Wave / workgroup per row: forward [64, 300]
+// 4.8 / 4.0 us, [1500, 300] 5.3 / 5.0, [3000, 300] 5.8 / 6.6, [2048, 1000] 6.4 / 6.3, [3000, 1000]
+// 7.4 / 8.3; log-softmax [1024, 300] 5.0 / 4.5, [2048, 300] 5.1 / 5.5.
 template <bool LOG>
 constexpr uint64_t kSoftmaxFewRows = LOG ? 1536 : 2048;
+// The backward's, in whole 128-byte lines, wave / workgroup: [64, 128] 3.1 / 2.6, [1024, 128] 3.2 / 3.1,
+// [2048, 128] 3.2 / 3.9, [1500, 256] 4.3 / 4.7; log-softmax's [64, 512] 4.4 / 3.5, [2048, 512] 5.3 / 5.8. Where
+// rows share lines, workgroups of other XCDs update them at once, and a wave's neighbours are its own:
+// [64, 4] 2.9 / 4.0, [64, 300] 3.3 / 3.3, [1024, 300] 3.5 / 4.1; log-softmax's [64, 300] 3.6 / 3.3, [1024, 300]
+// 3.9 / 4.2. Rows that are no whole float4 (the workgroup's three passes): [2400, 10] 3.2 / 3.7, [4096, 3]
+// 3.8 / 4.3, [2048, 301] 4.3 / 4.1, [2400, 514] 5.4 / 5.7; log-softmax's [2048, 514] 5.4 / 4.6, [3000, 129]
+// 4.9 / 4.4, [3000, 301] 5.4 / 5.2, [4096, 301] 5.7 / 5.9, [3000, 514] 6.3 / 6.8.
 template <bool LOG>
-constexpr uint64_t kSoftmaxBwdFewRows = LOG ? 1700 : 1280;
+bool softmax_bwd_waves(uint64_t N, uint64_t C) {
+  if (C > kSoftmaxBwdWaveRow) return false;
+  if (C % 4 != 0) return N >= (LOG ? 3072 : 2176);
+  if (C % 32 != 0) return !LOG || C <= 16 || N >= 768;
+  return N >= (LOG ? 1700 : 1280);
+}
+// Rows that are no whole float4 and no longer than this take the forward's three passes rather than a
+// workgroup's registers, of whose lanes they leave most idle: [1024, 301] 4.1 / 4.5 us, [1024, 514]
+// 4.7 / 4.6.
+constexpr uint32_t kSoftmaxPasses = 2 * kCeBlock;
+// The backward's, whose 512 lanes have twice as many idle: rows that are all resident at once (2048
+// workgroups), and more of short ones while the tensors stay in the caches. Three passes / registers:
+// [512, 1001] 4.1 / 4.1, [1024, 301] 3.5 / 4.5, [2048, 1001] 6.7 / 7.6, [2400, 1001] 9.1 / 8.6;
+// [1024, 1301] 5.2 / 5.3, [2048, 1301] 7.9 / 8.6, [2048, 1602] 10.3 / 10.1, [512, 1301] 4.6 / 4.3; [4096, 770]
+// 10.3 / 11.5, [8192, 901] 21.2 / 21.2, [8192, 1021] 26.5 / 22.4, [30000, 770] 71.6 / 64.8.
+bool softmax_bwd_passes(uint64_t N, uint64_t C) {
+  if (N <= 2048) return C <= (N > 1024 ? 1344u : 1024u);
+  return C <= 900 && N * C < uint64_t(1) << 23;
+}
 template <uint32_t MAX_ROW, class F>
 void with_row_lanes(uint32_t C, F &&f) {
   using std::integral_constant;
@@ -1207,8 +1230,6 @@ uint64_t ce_step_grid(uint64_t N, uint64_t C) {
   return N < grid ? N : grid;
 }
 
-// The one-pass step over `grid` workgroups with their column sums in part[grid][C], then the tail:
-// their sum into dbias and the loss's mean, as wanted.
 // The step's tail: dbias from the column sums part[G][C] when dbias is wanted, and the mean of
 // loss[0 .. N) when mean_loss is; one launch, or none when neither is wanted.
 void step_tail(const float *part, float *dbias, uint64_t C, unsigned G, const float *loss,
@@ -1220,6 +1241,8 @@ void step_tail(const float *part, float *dbias, uint64_t C, unsigned G, const fl
                                                              mean_loss, uint32_t(N));
 }
 
+// The one-pass step over `grid` workgroups with their column sums in part[grid][C], then the tail:
+// their sum into dbias and the loss's mean, as wanted.
 void ce_step_launch(int V, unsigned grid, float *part, const float *logits, const int32_t *labels,
                     const float *dloss, float *stats, float *loss, float *dlogits, float *dbias,
                     float *mean_loss, uint64_t N, uint64_t C) {
@@ -1744,7 +1767,7 @@ void softmax_forward(const Tensor **inputs, Tensor *output, KernelParams params,
   // float4 units per lane for a register-resident row (0: the three-pass kernel)
   int V = 0;
   const bool ragged = C % 4 != 0 || !aligned16(px0) || !aligned16(py0);
-  if (!ragged || C > kCeBlock)  // (else a lane has one element at most: the three-pass kernel)
+  if (!ragged || C > kSoftmaxPasses)
     for (int v = 1; v <= 32 && !V; v *= 2)
       if (uint64_t(C) <= uint64_t(kSoftmaxBlock) * 4 * v) V = v;
   // long rows of whole float4: the persistent form (rows at a time below 2^31)
@@ -1797,7 +1820,7 @@ void softmax_backward(Tensor **inputs, const Tensor *output, KernelParams params
   int V = 0;
   const bool ragged = C % 4 != 0 || !aligned16(output->data) || !aligned16(output->grad->data) ||
                       !aligned16(x->grad->data);
-  if (!ragged || C > kCeBlock)
+  if (!ragged || !softmax_bwd_passes(N, C))
     for (int v = 1; v <= 16 && !V && v * BS <= 8192; v *= 2)
       if (uint64_t(C) <= uint64_t(BS) * 4 * v) V = v;
   for (uint64_t r0 = 0; r0 < N; r0 += R) {
@@ -1805,7 +1828,7 @@ void softmax_backward(Tensor **inputs, const Tensor *output, KernelParams params
     const float *py = static_cast<const float *>(output->data) + r0 * C;
     const float *pg = static_cast<const float *>(output->grad->data) + r0 * C;
     float *pd = static_cast<float *>(x->grad->data) + r0 * C;
-    if (C <= kSoftmaxBwdWaveRow && N >= kSoftmaxBwdFewRows<LOG>) {
+    if (softmax_bwd_waves<LOG>(N, C)) {
       with_row_lanes<kSoftmaxWaveRow>(C, [&](auto lanes, auto units) {
         constexpr int L = decltype(lanes)::value, U = decltype(units)::value;
         softmax_bwd_rows_kernel<LOG, L, U>
@@ -1967,7 +1990,7 @@ void softmax_cross_entropy_step_hip(const float *logits, const int32_t *labels, 
   }
   const uint64_t grid = ce_step_grid(N, C);
   // the workgroups' column sums
-  // (rows that are no whole float4 were three passes once, which a capture took without workspace)
+  // (a capture of rows that are no whole float4 needs no workspace sized before it)
   float *part = static_cast<float *>(whole ? workspace(sizeof(float) * grid * C)
                                            : partials(sizeof(float) * grid * C, where));
   if (!part) return;

@@ -123,6 +123,17 @@ def test_softmax_row_counts(N, log):
     softmax_case((N, 300), log)
 
 
+@pytest.mark.parametrize("log", [False, True], ids=["softmax", "log_softmax"])
+@pytest.mark.parametrize("N, C", [(2175, 3), (2176, 301), (3071, 301), (3072, 3), (300, 511), (300, 514),
+                                  (1024, 1023), (1025, 1026), (1025, 1343), (1025, 1345), (2048, 1022),
+                                  (2049, 1022), (10894, 770), (10895, 770), (9, 4), (9, 16), (9, 20),
+                                  (767, 20), (768, 300), (767, 300)])
+def test_softmax_lines(N, C, log):
+    """Each side of the lines between three passes, a wave and a workgroup's registers: rows that are
+    no whole float4, and rows that share a 128-byte line with their neighbours."""
+    softmax_case((N, C), log)
+
+
 def _offset(rt, x, off):
     """x at `off` floats past a 16-byte boundary."""
     base = rt.DeviceTensor.from_numpy(np.concatenate([np.zeros(off, np.float32), x.ravel()]))
