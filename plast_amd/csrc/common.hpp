@@ -84,7 +84,10 @@ constexpr int kBlock = 256;  // threads per workgroup for streaming kernels (4 w
 #define PLAST_ROW_WAVES 2048
 #endif
 // The same where several axes are reduced, whose runs are shorter and decoded one by one: config 3's
-// B gradient (512 outputs, 268 MB) 54.6 us with 2048 segments, 45.0 with 4096, 45.7 with 8192.
+// B gradient (512 outputs, 268 MB) 51.4 us with 2048 segments, 44.1 with 4096, 45.1 with 8192, of a
+// multiplied one 86.7, 84.0, 85.5. Larger ones go either way: over [128, 1024, 196] 24.4, 21.5, 22.0
+// and multiplied 36.5, 39.7, 39.6, over [500, 10, 30000] 110, 103, 96 and 200, 204, 186; smaller ones
+// are the same with each.
 #ifndef PLAST_MULTI_WAVES
 #define PLAST_MULTI_WAVES 4096
 #endif
@@ -122,8 +125,8 @@ constexpr int kBlock = 256;  // threads per workgroup for streaming kernels (4 w
 #define PLAST_COL_FIN_Q 16
 #endif
 // Small leading-axis sums (at most PLAST_COL_SMALL_MAX input elements) in one launch: workgroups
-// of PLAST_COL_SMALL_S4 float4 columns (PLAST_COL_SMALL_S4_3 for three operands and more) that
-// walk every row, instead of row chunks plus a finalize; PLAST_COL_SMALL3 = 0 sends three-operand
+// of PLAST_COL_SMALL_S4 float4 columns (PLAST_COL_SMALL_S4_3 for three operands and more, and for two
+// over narrow rows: col_small_one) that walk every row, over the sizes of col_slices, instead of row chunks plus a finalize; PLAST_COL_SMALL3 = 0 sends three-operand
 // producers to the chunked pass, whose chunks keep at least PLAST_COL_MIN_ROWS3 rows.
 // PLAST_COL_SMALL_XCD numbers the column slices per XCD, so that the slices sharing a 128-byte
 // line run on one XCD. Measured in one process (device time of calls replayed from a graph),

@@ -166,8 +166,9 @@ template <Bin OP, bool B>
 struct BinGradBody : ScalarBody<BinGradBody<OP, B>> {
   static constexpr int NIN = 2 + int(kGradUsesA<OP, B>) + int(kGradUsesB<OP, B>);
   // d and g cover the space: where an operand is broadcast they keep nontemporal loads (mul's gradient
-  // of the unbroadcast operand, 67M elements: 158 us with every load ordinary, 128 so; with ordinary
-  // stores 138)
+  // of the unbroadcast operand beside a row: [16384, 4096] 146 us with every load ordinary, 126 so, with
+  // ordinary stores 138; [2048, 2048] 12.6 and 9.2 after other work, but 6.8 and 9.0 where the call
+  // before left all three arrays in the last-level cache, [8192, 4096] 57 and 65)
   static constexpr uint32_t kStreamed = 3;
   uint64_t simd_end;
   bool index_free() const { return simd_end == 0; }

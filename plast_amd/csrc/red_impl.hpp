@@ -5,14 +5,16 @@
 //   rows   — the innermost axis is reduced and unit-stride: one wave64 per (row, segment), float4
 //            loads, wave shuffle reduction; long rows split into segments whose partials a finalize
 //            pass combines in order;
-//   cols   — the innermost axis is kept and unit-stride: each lane owns four adjacent outputs and
-//            walks its chunk of the reduced axis in order; chunks combine in order in a finalize
-//            pass (no atomics anywhere, so results are deterministic);
+//   cols   — the innermost axis is kept and unit-stride: each lane owns four adjacent outputs (or
+//            one, or a share of the flat array of narrow rows: launch_rules.hpp) and walks its chunk
+//            of the reduced axis in order; chunks combine in order in a finalize pass (no atomics
+//            anywhere, so results are deterministic);
 //            With further reduced axes outside (a bias gradient over batch and space, say), both
-//            walk the flattened reduced index: lexicographic over the reduced axes, the innermost
-//            one in runs of its extent (MULTI kernels; reduced_offset decodes it). The generic
-//            kernel's one lane per output took 32.6 ms for config 3's B gradient (512 outputs of
-//            131072 terms, 268 MB); config 3's training graph went from 33.9 to 0.59 ms;
+//            (the columns for plain sums alone) walk the flattened reduced index: lexicographic over
+//            the reduced axes, the innermost one in runs of its extent (MULTI kernels;
+//            reduced_offset decodes it). The generic kernel's one lane per output took 32.6 ms for
+//            config 3's B gradient (512 outputs of 131072 terms, 268 MB); config 3's training graph
+//            went from 33.9 to 0.55 ms;
 //   generic— any layout: one lane per output, serial walk in index order.
 //
 // Max/min reproduce the reference's literal fold `acc > x ? acc : x` from -FLT_MAX
