@@ -1509,9 +1509,13 @@ bool launch_reduction(const Prod &prod, const void *const *in, void *out, Space 
                        : workspace(sizeof(Part) * A.rows * segs);
         if (!A.part) return false;
       }
-      // short rows: 2, 8 or 32 lanes each. [50000, 77] a wave per row / 8 lanes: see the kernel.
+      // short rows: 2, 8 or 32 lanes each. [50000, 77] a wave per row / 8 lanes: see the kernel. An
+      // argmax walks a lane's values one after the other: rows above 16 take 8 lanes ([1024, 31] 4.2 us
+      // in 2, 3.4 in 8; [65536, 17] 4.0 and 4.5), and few rows above 64 take 32 ([1024, 127] 4.2 in 8, 3.6
+      // in 32, [8192, 100] 4.2 and 3.9; [8192, 45] 3.7 and 4.1).
       if (!multi && A.len <= 16 * 32) {
-        const int lanes = A.len <= 16 * 2 ? 2 : A.len <= 16 * 8 ? 8 : 32;
+        const bool arg = std::is_same<Comb, ArgmaxComb>::value, few = arg && A.rows <= 8192;
+        const int lanes = A.len <= (arg ? 16 : 32) ? 2 : A.len <= (few ? 64 : 128) ? 8 : 32;
         const unsigned sgrid = ceil_div(A.rows, (kBlock / 64) * (64 / lanes));
         if (lanes == 2) red_rows_short_kernel<Prod, Comb, 2><<<sgrid, kBlock, 0, stream()>>>(A1, prod);
         else if (lanes == 8) red_rows_short_kernel<Prod, Comb, 8><<<sgrid, kBlock, 0, stream()>>>(A1, prod);

@@ -30,6 +30,11 @@ def _cases():
             for d in ("special", "ties"):
                 out.append(Case(f"{op}_rows_{s}_{d}", op, "fwd", [Arr(s, d, 10 + i)], _red_shape(s, 1, 0),
                                 (1, 0, 0.0), "i64" if op == "argmax" else "f32"))
+    # argmax rows on each side of their lane counts' lines
+    for i, s in enumerate([(99, 16), (99, 17), (99, 64), (8192, 65), (8192, 128), (8193, 65), (8193, 128), (8193, 129)]):
+        for d in ("special", "ties"):
+            out.append(Case(f"argmax_rows_{s}_{d}", "argmax", "fwd", [Arr(s, d, 30 + i)], _red_shape(s, 1, 0),
+                            (1, 0, 0.0), "i64"))
     for i, s in enumerate(COLS):
         for op in OPS:
             for d in ("special", "normal"):
