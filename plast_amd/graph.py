@@ -107,13 +107,17 @@ class Graph:
         """The calls, bound on the first pass and again when the DAG holds other nodes: its head (the
         node array and the count) and the array are compared with what they held then."""
         run = self._run
-        if run is None or run[0] is not self.dag or run[1].raw != run[2] or run[3].raw != run[4]:
-            dag = self.dag
-            head = (C.c_char * abi.DAG.capacity.offset).from_buffer(dag)
-            size = dag.count * C.sizeof(C.c_void_p)
-            nodes = (C.c_char * size).from_address(C.addressof(dag.nodes.contents)) if size else (C.c_char * 0)()
-            run = self._run = dag, head, head.raw, nodes, nodes.raw, self._calls()
-        return run[5]
+        if run is not None:
+            dag, head, was_head, nodes, was_nodes, calls = run
+            if dag is self.dag and head() == was_head and nodes() == was_nodes:
+                return calls
+        dag = self.dag
+        size = dag.count * C.sizeof(C.c_void_p)
+        head = memoryview((C.c_char * abi.DAG.capacity.offset).from_buffer(dag)).tobytes
+        nodes = memoryview((C.c_char * size).from_address(C.addressof(dag.nodes.contents)) if size
+                           else (C.c_char * 0)()).tobytes
+        self._run = dag, head, head(), nodes, nodes(), self._calls()
+        return self._run[5]
 
     def forward(self) -> None:
         """dag_forward (graph.c:57-60): each node's GPU forward slot in order."""
